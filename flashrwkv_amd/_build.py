@@ -61,6 +61,7 @@ def _run(cmd: list[str]) -> None:
 FILE_FLAGS = {
     "chunk_fwd": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "chunk_bwd": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+    "chunk_transfer": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
 }
 
 

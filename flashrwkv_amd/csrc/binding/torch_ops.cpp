@@ -267,6 +267,29 @@ TicketPtr prepare_recurrent_metadata(Tensor query_start_loc, Tensor state_indice
                                              state_pool_size, max_seqlen);
 }
 
+// Device scratch of the given size from PyTorch's caching allocator (on the
+// current stream), or an undefined tensor for 0 bytes.
+Tensor workspace_like(const Tensor& like, size_t bytes) {
+  if (bytes == 0) return Tensor();
+  return at::empty({static_cast<int64_t>(bytes)}, like.options().dtype(at::kByte));
+}
+
+// Scratch of a split call (undefined when the call does not split); total and
+// longest as for frwkv_split_scratch_bytes.
+Tensor split_scratch(int kernel, int64_t sequences, int64_t heads, int64_t head_size,
+                     int64_t total, int64_t longest, const Tensor& like) {
+  return workspace_like(like, frwkv_split_scratch_bytes(
+                                  kernel, static_cast<int32_t>(sequences),
+                                  static_cast<int32_t>(heads), static_cast<int32_t>(head_size),
+                                  static_cast<int32_t>(total), static_cast<int32_t>(longest)));
+}
+void* scratch_ptr(const Tensor& scratch) {
+  return scratch.defined() ? scratch.data_ptr() : nullptr;
+}
+size_t scratch_size(const Tensor& scratch) {
+  return scratch.defined() ? static_cast<size_t>(scratch.numel()) : 0;
+}
+
 // Layout checks of the fp32-state recurrent op (csrc/validation.cpp:27-129
 // rules; fp32 tokens only through the internal op).
 void check_recurrent_layout(const Tensor& cu, const Tensor& slots,
@@ -362,7 +385,13 @@ void recurrent_impl(const Tensor& cu, const Tensor& slots, Tensor& state,
       (g_recurrent_long_route.load(std::memory_order_relaxed) == 1 || stream_is_capturing(state))) {
     max_seqlen = -1;
   }
-  check_rc(frwkv_recurrent_forward(
+  // Long bf16 sequences run on the chunk kernel, split when there are few.
+  Tensor scratch;
+  if (max_seqlen >= 64 && r.scalar_type() == at::kBFloat16) {
+    scratch = split_scratch(FRWKV_SPLIT_RECURRENT, slots.numel(), state.size(1), state.size(2),
+                            r.size(0), max_seqlen, r);
+  }
+  check_rc(frwkv_recurrent_forward_split(
       io_code(r.scalar_type()), decay_mode, static_cast<int32_t>(slots.numel()),
       static_cast<int32_t>(state.size(1)), static_cast<int32_t>(state.size(2)),
       static_cast<int32_t>(r.size(0)), static_cast<int32_t>(max_seqlen),
@@ -371,7 +400,8 @@ void recurrent_impl(const Tensor& cu, const Tensor& slots, Tensor& state,
       state.data_ptr<float>(), r.data_ptr(), decay.data_ptr(),
       decay_bias.has_value() ? decay_bias->data_ptr() : nullptr, k.data_ptr(),
       v.data_ptr(), a.data_ptr(), b.data_ptr(), output.data_ptr(),
-      static_cast<float>(scale), current_stream(state)));
+      static_cast<float>(scale), scratch_ptr(scratch), scratch_size(scratch),
+      current_stream(state)));
 }
 
 // Process-wide route of long bf16 sequences in the fp32-state op (not a
@@ -461,7 +491,7 @@ void check_chunk_metadata(const Tensor& cu, const Tensor& slots, const Tensor& r
 void chunk_impl(const Tensor& r, const Tensor& decay, const Tensor& k, const Tensor& v,
                 const Tensor& a, const Tensor& b, Tensor& pool, const Tensor& cu,
                 const Tensor& slots, double scale, const std::optional<Tensor>& decay_bias,
-                int decay_mode, const Tensor& output) {
+                int decay_mode, const Tensor& output, int64_t max_seqlen) {
   TORCH_CHECK(std::isfinite(scale), "scale must be finite");
   check_device_contiguous(pool, "state_pool");
   TORCH_CHECK(pool.device() == r.device(), "state_pool must be on the same device as r");
@@ -481,15 +511,21 @@ void chunk_impl(const Tensor& r, const Tensor& decay, const Tensor& k, const Ten
   c10::DeviceGuard guard(r.device());
   refuse_capture(r, "the chunked WKV7 forward");
   Prepared launch = device_prepare(cu, slots, r.size(0), pool.size(0));
-  check_rc(frwkv_chunk_forward(
+  // An unknown longest sequence is taken as the mean one.
+  const int64_t mean = (r.size(0) + slots.numel() - 1) / slots.numel();
+  const int32_t longest =
+      static_cast<int32_t>(max_seqlen > 0 ? std::min(max_seqlen, r.size(0)) : mean);
+  const Tensor scratch =
+      split_scratch(FRWKV_SPLIT_CHUNK, slots.numel(), r.size(1), 64, r.size(0), longest, r);
+  check_rc(frwkv_chunk_forward_split(
       io_code(r.scalar_type()), decay_mode, pool_code, static_cast<int32_t>(slots.numel()),
       static_cast<int32_t>(r.size(1)), 64, static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(pool.size(0)), launch.cu_snapshot.data_ptr<int32_t>(),
       launch.slot_snapshot.data_ptr<int32_t>(), launch.status.data_ptr<int32_t>(),
       pool.data_ptr(), r.data_ptr(), decay.data_ptr(),
       decay_bias.has_value() ? decay_bias->data_ptr() : nullptr, k.data_ptr(), v.data_ptr(),
-      a.data_ptr(), b.data_ptr(), output.data_ptr(), static_cast<float>(scale),
-      current_stream(r)));
+      a.data_ptr(), b.data_ptr(), output.data_ptr(), static_cast<float>(scale), longest,
+      scratch_ptr(scratch), scratch_size(scratch), current_stream(r)));
 }
 
 // Public op (reference infer_chunk_bf16_forward_varlen.cpp:77-171): bf16
@@ -504,7 +540,7 @@ std::tuple<Tensor, Tensor> infer_chunk_bf16_forward_varlen(
   TORCH_CHECK(max_seqlen > 0, "max_seqlen must be positive");
   Tensor output = at::empty_like(v);
   chunk_impl(r, decay_logits, k, v, a, b, state_pool, cu_seqlens, state_indices, scale,
-             decay_bias, FRWKV_DECAY_LOGITS, output);
+             decay_bias, FRWKV_DECAY_LOGITS, output, max_seqlen);
   return {output, state_pool};
 }
 
@@ -518,7 +554,7 @@ Tensor chunk_forward_internal(Tensor r, Tensor decay, Tensor k, Tensor v, Tensor
   check_chunk_tokens(r, decay, k, v, a, b, /*bf16_only=*/false);
   Tensor output = at::empty_like(v);
   chunk_impl(r, decay, k, v, a, b, state_pool, cu_seqlens, state_indices, scale, decay_bias,
-             static_cast<int>(decay_mode), output);
+             static_cast<int>(decay_mode), output, /*max_seqlen=*/-1);
   return output;
 }
 
@@ -538,13 +574,6 @@ float* checked_interior(const std::optional<Tensor>& interior, const Tensor& r, 
                   static_cast<size_t>(interior->numel()) * sizeof(float) >= need,
               "interior must be float32 with at least ", need, " bytes");
   return interior->data_ptr<float>();
-}
-
-// Device scratch of the given size from PyTorch's caching allocator (on the
-// current stream), or an undefined tensor for 0 bytes.
-Tensor workspace_like(const Tensor& like, size_t bytes) {
-  if (bytes == 0) return Tensor();
-  return at::empty({static_cast<int64_t>(bytes)}, like.options().dtype(at::kByte));
 }
 
 void check_statetune_metadata(const Tensor& offsets, const Tensor& starts,
@@ -599,7 +628,9 @@ void statetune_forward_impl(const Tensor& offsets, const Tensor& starts, const T
   float* interior_ptr = checked_interior(interior, r, d);
   c10::DeviceGuard guard(state.device());
   refuse_capture(r, "the StateTune forward");
-  check_rc(frwkv_statetune_forward(
+  const Tensor scratch = split_scratch(FRWKV_SPLIT_CALLER_CHUNKS, state.size(0), state.size(1), d,
+                                       starts.numel(), /*longest=*/0, r);
+  check_rc(frwkv_statetune_forward_split(
       io_code(r.scalar_type()), decay_mode, static_cast<int32_t>(state.size(0)),
       static_cast<int32_t>(state.size(1)), static_cast<int32_t>(d), static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(starts.numel()), offsets.data_ptr<int32_t>(),
@@ -607,7 +638,7 @@ void statetune_forward_impl(const Tensor& offsets, const Tensor& starts, const T
       r.data_ptr(), decay.data_ptr(), nullptr, k.data_ptr(), v.data_ptr(), a.data_ptr(),
       b.data_ptr(), output.data_ptr(), boundary.data_ptr<float>(),
       state_dot_a.data_ptr<float>(), interior_ptr, static_cast<float>(scale),
-      current_stream(state)));
+      scratch_ptr(scratch), scratch_size(scratch), current_stream(state)));
 }
 
 // Reference statetune_recurrent_fp32io16_forward.cpp:26-44 (decay logits).
@@ -803,12 +834,15 @@ void clampw_forward(Tensor r, Tensor w, Tensor k, Tensor v, Tensor a, Tensor b, 
   check_clampw_side(r, s, sa);
   c10::DeviceGuard guard(r.device());
   refuse_capture(r, "the clampw-v3 pretraining forward");
-  check_rc(frwkv_pretrain_forward(
+  const Tensor scratch =
+      split_scratch(FRWKV_SPLIT_CHUNK, r.size(0), r.size(2), head_size, r.size(0) * r.size(1),
+                    r.size(1), r);
+  check_rc(frwkv_pretrain_forward_split(
       io_code(r.scalar_type()), FRWKV_DECAY_LOGITS, static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(r.size(1)), static_cast<int32_t>(r.size(2)),
       static_cast<int32_t>(head_size), r.data_ptr(), w.data_ptr(), k.data_ptr(), v.data_ptr(),
       a.data_ptr(), b.data_ptr(), y.data_ptr(), s.data_ptr<float>(), sa.data_ptr<float>(),
-      current_stream(r)));
+      scratch_ptr(scratch), scratch_size(scratch), current_stream(r)));
 }
 
 void clampw_backward(Tensor r, Tensor w, Tensor k, Tensor v, Tensor a, Tensor b, Tensor dy,
@@ -913,13 +947,13 @@ std::tuple<Tensor, Tensor> rl_infctx_forward(Tensor offsets, Tensor starts, Tens
   Tensor output = at::empty_like(v);
   const Tensor cu = at::tensor(cu_host, at::TensorOptions().dtype(at::kInt)).to(state.device());
   const Tensor slots = at::arange(batch, at::TensorOptions().dtype(at::kInt).device(state.device()));
+  int64_t max_len = 0;
+  for (int64_t s = 0; s < batch; ++s) max_len = std::max<int64_t>(max_len, cu_host[s + 1] - cu_host[s]);
   if (state.size(2) == 64) {
     check_chunk_tokens(r, decay_logits, k, v, a, b, /*bf16_only=*/false);
     chunk_impl(r, decay_logits, k, v, a, b, working, cu, slots, scale, decay_bias,
-               FRWKV_DECAY_LOGITS, output);
+               FRWKV_DECAY_LOGITS, output, max_len);
   } else {
-    int64_t max_len = 0;
-    for (int64_t s = 0; s < batch; ++s) max_len = std::max<int64_t>(max_len, cu_host[s + 1] - cu_host[s]);
     recurrent_impl(cu, slots, working, r, decay_logits, k, v, a, b, output, scale, decay_bias,
                    std::nullopt, max_len, FRWKV_DECAY_LOGITS, /*allow_fp32_tokens=*/false);
   }

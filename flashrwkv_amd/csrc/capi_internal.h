@@ -69,11 +69,12 @@ size_t frwkv_train_slice_bytes(int32_t head_size, int32_t num_heads, int32_t tot
 
 // The recurrent operator's route for long sequences (chunk_fwd.hip): the
 // split-precision chunk kernel on bf16 tokens, head size 64, fp32 pool.
-// Arguments as frwkv_recurrent_forward's, already checked by it.
+// Arguments as frwkv_recurrent_forward_split's, already checked by it.
 int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32_t num_heads,
                                     int32_t total_tokens, int32_t state_pool_size,
                                     const int32_t* cu_seqlens, const int32_t* state_indices,
                                     const int32_t* metadata_status, float* state_pool,
                                     const void* r, const void* decay, const void* decay_bias,
                                     const void* k, const void* v, const void* a, const void* b,
-                                    void* output, float scale, void* stream);
+                                    void* output, float scale, int32_t max_seqlen, void* scratch,
+                                    size_t scratch_bytes, void* stream);

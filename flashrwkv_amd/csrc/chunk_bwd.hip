@@ -176,25 +176,6 @@ __device__ __forceinline__ float prefix16(float x) {
 __device__ __forceinline__ float suffix16(float x) {
   return row_shl_add<8>(row_shl_add<4>(row_shl_add<2>(row_shl_add<1>(x))));
 }
-// Products over the 16 lanes of a DPP row (n = lane % 16): lanes n < N keep
-// x (the shifted-in value reads 0, and the select restores x).
-template <int N>
-__device__ __forceinline__ float row_shr_mul(float x, int n) {
-  const float y = x * __int_as_float(
-                          __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x110 + N, 0xf, 0xf, true));
-  return n >= N ? y : x;
-}
-__device__ __forceinline__ float prefix16_mul(float x, int n) {
-  return row_shr_mul<8>(row_shr_mul<4>(row_shr_mul<2>(row_shr_mul<1>(x, n), n), n), n);
-}
-// The exclusive product from the inclusive one: lane n takes lane n - 1's,
-// lane 0 the empty product 1.
-__device__ __forceinline__ float exclusive16(float incl, int n) {
-  const float y = __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(incl), 0x111, 0xf, 0xf, true));
-  return n >= 1 ? y : 1.0f;
-}
-
 // Stores a C-layout block (lane (g, n) holds X[4g + j][n]) into a row-major
 // [row][col] bf16 tile at dst: four 2-byte stores per lane, the 16 lanes of a
 // group writing 32 consecutive bytes of one row.

@@ -49,6 +49,7 @@
 #include "wkv7_device.h"
 #include "wkv7_mfma.h"
 #include "chunk_common.h"
+#include "chunk_parts.h"
 
 namespace frwkv {
 namespace {
@@ -101,53 +102,6 @@ using ExtraTiles = typename ExtraTilesOf<kPrecise>::type;
 __device__ __forceinline__ const uint16_t* tri_block(const ChunkSmem& sm, int m, int p, int q) {
   return sm.tri[m] + tri_index(p, q) * kTriBlock;
 }
-
-struct ChunkFwdParams {
-  int32_t num_heads;
-  // Packed varlen batches of at most 64 sequences (cu_seqlens mode) run
-  // their sequences longest first: workgroup b takes the sequence of length
-  // rank b / H. 0 keeps the natural order.
-  int32_t longest_first_sequences;
-  int32_t total_tokens;
-  int32_t state_slots;
-  const int32_t* cu_seqlens;    // sequence token ranges when seg_offsets == null
-  const int32_t* seg_offsets;   // [B+1] segment lists (StateTune chunks) or null
-  const int32_t* seg_starts;
-  const int32_t* seg_ends;
-  int32_t num_segments;         // length of seg_starts / seg_ends / boundary
-  const int32_t* slots;         // [B] state slot per sequence, or null (identity)
-  const int32_t* status;        // metadata status word, or null
-  void* state;
-  const void* r;
-  const void* decay;
-  const void* bias;
-  const void* k;
-  const void* v;
-  const void* a;
-  const void* b;
-  void* out;
-  float* boundary;              // state at each segment start, or null
-  float* state_dot_a;           // per-token a^T S_{t-1}, or null
-  float scale;
-  int64_t out_elems;
-  // Dense layout: > 0 means every sequence has dense_t tokens (sequence s
-  // covers tokens s * dense_t ..), with no cu_seqlens or segment arrays.
-  int32_t dense_t;
-  // 1: boundary is [B, H, dense_t / 16, D, D], the state every 16 tokens.
-  int32_t boundary16;
-  // 1: the initial states are read and never written back (replay from
-  // stored boundaries).
-  int32_t read_only_state;
-  // [ceil(total_tokens / 64), H, D, D] or null: the state at every 64-token
-  // piece start inside a segment (not at the segment start), at slot
-  // (piece start) / 64. Interior starts of different segments lie more than
-  // 64 tokens apart, so the slots are distinct.
-  float* interior;
-  // 1 (replay layout, one segment per unit): only the interior states are
-  // wanted; segments of at most 64 tokens have none and are skipped, and a
-  // segment's last piece is not computed.
-  int32_t fill_only;
-};
 
 // Token rows of one chunk held by a thread: r, w, k, a, b for 2 tokens x 8
 // features (prepare layout), and two 16-byte pieces of the chunk's V tile
@@ -730,6 +684,100 @@ __device__ void state_pass(const ChunkSmem& sm, const ExtraTiles<kPrecise>& ext,
   }
 }
 
+// Start state of part `part`, wave w's columns in C layout (S[kb][j]: row
+// 16kb + 4g + j, column 16w + n): part 0 takes the kept start state, part j the
+// first part's end state through the maps of parts 1 .. j - 1,
+// S <- M_i S + N_i. The four waves need all of each map, so maps go through
+// LDS, four at a time (the chunk tiles' space, not yet in use), split into
+// bf16 hi + lo there: M S is the three products hi hi + hi lo + lo hi, about
+// 2^-16 relative error per step, on an fp32 state. The next four maps are
+// loaded while these are applied. (Every wave reading the maps from memory as
+// fp32 MFMA operands took 3.2 us per step; this takes 0.5.)
+constexpr int kComposeMaps = 4;
+__device__ __forceinline__ void compose_start(ChunkSmem& sm, const ChunkFwdParams& p, int unit,
+                                              int part, f32x4 (&S)[4]) {
+  const int tid = threadIdx.x;
+  const int w = uniform(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4, n = lane & 15;
+  uint16_t* const tiles = reinterpret_cast<uint16_t*>(&sm);  // [map][hi, lo][row][col]
+  static_assert(sizeof(ChunkSmem) >= kComposeMaps * 2 * kOpTile * sizeof(uint16_t),
+                "the maps fit the chunk tiles");
+  const int col = (4 * g) * kHead + 16 * w + n;
+  auto load_slab = [&](int i, int which, f32x4 (&x)[4]) {
+    const float* src = part_state(p, unit, i, which) + col;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[kb][j] = src[(16 * kb + j) * kHead];
+    }
+  };
+  load_slab(0, part > 0 ? 1 : 0, S);
+  if (part < 2) return;
+  // The thread's share of a map: row tid / 4, 16 columns.
+  const int share = (tid >> 2) * kHead + 16 * (tid & 3);
+  const int place = (tid >> 2) * kOpStride + 16 * (tid & 3);
+  f32x4 m[kComposeMaps][4], off[kComposeMaps][4];
+  auto load_maps = [&](int first) {
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        const float* src = part_state(p, unit, first + u, 0) + share;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) m[u][c] = *reinterpret_cast<const f32x4*>(src + 4 * c);
+      }
+    }
+  };
+  load_maps(1);
+  for (int first = 1; first < part; first += kComposeMaps) {
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) load_slab(first + u, 1, off[u]);
+    }
+    if (first > 1) __syncthreads();  // the maps before these are applied
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        uint16_t* hi = tiles + 2 * u * kOpTile + place;
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) {
+          const float x[8] = {m[u][c][0],     m[u][c][1],     m[u][c][2],     m[u][c][3],
+                              m[u][c + 1][0], m[u][c + 1][1], m[u][c + 1][2], m[u][c + 1][3]};
+          store8_bf16_split(hi + 4 * c, hi + kOpTile + 4 * c, x);
+        }
+      }
+    }
+    __syncthreads();
+    load_maps(first + kComposeMaps);
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        const uint16_t* hi = tiles + 2 * u * kOpTile;
+        const uint16_t* lo = hi + kOpTile;
+        i16x4 sh[4], sl[4];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) to_operand_split(S[kb], sh[kb], sl[kb]);
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) S[kb] = off[u][kb];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const i16x8 bh = cat(sh[2 * kk], sh[2 * kk + 1]);
+          const i16x8 bl = cat(sl[2 * kk], sl[2 * kk + 1]);
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) {
+            const i16x8 ah = lds_operand32<kOpStride>(hi, 16 * rb + n, 32 * kk, g);
+            const i16x8 al = lds_operand32<kOpStride>(lo, 16 * rb + n, 32 * kk, g);
+            S[rb] = mfma32(al, bh, S[rb]);
+            S[rb] = mfma32(ah, bl, S[rb]);
+            S[rb] = mfma32(ah, bh, S[rb]);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();  // before the chunk tiles are written
+}
+
 // The sequence of the given rank in order of decreasing length (ties in
 // index order), for batches of at most 64 sequences: lane s holds sequence
 // s's length, counts the sequences ahead of it, and the lane whose count is
@@ -753,7 +801,8 @@ __device__ __forceinline__ int sequence_by_length_rank(const ChunkFwdParams& p, 
 // operator's chunk route). Those paths then compile away, and with them the
 // scalar registers their descriptors and offsets would hold across the chunk
 // loop (spilled to VGPR lanes and reloaded every chunk otherwise).
-template <typename T, DecayMode M, typename PoolT, bool kPrecise, bool kLean>
+// kParts: the workgroup walks one part of its sequence (chunk_parts.h).
+template <typename T, DecayMode M, typename PoolT, bool kPrecise, bool kLean, bool kParts>
 __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_kernel(
     ChunkFwdParams p) {
   __shared__ ChunkSmem sm;
@@ -772,9 +821,14 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   const int tp = lane & 7;   // token pair
   const int kg = lane >> 3;  // feature group
   const int heads = p.num_heads;
-  int seq = blockIdx.x / heads;
-  if (p.longest_first_sequences > 0) seq = sequence_by_length_rank(p, seq, lane);
-  const int head = blockIdx.x % heads;
+  // Parts: block part * units + unit, so that (for a unit count divisible by
+  // the 8 XCDs) a unit's parts share an XCD, and its L2, in both launches.
+  const int units = kParts ? static_cast<int>(gridDim.x) / p.parts : 0;
+  const int part = kParts ? static_cast<int>(blockIdx.x) / units : 0;
+  const int unit = kParts ? static_cast<int>(blockIdx.x) % units : static_cast<int>(blockIdx.x);
+  int seq = unit / heads;
+  if (!kParts && p.longest_first_sequences > 0) seq = sequence_by_length_rank(p, seq, lane);
+  const int head = unit % heads;
   // Metadata values are workgroup-uniform; readfirstlane keeps them (and
   // every buffer descriptor derived from them) in scalar registers.
   const int slot = uniform(p.slots != nullptr ? p.slots[seq] : seq);
@@ -796,6 +850,29 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   } else if (segmented) {
     seg_lo = seq;
     seg_hi = min(seq + 1, p.num_segments);
+  }
+
+  // The workgroup's part: a run of the sequence's segments, or of its 64-token
+  // chunks (part_lo, part_hi).
+  bool last_part = true;
+  int part_lo = 0, part_hi = 0;
+  if constexpr (kParts) {
+    PartRange pr;
+    if (segmented) {
+      pr = part_range(p, max(seg_hi - seg_lo, 0), part);
+      seg_hi = seg_lo + pr.end;
+      seg_lo += pr.begin;
+    } else {
+      int len = p.dense_t;
+      if (len == 0) {
+        len = min(p.cu_seqlens[seq + 1], p.total_tokens) - max(p.cu_seqlens[seq], 0);
+      }
+      pr = part_range(p, (uniform(max(len, 0)) + kChunk - 1) / kChunk, part);
+      part_lo = pr.begin * kChunk;
+      part_hi = pr.end * kChunk;
+    }
+    if (!pr.exists) return;
+    last_part = pr.last;
   }
 
   // Interior-state fill (replay layout, one segment per unit): a segment of
@@ -829,6 +906,9 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   const uint32_t s_off = static_cast<uint32_t>((4 * g) * kHead + 16 * wave + n) * kPoolBytes;
   // A null state means S0 = 0 and no final state (the pretraining layout).
   f32x4 S[4];
+  if constexpr (kParts) {
+    compose_start(sm, p, unit, part, S);
+  } else {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -842,6 +922,7 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
         S[kb][j] = to_f32<PoolT>(__builtin_amdgcn_raw_buffer_load_b16(state_rs, s_off, so, 0));
       }
     }
+  }
   }
 
   // Segment bounds, 64 segments at a time in VGPR lanes (lane i: segment
@@ -870,6 +951,12 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
     }
     t_begin = uniform(max(t_begin, 0));
     t_end = uniform(min(t_end, p.total_tokens));
+    if constexpr (kParts) {
+      if (!segmented) {
+        t_end = min(t_begin + part_hi, t_end);
+        t_begin += part_lo;
+      }
+    }
   };
   // Chunk following (seg, c0): c0 + 64 in the same segment, else the start
   // of the next non-empty segment. Returns false at the end of the sequence.
@@ -985,7 +1072,7 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
       // Every-16-tokens boundary layout [B, H, dense_t / 16, D, D]: the state
       // at token c0 + i (i a multiple of 16) of this sequence.
       const int64_t b16_base = (static_cast<int64_t>(seq) * heads + head) * (p.dense_t / 16) +
-                               (c0 - t_begin) / 16;
+                               (c0 - (kParts ? seq * p.dense_t : t_begin)) / 16;
       auto b16_rs = [&](int i, int count) {
         if (!boundary16 || count <= 0) return buffer_rsrc(static_cast<float*>(nullptr), 0u);
         return buffer_rsrc(boundary + (b16_base + i / 16) * kHead * kHead,
@@ -1065,7 +1152,7 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
     }
   }
 
-  if (!has_state || (!kLean && p.read_only_state)) return;
+  if (!has_state || (!kLean && p.read_only_state) || !last_part) return;
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -1090,11 +1177,22 @@ int launch_chunk(const ChunkFwdParams& p, int units, hipStream_t stream) {
                     p.boundary == nullptr && p.state_dot_a == nullptr &&
                     p.interior == nullptr && !p.fill_only && !p.boundary16 &&
                     !p.read_only_state && p.state != nullptr;
-  if (lean) {
-    hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, true>), dim3(units),
+  if (p.parts > 1) {
+    const int rc = launch_chunk_transfer<T, M, PoolT, kPrecise>(p, units, stream);
+    if (rc != FRWKV_OK) return rc;
+    const dim3 grid(units * p.parts);
+    if (lean) {
+      hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, true, true>), grid,
+                         dim3(kChunkThreads), 0, stream, p);
+    } else if constexpr (!kPrecise && __is_same(PoolT, float)) {
+      hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, false, true>), grid,
+                         dim3(kChunkThreads), 0, stream, p);
+    }
+  } else if (lean) {
+    hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, true, false>), dim3(units),
                        dim3(kChunkThreads), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, false>), dim3(units),
+  } else if constexpr (!kPrecise && __is_same(PoolT, float)) {
+    hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, false, false>), dim3(units),
                        dim3(kChunkThreads), 0, stream, p);
   }
   return check_launch("chunk_fwd_kernel");
@@ -1142,6 +1240,26 @@ int check_token_pointers(const void* r, const void* decay, const void* k, const 
 }  // namespace
 }  // namespace frwkv
 
+extern "C" size_t frwkv_split_scratch_bytes(int kernel, int32_t num_sequences,
+                                            int32_t num_heads, int32_t head_size,
+                                            int32_t total, int32_t longest) {
+  using namespace frwkv;
+  if (head_size != 64 || num_sequences <= 0 || num_heads <= 0 || total <= 0) return 0;
+  const int64_t units = static_cast<int64_t>(num_sequences) * num_heads;
+  switch (kernel) {
+    case FRWKV_SPLIT_CHUNK:
+      return part_bytes(units, plan_parts(num_sequences, num_heads, chunks_of(total),
+                                          chunks_of(longest), kForwardTime, kTransferTime));
+    case FRWKV_SPLIT_RECURRENT:
+      return part_bytes(units, plan_parts(num_sequences, num_heads, chunks_of(total),
+                                          chunks_of(longest), kPreciseTime, kTransferTime));
+    case FRWKV_SPLIT_CALLER_CHUNKS:
+      return part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total));
+    default:
+      return 0;
+  }
+}
+
 extern "C" int frwkv_chunk_forward(
     int io_dtype, int decay_mode, int pool_dtype, int32_t num_sequences,
     int32_t num_heads, int32_t head_size, int32_t total_tokens, int32_t state_pool_size,
@@ -1149,6 +1267,21 @@ extern "C" int frwkv_chunk_forward(
     const int32_t* metadata_status, void* state_pool, const void* r, const void* decay,
     const void* decay_bias, const void* k, const void* v, const void* a, const void* b,
     void* output, float scale, void* stream) {
+  return frwkv_chunk_forward_split(io_dtype, decay_mode, pool_dtype, num_sequences, num_heads,
+                                   head_size, total_tokens, state_pool_size, cu_seqlens,
+                                   state_indices, metadata_status, state_pool, r, decay,
+                                   decay_bias, k, v, a, b, output, scale, /*max_seqlen=*/-1,
+                                   nullptr, 0, stream);
+}
+
+extern "C" int frwkv_chunk_forward_split(
+    int io_dtype, int decay_mode, int pool_dtype, int32_t num_sequences,
+    int32_t num_heads, int32_t head_size, int32_t total_tokens, int32_t state_pool_size,
+    const int32_t* cu_seqlens, const int32_t* state_indices,
+    const int32_t* metadata_status, void* state_pool, const void* r, const void* decay,
+    const void* decay_bias, const void* k, const void* v, const void* a, const void* b,
+    void* output, float scale, int32_t max_seqlen, void* scratch, size_t scratch_bytes,
+    void* stream) {
   using namespace frwkv;
   if (!cu_seqlens || !state_indices || !metadata_status || !state_pool) {
     return set_error(FRWKV_ERR_INVALID_ARGUMENT, "frwkv_chunk_forward: null pointer argument");
@@ -1188,6 +1321,10 @@ extern "C" int frwkv_chunk_forward(
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
   const int units = num_sequences * num_heads;
+  use_parts(p, units,
+            plan_parts(num_sequences, num_heads, chunks_of(total_tokens), chunks_of(max_seqlen),
+                       kForwardTime, kTransferTime),
+            scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (pool_dtype == FRWKV_DTYPE_F32) return dispatch_chunk_io<float>(p, io_dtype, decay_mode, units, s);
   if (pool_dtype == FRWKV_DTYPE_BF16) return dispatch_chunk_io<Bf16>(p, io_dtype, decay_mode, units, s);
@@ -1203,6 +1340,20 @@ extern "C" int frwkv_statetune_forward(
     const void* decay_bias, const void* k, const void* v, const void* a, const void* b,
     void* output, float* boundary, float* state_dot_a, float* interior, float scale,
     void* stream) {
+  return frwkv_statetune_forward_split(
+      io_dtype, decay_mode, num_sequences, num_heads, head_size, total_tokens, num_chunks,
+      sequence_chunk_offsets, chunk_token_starts, chunk_token_ends, state, r, decay, decay_bias,
+      k, v, a, b, output, boundary, state_dot_a, interior, scale, nullptr, 0, stream);
+}
+
+extern "C" int frwkv_statetune_forward_split(
+    int io_dtype, int decay_mode, int32_t num_sequences, int32_t num_heads,
+    int32_t head_size, int32_t total_tokens, int32_t num_chunks,
+    const int32_t* sequence_chunk_offsets, const int32_t* chunk_token_starts,
+    const int32_t* chunk_token_ends, float* state, const void* r, const void* decay,
+    const void* decay_bias, const void* k, const void* v, const void* a, const void* b,
+    void* output, float* boundary, float* state_dot_a, float* interior, float scale,
+    void* scratch, size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   if (!sequence_chunk_offsets || !chunk_token_starts || !chunk_token_ends || !state ||
       !boundary || !state_dot_a) {
@@ -1253,6 +1404,8 @@ extern "C" int frwkv_statetune_forward(
   p.interior = interior;
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
+  use_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
+            plan_caller_chunks(num_sequences, num_heads, num_chunks), scratch, scratch_bytes);
   return dispatch_chunk_io<float>(p, io_dtype, decay_mode, num_sequences * num_heads,
                                   static_cast<hipStream_t>(stream));
 }
@@ -1324,6 +1477,16 @@ extern "C" int frwkv_pretrain_forward(int io_dtype, int decay_mode, int32_t batc
                                       const void* v, const void* a, const void* b,
                                       void* output, float* boundary, float* state_dot_a,
                                       void* stream) {
+  return frwkv_pretrain_forward_split(io_dtype, decay_mode, batch, tokens, num_heads, head_size,
+                                      r, decay, k, v, a, b, output, boundary, state_dot_a,
+                                      nullptr, 0, stream);
+}
+
+extern "C" int frwkv_pretrain_forward_split(
+    int io_dtype, int decay_mode, int32_t batch, int32_t tokens, int32_t num_heads,
+    int32_t head_size, const void* r, const void* decay, const void* k, const void* v,
+    const void* a, const void* b, void* output, float* boundary, float* state_dot_a,
+    void* scratch, size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   if (!boundary || !state_dot_a) {
     return set_error(FRWKV_ERR_INVALID_ARGUMENT, "frwkv_pretrain_forward: null pointer argument");
@@ -1366,6 +1529,10 @@ extern "C" int frwkv_pretrain_forward(int io_dtype, int decay_mode, int32_t batc
   p.state_dot_a = state_dot_a;
   p.scale = 1.0f;
   p.out_elems = static_cast<int64_t>(batch) * tokens * num_heads * head_size;
+  use_parts(p, static_cast<int64_t>(batch) * num_heads,
+            plan_parts(batch, num_heads, chunks_of(p.total_tokens), chunks_of(tokens),
+                       kForwardTime, kTransferTime),
+            scratch, scratch_bytes);
   return dispatch_chunk_io<float>(p, io_dtype, decay_mode, batch * num_heads,
                                   static_cast<hipStream_t>(stream));
 }
@@ -1431,7 +1598,8 @@ int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32
                                     const int32_t* metadata_status, float* state_pool,
                                     const void* r, const void* decay, const void* decay_bias,
                                     const void* k, const void* v, const void* a, const void* b,
-                                    void* output, float scale, void* stream) {
+                                    void* output, float scale, int32_t max_seqlen, void* scratch,
+                                    size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   ChunkFwdParams p{};
   p.num_heads = num_heads;
@@ -1453,6 +1621,10 @@ int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * kHead;
   const int units = num_sequences * num_heads;
+  use_parts(p, units,
+            plan_parts(num_sequences, num_heads, chunks_of(total_tokens), chunks_of(max_seqlen),
+                       kPreciseTime, kTransferTime),
+            scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (decay_mode == FRWKV_DECAY_LOGITS) {
     return launch_chunk<Bf16, DecayMode::kLogits, float, true>(p, units, s);

@@ -1010,6 +1010,20 @@ extern "C" int frwkv_recurrent_forward(
     float* state_pool, const void* r, const void* decay, const void* decay_bias,
     const void* k, const void* v, const void* a, const void* b, void* output,
     float scale, void* stream) {
+  return frwkv_recurrent_forward_split(io_dtype, decay_mode, num_sequences, num_heads, head_size,
+                                       total_tokens, max_seqlen, state_pool_size, cu_seqlens,
+                                       state_indices, metadata_status, state_pool, r, decay,
+                                       decay_bias, k, v, a, b, output, scale, nullptr, 0, stream);
+}
+
+extern "C" int frwkv_recurrent_forward_split(
+    int io_dtype, int decay_mode, int32_t num_sequences, int32_t num_heads,
+    int32_t head_size, int32_t total_tokens, int32_t max_seqlen,
+    int32_t state_pool_size, const int32_t* cu_seqlens,
+    const int32_t* state_indices, const int32_t* metadata_status,
+    float* state_pool, const void* r, const void* decay, const void* decay_bias,
+    const void* k, const void* v, const void* a, const void* b, void* output,
+    float scale, void* scratch, size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   if (!cu_seqlens || !state_indices || !metadata_status || !state_pool || !r ||
       !decay || !k || !v || !a || !b || !output) {
@@ -1034,7 +1048,8 @@ extern "C" int frwkv_recurrent_forward(
     return frwkv_recurrent_chunked_forward(decay_mode, num_sequences, num_heads, total_tokens,
                                            state_pool_size, cu_seqlens, state_indices,
                                            metadata_status, state_pool, r, decay, decay_bias,
-                                           k, v, a, b, output, scale, stream);
+                                           k, v, a, b, output, scale, max_seqlen, scratch,
+                                           scratch_bytes, stream);
   }
   RecurrentArgs p{num_sequences, num_heads, head_size, total_tokens, max_seqlen,
                   state_pool_size, cu_seqlens, state_indices, metadata_status,

@@ -120,6 +120,38 @@ int frwkv_recurrent_forward(int io_dtype, int decay_mode, int32_t num_sequences,
                             void* output, float scale, void* stream);
 
 /*
+ * Split calls. The chunked kernels walk one (sequence, head) with one
+ * workgroup; a call of few, long sequences can instead cut every sequence into
+ * parts that run side by side, given scratch memory for the parts' transfer
+ * states. Each *_split entry is the entry of the same name with that scratch:
+ * device memory of frwkv_split_scratch_bytes, 16-byte aligned, its content
+ * undefined before and after the call. With no scratch, or less than that, or
+ * where that is 0 (enough sequences to fill the GPU, or too short ones), the
+ * call runs unsplit, and is then exactly the entry of the same name. Results
+ * of the two agree up to the rounding of the state between parts.
+ *
+ * frwkv_split_scratch_bytes: total is the call's total tokens (B * T for
+ * pretraining) and longest its longest sequence in tokens (max_seqlen, T) for
+ * FRWKV_SPLIT_CHUNK (frwkv_chunk_forward_split, frwkv_pretrain_forward_split)
+ * and FRWKV_SPLIT_RECURRENT (frwkv_recurrent_forward_split); for
+ * FRWKV_SPLIT_CALLER_CHUNKS (frwkv_statetune_forward_split) total is
+ * num_chunks and longest is not used. No counterpart in the reference.
+ */
+enum { FRWKV_SPLIT_CHUNK = 0, FRWKV_SPLIT_RECURRENT = 1, FRWKV_SPLIT_CALLER_CHUNKS = 2 };
+size_t frwkv_split_scratch_bytes(int kernel, int32_t num_sequences, int32_t num_heads,
+                                 int32_t head_size, int32_t total, int32_t longest);
+int frwkv_recurrent_forward_split(int io_dtype, int decay_mode, int32_t num_sequences,
+                                  int32_t num_heads, int32_t head_size,
+                                  int32_t total_tokens, int32_t max_seqlen,
+                                  int32_t state_pool_size, const int32_t* cu_seqlens,
+                                  const int32_t* state_indices,
+                                  const int32_t* metadata_status, float* state_pool,
+                                  const void* r, const void* decay,
+                                  const void* decay_bias, const void* k, const void* v,
+                                  const void* a, const void* b, void* output, float scale,
+                                  void* scratch, size_t scratch_bytes, void* stream);
+
+/*
  * fp16-state recurrent forward (the Albatross family), pool [slots,H,D,D] of
  * fp16 updated in place at state_indices.
  * Replaces recurrent_fp16_from_decay_logits_cuda and its dispatch
@@ -199,6 +231,20 @@ int frwkv_chunk_forward(int io_dtype, int decay_mode, int pool_dtype,
                         const void* a, const void* b, void* output, float scale,
                         void* stream);
 
+/* frwkv_chunk_forward with scratch for a split call (see
+ * frwkv_split_scratch_bytes); max_seqlen is the longest sequence, or <= 0 if
+ * unknown (the call is then not split). */
+int frwkv_chunk_forward_split(int io_dtype, int decay_mode, int pool_dtype,
+                              int32_t num_sequences, int32_t num_heads,
+                              int32_t head_size, int32_t total_tokens,
+                              int32_t state_pool_size, const int32_t* cu_seqlens,
+                              const int32_t* state_indices,
+                              const int32_t* metadata_status, void* state_pool,
+                              const void* r, const void* decay, const void* decay_bias,
+                              const void* k, const void* v, const void* a, const void* b,
+                              void* output, float scale, int32_t max_seqlen, void* scratch,
+                              size_t scratch_bytes, void* stream);
+
 /*
  * Training (StateTune) forward with caller chunk metadata: sequence s owns
  * chunks sequence_chunk_offsets[s] .. sequence_chunk_offsets[s+1]-1, chunk c
@@ -235,6 +281,21 @@ int frwkv_statetune_forward(int io_dtype, int decay_mode, int32_t num_sequences,
                             const void* v, const void* a, const void* b,
                             void* output, float* boundary, float* state_dot_a,
                             float* interior, float scale, void* stream);
+
+/* frwkv_statetune_forward with scratch for a split call (see
+ * frwkv_split_scratch_bytes; head size 64). */
+int frwkv_statetune_forward_split(int io_dtype, int decay_mode, int32_t num_sequences,
+                                  int32_t num_heads, int32_t head_size,
+                                  int32_t total_tokens, int32_t num_chunks,
+                                  const int32_t* sequence_chunk_offsets,
+                                  const int32_t* chunk_token_starts,
+                                  const int32_t* chunk_token_ends, float* state,
+                                  const void* r, const void* decay,
+                                  const void* decay_bias, const void* k, const void* v,
+                                  const void* a, const void* b, void* output,
+                                  float* boundary, float* state_dot_a, float* interior,
+                                  float scale, void* scratch, size_t scratch_bytes,
+                                  void* stream);
 
 /* Bytes of the interior-state buffer of frwkv_statetune_forward /
  * frwkv_statetune_backward: ceil(total_tokens / P) x H x D x D elements of
@@ -357,6 +418,15 @@ int frwkv_pretrain_forward(int io_dtype, int decay_mode, int32_t batch, int32_t 
                            const void* decay, const void* k, const void* v,
                            const void* a, const void* b, void* output, float* boundary,
                            float* state_dot_a, void* stream);
+
+/* frwkv_pretrain_forward with scratch for a split call (see
+ * frwkv_split_scratch_bytes; head size 64). */
+int frwkv_pretrain_forward_split(int io_dtype, int decay_mode, int32_t batch, int32_t tokens,
+                                 int32_t num_heads, int32_t head_size, const void* r,
+                                 const void* decay, const void* k, const void* v,
+                                 const void* a, const void* b, void* output,
+                                 float* boundary, float* state_dot_a, void* scratch,
+                                 size_t scratch_bytes, void* stream);
 
 /*
  * Pretraining backward: recomputes every chunk from the boundary written by
