@@ -122,11 +122,12 @@ def statetune_recurrent_fp32io16_backward(sequence_chunk_offsets, chunk_token_st
 def statetune_backward_internal(sequence_chunk_offsets, chunk_token_starts, chunk_token_ends,
                                 r, decay, k, v, a, b, grad_output, grad_final_state, boundary,
                                 grad_r, grad_decay, grad_k, grad_v, grad_a, grad_b,
-                                grad_initial_state, interior, scale, decay_mode):
+                                grad_initial_state, interior, scale, decay_mode,
+                                state_dot_a=None):
     ops.statetune_backward_internal(
         sequence_chunk_offsets, chunk_token_starts, chunk_token_ends, r, decay, k, v, a, b,
         grad_output, grad_final_state, boundary, grad_r, grad_decay, grad_k, grad_v, grad_a,
-        grad_b, grad_initial_state, interior, float(scale), int(decay_mode))
+        grad_b, grad_initial_state, interior, float(scale), int(decay_mode), state_dot_a)
 
 
 def rl_infctx_chunk_fp32io16_forward(sequence_chunk_offsets, chunk_token_starts,

@@ -29,7 +29,7 @@ SIGNATURES = {
     "frwkv_last_error": [],
     "frwkv_metadata_validate": [_VP, _VP, _I32, _I32, _I32, _VP, _VP, _VP, _VP],
     "frwkv_recurrent_forward": [_INT, _INT] + [_I32] * 6 + [_VP] * 12 + [_F32, _VP],
-    "frwkv_split_scratch_bytes": [_INT] + [_I32] * 5,
+    "frwkv_split_scratch_bytes": [_INT] * 3 + [_I32] * 5,
     "frwkv_recurrent_forward_split": [_INT, _INT] + [_I32] * 6 + [_VP] * 12
                                      + [_F32, _VP, _SZ, _VP],
     "frwkv_chunk_forward": [_INT] * 3 + [_I32] * 5 + [_VP] * 12 + [_F32, _VP],
@@ -41,11 +41,15 @@ SIGNATURES = {
     "frwkv_statetune_interior_bytes": [_I32] * 3,
     "frwkv_statetune_interior": [_INT] * 2 + [_I32] * 4 + [_VP] * 11 + [_VP],
     "frwkv_statetune_backward": [_INT] * 2 + [_I32] * 5 + [_VP] * 22 + [_SZ, _F32, _VP],
+    "frwkv_statetune_backward_split": [_INT] * 2 + [_I32] * 5 + [_VP] * 22
+                                      + [_SZ, _F32, _VP, _VP, _SZ, _VP],
     "frwkv_statetune_backward_workspace_bytes": [_I32] * 3 + [_INT],
     "frwkv_statetune_backward_noalloc": [_INT] * 2 + [_I32] * 5 + [_VP] * 21 + [_F32, _VP],
     "frwkv_pretrain_forward": [_INT] * 2 + [_I32] * 4 + [_VP] * 10,
     "frwkv_pretrain_forward_split": [_INT] * 2 + [_I32] * 4 + [_VP] * 10 + [_SZ, _VP],
     "frwkv_pretrain_backward": [_INT] * 2 + [_I32] * 4 + [_VP] * 15 + [_SZ, _VP],
+    "frwkv_pretrain_backward_split": [_INT] * 2 + [_I32] * 4 + [_VP] * 15
+                                     + [_SZ, _VP, _VP, _SZ, _VP],
     "frwkv_pretrain_backward_workspace_bytes": [_I32] * 4,
     "frwkv_chunk_replay": [_INT] * 2 + [_I32] * 4 + [_VP] * 12 + [_F32, _VP],
     "frwkv_recurrent_fp16_forward": [_I32] * 6 + [_VP] * 13 + [_F32, _VP],

@@ -276,10 +276,11 @@ Tensor workspace_like(const Tensor& like, size_t bytes) {
 
 // Scratch of a split call (undefined when the call does not split); total and
 // longest as for frwkv_split_scratch_bytes.
-Tensor split_scratch(int kernel, int64_t sequences, int64_t heads, int64_t head_size,
-                     int64_t total, int64_t longest, const Tensor& like) {
+Tensor split_scratch(int kernel, int decay_mode, int64_t sequences, int64_t heads,
+                     int64_t head_size, int64_t total, int64_t longest, const Tensor& like) {
   return workspace_like(like, frwkv_split_scratch_bytes(
-                                  kernel, static_cast<int32_t>(sequences),
+                                  kernel, io_code(like.scalar_type()), decay_mode,
+                                  static_cast<int32_t>(sequences),
                                   static_cast<int32_t>(heads), static_cast<int32_t>(head_size),
                                   static_cast<int32_t>(total), static_cast<int32_t>(longest)));
 }
@@ -385,11 +386,11 @@ void recurrent_impl(const Tensor& cu, const Tensor& slots, Tensor& state,
       (g_recurrent_long_route.load(std::memory_order_relaxed) == 1 || stream_is_capturing(state))) {
     max_seqlen = -1;
   }
-  // Long bf16 sequences run on the chunk kernel, split when there are few.
+  // Long sequences run faster with scratch (frwkv_split_scratch_bytes).
   Tensor scratch;
-  if (max_seqlen >= 64 && r.scalar_type() == at::kBFloat16) {
-    scratch = split_scratch(FRWKV_SPLIT_RECURRENT, slots.numel(), state.size(1), state.size(2),
-                            r.size(0), max_seqlen, r);
+  if (max_seqlen > 2) {
+    scratch = split_scratch(FRWKV_SPLIT_RECURRENT, decay_mode, slots.numel(), state.size(1),
+                            state.size(2), r.size(0), max_seqlen, r);
   }
   check_rc(frwkv_recurrent_forward_split(
       io_code(r.scalar_type()), decay_mode, static_cast<int32_t>(slots.numel()),
@@ -516,7 +517,8 @@ void chunk_impl(const Tensor& r, const Tensor& decay, const Tensor& k, const Ten
   const int32_t longest =
       static_cast<int32_t>(max_seqlen > 0 ? std::min(max_seqlen, r.size(0)) : mean);
   const Tensor scratch =
-      split_scratch(FRWKV_SPLIT_CHUNK, slots.numel(), r.size(1), 64, r.size(0), longest, r);
+      split_scratch(FRWKV_SPLIT_CHUNK, decay_mode, slots.numel(), r.size(1), 64, r.size(0), longest,
+                    r);
   check_rc(frwkv_chunk_forward_split(
       io_code(r.scalar_type()), decay_mode, pool_code, static_cast<int32_t>(slots.numel()),
       static_cast<int32_t>(r.size(1)), 64, static_cast<int32_t>(r.size(0)),
@@ -628,8 +630,8 @@ void statetune_forward_impl(const Tensor& offsets, const Tensor& starts, const T
   float* interior_ptr = checked_interior(interior, r, d);
   c10::DeviceGuard guard(state.device());
   refuse_capture(r, "the StateTune forward");
-  const Tensor scratch = split_scratch(FRWKV_SPLIT_CALLER_CHUNKS, state.size(0), state.size(1), d,
-                                       starts.numel(), /*longest=*/0, r);
+  const Tensor scratch = split_scratch(FRWKV_SPLIT_CALLER_CHUNKS, decay_mode, state.size(0),
+                                       state.size(1), d, starts.numel(), r.size(0), r);
   check_rc(frwkv_statetune_forward_split(
       io_code(r.scalar_type()), decay_mode, static_cast<int32_t>(state.size(0)),
       static_cast<int32_t>(state.size(1)), static_cast<int32_t>(d), static_cast<int32_t>(r.size(0)),
@@ -676,7 +678,8 @@ void statetune_backward_impl(const Tensor& offsets, const Tensor& starts, const 
                              std::optional<Tensor> grad_v, std::optional<Tensor> grad_a,
                              std::optional<Tensor> grad_b,
                              std::optional<Tensor> grad_initial_state, int64_t num_sequences,
-                             const std::optional<Tensor>& interior, double scale,
+                             const std::optional<Tensor>& interior,
+                             const std::optional<Tensor>& state_dot_a, double scale,
                              int decay_mode) {
   TORCH_CHECK(std::isfinite(scale), "scale must be finite");
   check_chunk_tokens(r, decay, k, v, a, b, /*bf16_only=*/false, /*any_head_size=*/true);
@@ -731,17 +734,33 @@ void statetune_backward_impl(const Tensor& offsets, const Tensor& starts, const 
                   grad_initial_state->numel() == num_sequences * heads * d * d,
               "grad_initial_state must have shape [B,H,D,D] float32");
   const float* interior_ptr = checked_interior(interior, r, d);
+  const float* sda_ptr = nullptr;
+  if (state_dot_a.has_value() && state_dot_a->defined()) {
+    check_device_contiguous(*state_dot_a, "state_dot_a");
+    check_same_device(r, *state_dot_a, "state_dot_a");
+    TORCH_CHECK(state_dot_a->scalar_type() == at::kFloat && state_dot_a->sizes() == r.sizes(),
+                "state_dot_a must have shape [total_tokens,H,D] float32");
+    sda_ptr = state_dot_a->data_ptr<float>();
+  }
   c10::DeviceGuard guard(r.device());
   refuse_capture(r, "the StateTune backward");
   const bool has_dy = grad_output.has_value() && grad_output->defined();
   const bool has_ds = grad_final_state.has_value() && grad_final_state->defined();
   // Without the forward's interior states the call recomputes them into the
   // workspace (chunks longer than one piece only), so any chunk length works.
-  const size_t ws_bytes = frwkv_statetune_backward_workspace_bytes(
-      static_cast<int32_t>(d), static_cast<int32_t>(heads), static_cast<int32_t>(r.size(0)),
-      interior_ptr != nullptr);
+  Tensor scratch;
+  if (d == 64 || (sda_ptr != nullptr && interior_ptr != nullptr)) {
+    scratch = split_scratch(FRWKV_SPLIT_CALLER_CHUNKS_BACKWARD, decay_mode, num_sequences, heads, d,
+                            starts.numel(), r.size(0), r);
+  }
+  const size_t ws_bytes =
+      d == 256 && scratch.defined()
+          ? 0
+          : frwkv_statetune_backward_workspace_bytes(
+                static_cast<int32_t>(d), static_cast<int32_t>(heads),
+                static_cast<int32_t>(r.size(0)), interior_ptr != nullptr);
   Tensor ws = workspace_like(r, ws_bytes);
-  check_rc(frwkv_statetune_backward(
+  check_rc(frwkv_statetune_backward_split(
       io_code(r.scalar_type()), decay_mode, static_cast<int32_t>(num_sequences),
       static_cast<int32_t>(heads), static_cast<int32_t>(d), static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(starts.numel()), offsets.data_ptr<int32_t>(),
@@ -750,7 +769,8 @@ void statetune_backward_impl(const Tensor& offsets, const Tensor& starts, const 
       a.data_ptr(), b.data_ptr(), has_dy ? grad_output->data_ptr() : nullptr,
       has_ds ? grad_final_state->data_ptr<float>() : nullptr, gr, gd, gk, gv, ga, gb,
       grad_initial_state->data_ptr<float>(), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
-      static_cast<float>(scale), current_stream(r)));
+      static_cast<float>(scale), sda_ptr, scratch_ptr(scratch), scratch_size(scratch),
+      current_stream(r)));
 }
 
 void statetune_recurrent_fp32io16_backward(
@@ -765,7 +785,7 @@ void statetune_recurrent_fp32io16_backward(
   statetune_backward_impl(offsets, starts, ends, r, decay_logits, k, v, a, b, grad_output,
                           grad_final_state, boundary, grad_r, grad_decay_logits, grad_k,
                           grad_v, grad_a, grad_b, grad_initial_state, final_state.size(0),
-                          std::nullopt, scale, FRWKV_DECAY_LOGITS);
+                          std::nullopt, std::nullopt, scale, FRWKV_DECAY_LOGITS);
 }
 
 void statetune_backward_internal(
@@ -773,13 +793,14 @@ void statetune_backward_internal(
     Tensor a, Tensor b, std::optional<Tensor> grad_output,
     std::optional<Tensor> grad_final_state, Tensor boundary, Tensor grad_r, Tensor grad_decay,
     Tensor grad_k, Tensor grad_v, Tensor grad_a, Tensor grad_b, Tensor grad_initial_state,
-    std::optional<Tensor> interior, double scale, int64_t decay_mode) {
+    std::optional<Tensor> interior, double scale, int64_t decay_mode,
+    std::optional<Tensor> state_dot_a) {
   TORCH_CHECK(decay_mode == FRWKV_DECAY_LOGITS || decay_mode == FRWKV_DECAY_RAW_W,
               "decay_mode must be 0 (logits) or 1 (raw retention)");
   statetune_backward_impl(offsets, starts, ends, r, decay, k, v, a, b, grad_output,
                           grad_final_state, boundary, grad_r, grad_decay, grad_k, grad_v,
                           grad_a, grad_b, grad_initial_state, offsets.numel() - 1, interior,
-                          scale, static_cast<int>(decay_mode));
+                          state_dot_a, scale, static_cast<int>(decay_mode));
 }
 
 // ---------------------------------------------------------------------------
@@ -835,8 +856,8 @@ void clampw_forward(Tensor r, Tensor w, Tensor k, Tensor v, Tensor a, Tensor b, 
   c10::DeviceGuard guard(r.device());
   refuse_capture(r, "the clampw-v3 pretraining forward");
   const Tensor scratch =
-      split_scratch(FRWKV_SPLIT_CHUNK, r.size(0), r.size(2), head_size, r.size(0) * r.size(1),
-                    r.size(1), r);
+      split_scratch(FRWKV_SPLIT_CHUNK, FRWKV_DECAY_LOGITS, r.size(0), r.size(2), head_size,
+                    r.size(0) * r.size(1), r.size(1), r);
   check_rc(frwkv_pretrain_forward_split(
       io_code(r.scalar_type()), FRWKV_DECAY_LOGITS, static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(r.size(1)), static_cast<int32_t>(r.size(2)),
@@ -853,18 +874,25 @@ void clampw_backward(Tensor r, Tensor w, Tensor k, Tensor v, Tensor a, Tensor b,
                        {&da, "da"}, {&db, "db"}}, head_size);
   check_clampw_side(r, s, sa);
   c10::DeviceGuard guard(r.device());
-  const size_t ws_bytes = frwkv_pretrain_backward_workspace_bytes(
-      static_cast<int32_t>(r.size(0)), static_cast<int32_t>(r.size(1)),
-      static_cast<int32_t>(r.size(2)), static_cast<int32_t>(head_size));
   refuse_capture(r, "the clampw-v3 pretraining backward");
+  const Tensor scratch =
+      split_scratch(FRWKV_SPLIT_PRETRAIN_BACKWARD, FRWKV_DECAY_LOGITS, r.size(0), r.size(2),
+                    head_size, r.size(0) * r.size(1), r.size(1), r);
+  const size_t ws_bytes =
+      head_size == 256 && scratch.defined()
+          ? 0
+          : frwkv_pretrain_backward_workspace_bytes(
+                static_cast<int32_t>(r.size(0)), static_cast<int32_t>(r.size(1)),
+                static_cast<int32_t>(r.size(2)), static_cast<int32_t>(head_size));
   Tensor ws = workspace_like(r, ws_bytes);
-  check_rc(frwkv_pretrain_backward(
+  check_rc(frwkv_pretrain_backward_split(
       io_code(r.scalar_type()), FRWKV_DECAY_LOGITS, static_cast<int32_t>(r.size(0)),
       static_cast<int32_t>(r.size(1)), static_cast<int32_t>(r.size(2)),
       static_cast<int32_t>(head_size), r.data_ptr(), w.data_ptr(), k.data_ptr(), v.data_ptr(),
       a.data_ptr(), b.data_ptr(), dy.data_ptr(), s.data_ptr<float>(), dr.data_ptr(),
       dw.data_ptr(), dk.data_ptr(), dv.data_ptr(), da.data_ptr(), db.data_ptr(),
-      ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(r)));
+      ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, sa.data_ptr<float>(),
+      scratch_ptr(scratch), scratch_size(scratch), current_stream(r)));
 }
 
 // ---------------------------------------------------------------------------
@@ -1517,7 +1545,7 @@ TORCH_LIBRARY(flashrwkv2, m) {
       "Tensor b, Tensor? grad_output, Tensor? grad_final_state, Tensor boundary, "
       "Tensor(a!) grad_r, Tensor(b!) grad_decay, Tensor(c!) grad_k, Tensor(d!) grad_v, "
       "Tensor(e!) grad_a, Tensor(f!) grad_b, Tensor(g!) grad_initial_state, "
-      "Tensor? interior, float scale, int decay_mode) -> ()",
+      "Tensor? interior, float scale, int decay_mode, Tensor? state_dot_a=None) -> ()",
       &statetune_backward_internal);
   m.def(
       "rl_infctx_chunk_fp32io16_forward(Tensor sequence_chunk_offsets, Tensor chunk_token_starts, "

@@ -66,6 +66,7 @@
 
 #include "capi_internal.h"
 #include "chunk_common.h"
+#include "piece32.h"
 
 namespace frwkv {
 namespace {
@@ -159,23 +160,6 @@ __device__ __forceinline__ const uint16_t* tri_blk(const uint16_t* m, int p, int
   return m + tri_index(p, q) * kTriBlock;
 }
 
-// Inclusive prefix / suffix sums over the 16 lanes of a DPP row.
-template <int N>
-__device__ __forceinline__ float row_shr_add(float x) {
-  return x + __int_as_float(
-                 __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x110 + N, 0xf, 0xf, true));
-}
-template <int N>
-__device__ __forceinline__ float row_shl_add(float x) {
-  return x + __int_as_float(
-                 __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x100 + N, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float prefix16(float x) {
-  return row_shr_add<8>(row_shr_add<4>(row_shr_add<2>(row_shr_add<1>(x))));
-}
-__device__ __forceinline__ float suffix16(float x) {
-  return row_shl_add<8>(row_shl_add<4>(row_shl_add<2>(row_shl_add<1>(x))));
-}
 // Stores a C-layout block (lane (g, n) holds X[4g + j][n]) into a row-major
 // [row][col] bf16 tile at dst: four 2-byte stores per lane, the 16 lanes of a
 // group writing 32 consecutive bytes of one row.
@@ -1409,6 +1393,24 @@ extern "C" int frwkv_statetune_backward(
     const float* grad_final_state, void* grad_r, void* grad_decay, void* grad_k, void* grad_v,
     void* grad_a, void* grad_b, float* grad_initial_state, void* workspace,
     size_t workspace_bytes, float scale, void* stream) {
+  return frwkv_statetune_backward_split(
+      io_dtype, decay_mode, num_sequences, num_heads, head_size, total_tokens, num_chunks,
+      sequence_chunk_offsets, chunk_token_starts, chunk_token_ends, boundary, interior, r, decay,
+      decay_bias, k, v, a, b, grad_output, grad_final_state, grad_r, grad_decay, grad_k, grad_v,
+      grad_a, grad_b, grad_initial_state, workspace, workspace_bytes, scale,
+      /*state_dot_a=*/nullptr, nullptr, 0, stream);
+}
+
+extern "C" int frwkv_statetune_backward_split(
+    int io_dtype, int decay_mode, int32_t num_sequences, int32_t num_heads, int32_t head_size,
+    int32_t total_tokens, int32_t num_chunks, const int32_t* sequence_chunk_offsets,
+    const int32_t* chunk_token_starts, const int32_t* chunk_token_ends, const float* boundary,
+    const float* interior, const void* r, const void* decay, const void* decay_bias,
+    const void* k, const void* v, const void* a, const void* b, const void* grad_output,
+    const float* grad_final_state, void* grad_r, void* grad_decay, void* grad_k, void* grad_v,
+    void* grad_a, void* grad_b, float* grad_initial_state, void* workspace,
+    size_t workspace_bytes, float scale, const float* state_dot_a, void* scratch,
+    size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   if (!sequence_chunk_offsets || !chunk_token_starts || !chunk_token_ends || !boundary || !r ||
       !decay || !k || !v || !a || !b || !grad_r || !grad_decay || !grad_k || !grad_v ||
@@ -1426,6 +1428,42 @@ extern "C" int frwkv_statetune_backward(
   if (head_size != 64 && head_size != 128 && head_size != 256) {
     return set_error(FRWKV_ERR_UNSUPPORTED, "head size must be 64, 128, or 256, got %d",
                      head_size);
+  }
+  // Head size 256 with the forward's interior states and a^T S: the fp32 matrix
+  // form, in the scratch alone.
+  if (head_size == 256 && interior != nullptr && state_dot_a != nullptr && scratch != nullptr &&
+      decay_mode == FRWKV_DECAY_LOGITS &&
+      (io_dtype == FRWKV_DTYPE_BF16 || io_dtype == FRWKV_DTYPE_F16) &&
+      scratch_bytes >= piece32_backward_bytes(num_heads, total_tokens, num_chunks)) {
+    Piece32Params q{};
+    q.num_heads = num_heads;
+    q.num_sequences = num_sequences;
+    q.total_tokens = total_tokens;
+    q.seg_offsets = sequence_chunk_offsets;
+    q.seg_starts = chunk_token_starts;
+    q.seg_ends = chunk_token_ends;
+    q.num_segments = num_chunks;
+    q.r = r;
+    q.decay = decay;
+    q.bias = decay_bias;
+    q.k = k;
+    q.v = v;
+    q.a = a;
+    q.b = b;
+    q.scale = scale;
+    q.boundary = const_cast<float*>(boundary);
+    q.interior = const_cast<float*>(interior);
+    q.state_dot_a = const_cast<float*>(state_dot_a);
+    q.dy = grad_output;
+    q.dstate_final = grad_final_state;
+    q.dr = grad_r;
+    q.ddecay = grad_decay;
+    q.dk = grad_k;
+    q.dv = grad_v;
+    q.da = grad_a;
+    q.db = grad_b;
+    q.dstate0 = grad_initial_state;
+    return piece32_backward(q, io_dtype, scratch, static_cast<hipStream_t>(stream));
   }
   // Workspace: the gradient slices (head size 256), then, when interior is
   // null, the interior states this call recomputes from the boundaries. A
@@ -1502,6 +1540,23 @@ extern "C" int frwkv_pretrain_backward(int io_dtype, int decay_mode, int32_t bat
                                        void* grad_r, void* grad_decay, void* grad_k,
                                        void* grad_v, void* grad_a, void* grad_b,
                                        void* workspace, size_t workspace_bytes, void* stream) {
+  return frwkv_pretrain_backward_split(io_dtype, decay_mode, batch, tokens, num_heads, head_size,
+                                       r, decay, k, v, a, b, grad_output, boundary, grad_r,
+                                       grad_decay, grad_k, grad_v, grad_a, grad_b, workspace,
+                                       workspace_bytes, /*state_dot_a=*/nullptr, nullptr, 0,
+                                       stream);
+}
+
+extern "C" int frwkv_pretrain_backward_split(int io_dtype, int decay_mode, int32_t batch,
+                                       int32_t tokens, int32_t num_heads, int32_t head_size,
+                                       const void* r, const void* decay, const void* k,
+                                       const void* v, const void* a, const void* b,
+                                       const void* grad_output, const float* boundary,
+                                       void* grad_r, void* grad_decay, void* grad_k,
+                                       void* grad_v, void* grad_a, void* grad_b,
+                                       void* workspace, size_t workspace_bytes,
+                                       const float* state_dot_a, void* scratch,
+                                       size_t scratch_bytes, void* stream) {
   using namespace frwkv;
   if (!boundary || !r || !decay || !k || !v || !a || !b || !grad_output || !grad_r ||
       !grad_decay || !grad_k || !grad_v || !grad_a || !grad_b) {
@@ -1515,6 +1570,33 @@ extern "C" int frwkv_pretrain_backward(int io_dtype, int decay_mode, int32_t bat
   }
   if (static_cast<int64_t>(batch) * tokens > INT32_MAX) {
     return set_error(FRWKV_ERR_INVALID_ARGUMENT, "frwkv_pretrain_backward: B * T too large");
+  }
+  if (head_size == 256 && state_dot_a != nullptr && scratch != nullptr &&
+      decay_mode == FRWKV_DECAY_LOGITS &&
+      (io_dtype == FRWKV_DTYPE_BF16 || io_dtype == FRWKV_DTYPE_F16) &&
+      scratch_bytes >= piece32_backward_bytes(num_heads, batch * tokens, batch)) {
+    Piece32Params q{};
+    q.num_heads = num_heads;
+    q.num_sequences = batch;
+    q.total_tokens = batch * tokens;
+    q.dense_t = tokens;
+    q.r = r;
+    q.decay = decay;
+    q.k = k;
+    q.v = v;
+    q.a = a;
+    q.b = b;
+    q.scale = 1.0f;
+    q.boundary = const_cast<float*>(boundary);
+    q.state_dot_a = const_cast<float*>(state_dot_a);
+    q.dy = grad_output;
+    q.dr = grad_r;
+    q.ddecay = grad_decay;
+    q.dk = grad_k;
+    q.dv = grad_v;
+    q.da = grad_a;
+    q.db = grad_b;
+    return piece32_backward(q, io_dtype, scratch, static_cast<hipStream_t>(stream));
   }
   if (head_size == 128 || head_size == 256) {
     const size_t need = frwkv_train_slice_bytes(head_size, num_heads, batch * tokens);

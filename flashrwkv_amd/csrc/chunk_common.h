@@ -175,4 +175,22 @@ __device__ __forceinline__ float exclusive16(float incl, int n) {
   return n >= 1 ? y : 1.0f;
 }
 
+// Inclusive prefix / suffix sums over the 16 lanes of a DPP row.
+template <int N>
+__device__ __forceinline__ float row_shr_add(float x) {
+  return x + __int_as_float(
+                 __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x110 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ float row_shl_add(float x) {
+  return x + __int_as_float(
+                 __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x100 + N, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float prefix16(float x) {
+  return row_shr_add<8>(row_shr_add<4>(row_shr_add<2>(row_shr_add<1>(x))));
+}
+__device__ __forceinline__ float suffix16(float x) {
+  return row_shl_add<8>(row_shl_add<4>(row_shl_add<2>(row_shl_add<1>(x))));
+}
+
 }  // namespace frwkv

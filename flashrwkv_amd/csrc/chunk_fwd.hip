@@ -50,6 +50,7 @@
 #include "wkv7_mfma.h"
 #include "chunk_common.h"
 #include "chunk_parts.h"
+#include "piece32.h"
 
 namespace frwkv {
 namespace {
@@ -1240,11 +1241,32 @@ int check_token_pointers(const void* r, const void* decay, const void* k, const 
 }  // namespace
 }  // namespace frwkv
 
-extern "C" size_t frwkv_split_scratch_bytes(int kernel, int32_t num_sequences,
-                                            int32_t num_heads, int32_t head_size,
-                                            int32_t total, int32_t longest) {
+extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_mode,
+                                            int32_t num_sequences, int32_t num_heads,
+                                            int32_t head_size, int32_t total, int32_t longest) {
   using namespace frwkv;
-  if (head_size != 64 || num_sequences <= 0 || num_heads <= 0 || total <= 0) return 0;
+  if (num_sequences <= 0 || num_heads <= 0 || total <= 0) return 0;
+  if (kernel == FRWKV_SPLIT_RECURRENT &&
+      piece32_recurrent(io_dtype, decay_mode, head_size, longest)) {
+    const size_t bytes = piece32_forward_bytes(head_size, num_heads, total, num_sequences);
+    return bytes <= kPiece32RecurrentBytes ? bytes : 0;
+  }
+  if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS && kernel == FRWKV_SPLIT_CHUNK) {
+    return piece32_forward_bytes(head_size, num_heads, total, num_sequences);
+  }
+  if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS &&
+      kernel == FRWKV_SPLIT_CALLER_CHUNKS) {
+    return piece32_forward_bytes(head_size, num_heads, longest, total);
+  }
+  if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS) {
+    if (kernel == FRWKV_SPLIT_PRETRAIN_BACKWARD) {
+      return piece32_backward_bytes(num_heads, total, num_sequences);
+    }
+    if (kernel == FRWKV_SPLIT_CALLER_CHUNKS_BACKWARD) {
+      return piece32_backward_bytes(num_heads, longest, total);
+    }
+  }
+  if (head_size != 64) return 0;
   const int64_t units = static_cast<int64_t>(num_sequences) * num_heads;
   switch (kernel) {
     case FRWKV_SPLIT_CHUNK:
@@ -1368,6 +1390,33 @@ extern "C" int frwkv_statetune_forward_split(
   }
   if (!__builtin_isfinite(scale)) {
     return set_error(FRWKV_ERR_INVALID_ARGUMENT, "scale must be finite");
+  }
+  if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS && scratch != nullptr &&
+      (io_dtype == FRWKV_DTYPE_BF16 || io_dtype == FRWKV_DTYPE_F16) &&
+      scratch_bytes >= piece32_forward_bytes(head_size, num_heads, total_tokens, num_chunks)) {
+    Piece32Params q{};
+    q.num_heads = num_heads;
+    q.num_sequences = num_sequences;
+    q.total_tokens = total_tokens;
+    q.seg_offsets = sequence_chunk_offsets;
+    q.seg_starts = chunk_token_starts;
+    q.seg_ends = chunk_token_ends;
+    q.num_segments = num_chunks;
+    q.state = state;
+    q.state_slots = num_sequences;
+    q.r = r;
+    q.decay = decay;
+    q.bias = decay_bias;
+    q.k = k;
+    q.v = v;
+    q.a = a;
+    q.b = b;
+    q.out = output;
+    q.boundary = boundary;
+    q.interior = interior;
+    q.state_dot_a = state_dot_a;
+    q.scale = scale;
+    return piece32_forward(q, head_size, io_dtype, scratch, static_cast<hipStream_t>(stream));
   }
   if (head_size == 128 || head_size == 256) {
     return frwkv_train_recurrent_forward(io_dtype, decay_mode, num_sequences, num_heads,
@@ -1500,6 +1549,26 @@ extern "C" int frwkv_pretrain_forward_split(
   }
   if (static_cast<int64_t>(batch) * tokens > INT32_MAX) {
     return set_error(FRWKV_ERR_INVALID_ARGUMENT, "frwkv_pretrain_forward: B * T too large");
+  }
+  if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS && scratch != nullptr &&
+      (io_dtype == FRWKV_DTYPE_BF16 || io_dtype == FRWKV_DTYPE_F16) &&
+      scratch_bytes >= piece32_forward_bytes(head_size, num_heads, batch * tokens, batch)) {
+    Piece32Params q{};
+    q.num_heads = num_heads;
+    q.num_sequences = batch;
+    q.total_tokens = batch * tokens;
+    q.dense_t = tokens;
+    q.r = r;
+    q.decay = decay;
+    q.k = k;
+    q.v = v;
+    q.a = a;
+    q.b = b;
+    q.out = output;
+    q.boundary = boundary;
+    q.state_dot_a = state_dot_a;
+    q.scale = 1.0f;
+    return piece32_forward(q, head_size, io_dtype, scratch, static_cast<hipStream_t>(stream));
   }
   if (head_size == 128 || head_size == 256) {
     return frwkv_train_recurrent_forward(io_dtype, decay_mode, batch, num_heads, head_size,

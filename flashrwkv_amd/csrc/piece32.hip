@@ -1,0 +1,1048 @@
+// fp32 matrix form of the recurrence over 16-token pieces.
+//
+// The per-token kernels (recurrent.hip, train_recurrent.hip) do one dependent
+// step per token: about five VALU instructions per state element and a
+// reduction over the keys on the critical path. This file takes the chunk form
+// of chunk_fwd.hip with 16-token pieces and fp32 operands throughout, on the
+// fp32 matrix instruction (v_mfma_f32_16x16x4_f32, twice the rate of unpacked
+// fp32 VALU): per piece, with cumulative decays G (inclusive) and Gp
+// (exclusive), At = a 2^Gp, Rt = r 2^G, Bh = b 2^-G, Kh = k 2^-G,
+//   SA = T (At S0 + Lak V),  T = (I - Lab)^{-1},
+//   Y  = scale (Rt S0 + Arb SA + Ark V),
+//   S' = g (S0 + Bh^T SA + Kh^T V),  g = 2^G(last token).
+// Operands, sums and states are fp32, as in the per-token kernels; results
+// differ by the order of the sums. Decay logits only: their retention is at
+// least exp(-e^{-1/2}), so a piece's decay stays above 2^-14 and one reference
+// point serves a piece (raw retentions stay on the per-token kernels).
+//
+// Several kernels, so that the serial chain over pieces holds nothing but the
+// state products:
+//   piece32_prepare   every piece at once: decodes the rows, scans the decay
+//                     and writes the scaled tiles and the four triangles in
+//                     the operand layouts of the chain;
+//   piece32_forward   one wave per 64 keys x 16 value columns of a state,
+//                     walking the pieces; operands are read from the tiles
+//                     straight into registers, one piece ahead. Waves sharing
+//                     columns (D / 64 of them) add their key sums through LDS,
+//                     one barrier per piece; at D = 64 there is none;
+// and for the backward at D = 256, the same preparation, the adjoint chain
+// (piece32_adjoint_kernel) and every piece's gradients at once from its start
+// state and its adjoint (piece32_gradient_kernel).
+//
+// Operand layouts (16x16x4: A[m = n][k = g], B[k = g][n], C[m = 4g + j][n] for
+// lane (g, n)): step j of a 16-wide contraction takes k = 4g + j, so a 16 x 16
+// block as B operand is its C layout, and as A operand four consecutive
+// elements of one row.
+#include "capi_internal.h"
+#include "chunk_common.h"
+#include "piece32.h"
+
+namespace frwkv {
+namespace {
+
+constexpr int kPiece = 16;
+constexpr int kTriElems = kPiece * kPiece;
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// C += A B for 16 x 16 blocks in operand layouts.
+__device__ __forceinline__ f32x4 mm16(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c = mfma4(a[j], b[j], c);
+  return c;
+}
+
+// Tiles of one (piece, head), in floats.
+template <int D>
+struct Tiles {
+  static constexpr int kTile = kPiece * D;
+  // Forward: At, Rt [t][k]; Bh^T, Kh^T [k][t]; g [k]; T, Lak, Arb, Ark [t][i].
+  static constexpr int kAt = 0, kRt = kTile, kBhT = 2 * kTile, kKhT = 3 * kTile;
+  static constexpr int kG = 4 * kTile;
+  static constexpr int kTri = kG + D;
+  static constexpr int kForward = kTri + 4 * kTriElems;
+  // Backward: Bh, Kh [t][k]; At^T, Rt^T, Bh^T, Kh^T [k][t]; g [k]; T^T, Lak^T,
+  // Arb^T, Ark^T [i][t].
+  static constexpr int kBh = 0, kKh = kTile, kAtT = 2 * kTile, kRtT = 3 * kTile;
+  static constexpr int kBackBhT = 4 * kTile, kBackKhT = 5 * kTile;
+  static constexpr int kBackG = 6 * kTile;
+  static constexpr int kBackTri = kBackG + D;
+  static constexpr int kBackward = kBackTri + 4 * kTriElems;
+};
+
+// Pieces of sequence `seq`: slots first .. first + count - 1; with the packed
+// and dense layouts, piece i holds tokens begin + 16 i .. of [begin, end).
+struct Walk {
+  int first, count, begin, end;
+};
+__device__ __forceinline__ Walk walk_of(const Piece32Params& p, int seq) {
+  Walk w{0, 0, 0, 0};
+  if (p.seg_offsets != nullptr) {
+    const int lo = min(max(p.seg_offsets[seq], 0), p.num_segments);
+    const int hi = min(max(p.seg_offsets[seq + 1], lo), p.num_segments);
+    w.first = p.base[lo];
+    w.count = p.base[hi] - w.first;
+  } else if (p.dense_t > 0) {
+    w.begin = seq * p.dense_t;
+    w.end = w.begin + p.dense_t;
+    w.first = seq * (p.dense_t / kPiece);
+    w.count = p.dense_t / kPiece;
+  } else {
+    // floor(begin / 16) + seq: sequences of ascending, disjoint ranges then
+    // have disjoint slots.
+    w.begin = max(p.cu_seqlens[seq], 0);
+    w.end = min(p.cu_seqlens[seq + 1], p.total_tokens);
+    w.first = w.begin / kPiece + seq;
+    w.count = (max(w.end - w.begin, 0) + kPiece - 1) / kPiece;
+  }
+  w.first = uniform(w.first);
+  w.count = uniform(w.count);
+  w.begin = uniform(w.begin);
+  w.end = uniform(w.end);
+  return w;
+}
+// Piece i of a walk: {first token, tokens, caller chunk, piece of the chunk}.
+__device__ __forceinline__ int4 piece_at(const Piece32Params& p, const Walk& w, int i) {
+  if (p.seg_offsets != nullptr) {
+    const int4 e = p.table[w.first + i];
+    return make_int4(uniform(e.x), uniform(e.y), uniform(e.z), uniform(e.w));
+  }
+  const int start = w.begin + kPiece * i;
+  return make_int4(start, min(kPiece, w.end - start), 0, i);
+}
+
+// The packed sequence that owns a slot (or the last one that starts at or
+// before it): the first slots ascend, and every lane tries one of 64 equal
+// steps, so a batch of 64 sequences takes one round.
+__device__ __forceinline__ int sequence_of_slot(const Piece32Params& p, int slot, int lane) {
+  int lo = 0, hi = p.num_sequences;
+  while (hi - lo > 1) {
+    const int stride = (hi - lo + 63) / 64;
+    const int s = lo + lane * stride;
+    const bool before = s < hi && max(p.cu_seqlens[s], 0) / kPiece + s <= slot;
+    const int count = max(__builtin_popcountll(__builtin_amdgcn_ballot_w64(before)), 1);
+    lo = uniform(lo + (count - 1) * stride);
+    hi = min(lo + stride, hi);
+  }
+  return lo;
+}
+
+// Slots of the caller chunks' pieces in chunk order, one workgroup. Token
+// ranges are clamped to the call's; an empty chunk has one piece of no tokens
+// (its start state is an output too), and pieces beyond the slots (overlapping
+// chunks) are dropped.
+constexpr int kTableThreads = 1024;
+__global__ __launch_bounds__(kTableThreads) void piece32_table(Piece32Params p, int slots) {
+  __shared__ int sums[kTableThreads];
+  const int tid = threadIdx.x;
+  int before = 0;
+  for (int c0 = 0; c0 < p.num_segments; c0 += kTableThreads) {
+    const int c = c0 + tid;
+    int start = 0, len = 0;
+    if (c < p.num_segments) {
+      start = min(max(p.seg_starts[c], 0), p.total_tokens);
+      len = max(min(p.seg_ends[c], p.total_tokens) - start, 0);
+    }
+    const int count = c < p.num_segments ? max((len + kPiece - 1) / kPiece, 1) : 0;
+    sums[tid] = count;
+    __syncthreads();
+    for (int step = 1; step < kTableThreads; step *= 2) {
+      const int add = tid >= step ? sums[tid - step] : 0;
+      __syncthreads();
+      sums[tid] += add;
+      __syncthreads();
+    }
+    const int first = before + sums[tid] - count;
+    if (c < p.num_segments) {
+      p.base[c] = min(first, slots);
+      for (int i = 0; i < count && first + i < slots; ++i) {
+        p.table[first + i] = make_int4(start + kPiece * i, min(kPiece, len - kPiece * i), c, i);
+      }
+    }
+    before += sums[kTableThreads - 1];
+    __syncthreads();
+  }
+  if (tid == 0) p.base[p.num_segments] = min(before, slots);
+  for (int i = before + tid; i < slots; i += kTableThreads) p.table[i] = make_int4(0, 0, -1, 0);
+}
+
+// Four consecutive 16-bit values at a buffer offset, as loaded.
+__device__ __forceinline__ u32x2 load4(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ f32x4 widen4(u32x2 q) {
+  return f32x4{to_f32<T>(static_cast<uint16_t>(q.x)), to_f32<T>(static_cast<uint16_t>(q.x >> 16)),
+               to_f32<T>(static_cast<uint16_t>(q.y)), to_f32<T>(static_cast<uint16_t>(q.y >> 16))};
+}
+
+// Cumulative decay of a piece at token n of the lane's 16-lane row, from the
+// logits' log2 retentions: 2^G, 2^Gp and 2^-G of sums of logs. A sum of small
+// logs keeps the slow channels (the largest states) more exact than a product
+// of retentions near 1 (states 4.9e-7 off fp64 with the per-token product,
+// 5.7e-7 with a scanned one).
+struct Decay {
+  float sig;              // sigmoid of the logit
+  float incl, excl, inv;  // 2^G, 2^Gp, 2^-G
+};
+__device__ __forceinline__ Decay piece_decay(float logit, bool on) {
+  Decay d;
+  d.sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2E * logit));
+  const float sum = prefix16(on ? -(kExpNegHalf * kLog2E) * d.sig : 0.0f);
+  const float before = __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x111, 0xf, 0xf, true));
+  d.incl = __builtin_amdgcn_exp2f(sum);
+  d.excl = __builtin_amdgcn_exp2f(before);
+  d.inv = __builtin_amdgcn_exp2f(-sum);
+  return d;
+}
+
+// One workgroup of D / 64 waves per (piece, head); lane (g, n) of wave q holds
+// token n, keys 64q + 16kb + 4g .. +3, which is the A and the B operand layout
+// of the triangles' products over the keys.
+template <typename T, int D, bool kBackward>
+__global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
+  constexpr int kWaves = D / 64;
+  using L = Tiles<D>;
+  __shared__ f32x4 part[kWaves > 1 ? kWaves : 1][5][64];
+  if (p.status != nullptr && p.status[0] != 0) return;
+  const int heads = p.num_heads;
+  const int head = static_cast<int>(blockIdx.x) % heads;
+  const int index = static_cast<int>(blockIdx.x) / heads;
+  int slot, start, ntok;
+  if (p.seg_offsets != nullptr) {
+    slot = index;
+    const int4 e = p.table[slot];
+    start = uniform(e.x);
+    ntok = uniform(e.y);
+    if (e.z < 0) return;
+  } else {
+    slot = index;
+    const Walk w = walk_of(p, p.dense_t > 0 ? slot / (p.dense_t / kPiece)
+                                            : sequence_of_slot(p, slot, threadIdx.x & 63));
+    const int i = slot - w.first;
+    if (i >= w.count) return;
+    start = w.begin + kPiece * i;
+    ntok = min(kPiece, w.end - start);
+  }
+  const int wave = uniform(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const bool on = n < ntok;
+
+  using S16 = typename IoTraits<T>::storage;
+  const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
+  const int64_t row0 = (static_cast<int64_t>(start) * heads + head) * D;
+  auto rows = [&](const void* x) {
+    return buffer_rsrc(static_cast<const S16*>(x) + row0, static_cast<uint32_t>(ntok) * row_bytes);
+  };
+  const auto rw = rows(p.decay), ra = rows(p.a), rr = rows(p.r), rb = rows(p.b), rk = rows(p.k);
+  const uint32_t off = static_cast<uint32_t>(n) * row_bytes + 2 * (64 * wave + 4 * g);
+  u32x2 qw[4], qa[4], qr[4], qb[4], qk[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) qw[kb] = load4(rw, off + 32 * kb);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    qa[kb] = load4(ra, off + 32 * kb);
+    qr[kb] = load4(rr, off + 32 * kb);
+    qb[kb] = load4(rb, off + 32 * kb);
+    qk[kb] = load4(rk, off + 32 * kb);
+  }
+  float* const tiles = p.tiles + (static_cast<int64_t>(slot) * heads + head) *
+                                     (kBackward ? L::kBackward : L::kForward);
+  const int key0 = 64 * wave + 4 * g;  // + 16 kb + j
+  auto store_rows = [&](int tile, int key, f32x4 x) {  // [t][k]
+    *reinterpret_cast<f32x4*>(tiles + tile + n * D + key) = x;
+  };
+  auto store_cols = [&](int tile, int key, f32x4 x) {  // [k][t]
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tiles[tile + (key + j) * kPiece + n] = x[j];
+  };
+  f32x4 at[4], rt[4], bh[4], kh[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    f32x4 x = widen4<T>(qw[kb]);
+    if (p.bias != nullptr) {
+      const S16* bias = static_cast<const S16*>(p.bias) + static_cast<int64_t>(head) * D + key0 + 16 * kb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] += to_f32<T>(bias[j]);
+    }
+    const f32x4 av = widen4<T>(qa[kb]), rv = widen4<T>(qr[kb]), bv = widen4<T>(qb[kb]),
+                kv = widen4<T>(qk[kb]);
+    f32x4 total;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const Decay dec = piece_decay(x[j], on);
+      total[j] = dec.incl;
+      at[kb][j] = on ? av[j] * dec.excl : 0.0f;
+      rt[kb][j] = on ? rv[j] * dec.incl : 0.0f;
+      bh[kb][j] = on ? bv[j] * dec.inv : 0.0f;
+      kh[kb][j] = on ? kv[j] * dec.inv : 0.0f;
+    }
+    const int key = key0 + 16 * kb;
+    if (n == 15) {
+      *reinterpret_cast<f32x4*>(tiles + (kBackward ? L::kBackG : L::kG) + key) = total;
+    }
+    if constexpr (kBackward) {
+      store_rows(L::kBh, key, bh[kb]);
+      store_rows(L::kKh, key, kh[kb]);
+      store_cols(L::kAtT, key, at[kb]);
+      store_cols(L::kRtT, key, rt[kb]);
+      store_cols(L::kBackBhT, key, bh[kb]);
+      store_cols(L::kBackKhT, key, kh[kb]);
+    } else {
+      store_rows(L::kAt, key, at[kb]);
+      store_rows(L::kRt, key, rt[kb]);
+      store_cols(L::kBhT, key, bh[kb]);
+      store_cols(L::kKhT, key, kh[kb]);
+    }
+  }
+
+  // Triangles X[t][i] = sum_k X_t Y_i, as X^T in C layout (lane (g, n): row
+  // t = n, i = 4g + j), and Lab in C layout too for the inverse. The backward
+  // takes the transposed matrices: the same products with the operands
+  // exchanged (lane (g, n): i = n, t = 4g + j).
+  auto tri_product = [](f32x4 x, f32x4 y, f32x4 c) {
+    return kBackward ? mm16(x, y, c) : mm16(y, x, c);
+  };
+  f32x4 tri[5] = {zero4(), zero4(), zero4(), zero4(), zero4()};
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    tri[0] = mm16(bh[kb], at[kb], tri[0]);
+    tri[1] = mm16(at[kb], bh[kb], tri[1]);
+    tri[2] = tri_product(at[kb], kh[kb], tri[2]);
+    tri[3] = tri_product(rt[kb], bh[kb], tri[3]);
+    tri[4] = tri_product(rt[kb], kh[kb], tri[4]);
+  }
+  if constexpr (kWaves > 1) {
+#pragma unroll
+    for (int m = 0; m < 5; ++m) part[wave][m][lane] = tri[m];
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int q = 1; q < kWaves; ++q) {
+#pragma unroll
+      for (int m = 0; m < 5; ++m) tri[m] += part[q][m][lane];
+    }
+  }
+  f32x4 lab_r = tri[0], lab_c = tri[1], lak = tri[2], arb = tri[3], ark = tri[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = 4 * g + j;
+    lab_r[j] = i < n ? lab_r[j] : 0.0f;
+    lab_c[j] = n < i ? lab_c[j] : 0.0f;
+    const bool strict = kBackward ? n < i : i < n;  // source before target
+    lak[j] = strict ? lak[j] : 0.0f;
+    arb[j] = strict || i == n ? arb[j] : 0.0f;
+    ark[j] = strict || i == n ? ark[j] : 0.0f;
+  }
+  // L and L^T exchange their layouts: the inverse of I - L^T is T^T.
+  if constexpr (kBackward) {
+    const f32x4 x = lab_r;
+    lab_r = lab_c;
+    lab_c = x;
+  }
+  // (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8) for the strictly lower
+  // L. With X_R "lane (g, n) holds X[n][4g + j]" and X_C the C layout,
+  // Z = X Y is Z_C = X_R Y_C and Z_R = Y_C X_R.
+  const f32x4 p2c = mm16(lab_r, lab_c, zero4()), p2r = mm16(lab_c, lab_r, zero4());
+  const f32x4 p4c = mm16(p2r, p2c, zero4()), p4r = mm16(p2c, p2r, zero4());
+  const f32x4 p8c = mm16(p4r, p4c, zero4());
+  f32x4 t = lab_r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) t[j] += (4 * g + j == n) ? 1.0f : 0.0f;
+  t = mm16(p2c, t, t);
+  t = mm16(p4c, t, t);
+  t = mm16(p8c, t, t);
+  float* const out = tiles + (kBackward ? L::kBackTri : L::kTri) + n * kPiece + 4 * g;
+  *reinterpret_cast<f32x4*>(out) = t;
+  *reinterpret_cast<f32x4*>(out + kTriElems) = lak;
+  *reinterpret_cast<f32x4*>(out + 2 * kTriElems) = arb;
+  *reinterpret_cast<f32x4*>(out + 3 * kTriElems) = ark;
+}
+
+// The chain over a sequence's pieces. Wave: keys 64q .. +63 (q = wave % (D /
+// 64)), value columns col0 .. +15; S[kb][j] is key 64q + 16kb + 4g + j, column
+// col0 + n. kTrain: boundary, interior and a^T S outputs.
+template <typename T, int D, bool kTrain>
+__global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p) {
+  using L = Tiles<D>;
+  constexpr int kKeyWaves = D / 64;
+  constexpr int kSlabs = 4 / kKeyWaves;  // column slabs per workgroup
+  using S16 = typename IoTraits<T>::storage;
+  __shared__ f32x4 part[2][kKeyWaves > 1 ? 4 : 1][2][64];
+  if (p.status != nullptr && p.status[0] != 0) {
+    fill_nan<T>(static_cast<S16*>(p.out), p.out_elems);
+    return;
+  }
+  const int heads = p.num_heads;
+  const int units = p.num_sequences * heads;
+  // Blocks of one unit are `units` apart: on one XCD where that is a multiple
+  // of 8, so that they share its tiles' L2 lines.
+  const int unit = static_cast<int>(blockIdx.x) % units;
+  const int seq = unit / heads, head = unit % heads;
+  const int slot = uniform(p.slots != nullptr ? p.slots[seq] : seq);
+  if (p.state != nullptr && (slot < 0 || slot >= p.state_slots)) return;
+  const int wave = uniform(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int kq = wave % kKeyWaves;
+  const int col =
+      16 * (static_cast<int>(blockIdx.x) / units * kSlabs + wave / kKeyWaves) + n;
+  const int key0 = 64 * kq + 4 * g;  // + 16 kb + j
+  const Walk walk = walk_of(p, seq);
+
+  constexpr int64_t kState = static_cast<int64_t>(D) * D;
+  // Element (16 kb + j) * D floats after s_off; a null state reads as zero.
+  const uint32_t s_off = static_cast<uint32_t>(key0 * D + col) * 4;
+  float* const state =
+      p.state != nullptr ? p.state + (static_cast<int64_t>(slot) * heads + head) * kState : nullptr;
+  const auto state_rs = buffer_rsrc(state, state != nullptr ? static_cast<uint32_t>(kState) * 4 : 0u);
+  f32x4 S[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      S[kb][j] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(state_rs, s_off, (16 * kb + j) * D * 4, 0));
+    }
+  }
+  auto store_state = [&](float* dst) {
+    const auto rs = buffer_rsrc(dst, static_cast<uint32_t>(kState) * 4);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[kb][j]), rs, s_off,
+                                              (16 * kb + j) * D * 4, 0);
+      }
+    }
+  };
+
+  // A piece's operands: registers in operand layout.
+  struct Ops {
+    f32x4 at[4], rt[4], bt[4], kt[4];
+    f32x4 t, lak, arb, ark;
+    uint16_t v[4];  // V[4g + j][col]
+    int start, ntok, chunk, index;
+  };
+  const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
+  auto load = [&](Ops& o, int i) {
+    const int4 e = piece_at(p, walk, i);
+    o.start = e.x;
+    o.ntok = e.y;
+    o.chunk = e.z;
+    o.index = e.w;
+    const float* tiles =
+        p.tiles + (static_cast<int64_t>(walk.first + i) * heads + head) * L::kForward;
+    auto at4 = [&](int offset) { return *reinterpret_cast<const f32x4*>(tiles + offset); };
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      o.at[kb] = at4(L::kAt + n * D + key0 + 16 * kb);
+      o.rt[kb] = at4(L::kRt + n * D + key0 + 16 * kb);
+    }
+    const auto vs = buffer_rsrc(static_cast<const S16*>(p.v) +
+                                    (static_cast<int64_t>(e.x) * heads + head) * D,
+                                static_cast<uint32_t>(e.y) * row_bytes);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o.v[j] = __builtin_amdgcn_raw_buffer_load_b16(
+          vs, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
+    }
+    const int tri = L::kTri + n * kPiece + 4 * g;
+    o.lak = at4(tri + kTriElems);
+    o.t = at4(tri);
+    o.arb = at4(tri + 2 * kTriElems);
+    o.ark = at4(tri + 3 * kTriElems);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      const int key = 64 * kq + 16 * kb + n;
+      o.kt[kb] = at4(L::kKhT + key * kPiece + 4 * g);
+      o.bt[kb] = at4(L::kBhT + key * kPiece + 4 * g);
+    }
+  };
+
+  auto step = [&](const Ops& o, Ops& next, int i) {
+    f32x4 decay[4];  // read at the end of the step
+    {
+      const float* src = p.tiles +
+                         (static_cast<int64_t>(walk.first + i) * heads + head) * L::kForward +
+                         L::kG + key0;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) decay[kb] = *reinterpret_cast<const f32x4*>(src + 16 * kb);
+    }
+    if (i + 1 < walk.count) load(next, i + 1);
+    if constexpr (kTrain) {
+      if (p.dense_t > 0) {
+        store_state(p.boundary +
+                    ((static_cast<int64_t>(seq) * heads + head) * (p.dense_t / kPiece) + i) *
+                        kState);
+      } else if (o.index == 0) {
+        store_state(p.boundary + (static_cast<int64_t>(o.chunk) * heads + head) * kState);
+      } else if (p.interior != nullptr) {
+        store_state(p.interior +
+                    (static_cast<int64_t>(o.start / kPiece) * heads + head) * kState);
+      }
+    }
+    // Sums over the keys: two accumulators per product, so that consecutive
+    // matrix instructions do not wait for each other.
+    f32x4 rhs = zero4(), rhs2 = zero4(), y = zero4(), y2 = zero4();
+#pragma unroll
+    for (int kb = 0; kb < 4; kb += 2) {
+      rhs = mm16(o.at[kb], S[kb], rhs);
+      rhs2 = mm16(o.at[kb + 1], S[kb + 1], rhs2);
+      y = mm16(o.rt[kb], S[kb], y);
+      y2 = mm16(o.rt[kb + 1], S[kb + 1], y2);
+    }
+    rhs += rhs2;
+    y += y2;
+    if constexpr (kKeyWaves > 1) {
+      // Double-buffered: the next piece's barrier separates this read from
+      // the write after it.
+      part[i & 1][wave][0][lane] = rhs;
+      part[i & 1][wave][1][lane] = y;
+      __syncthreads();
+      const int first = wave - kq;
+      rhs = part[i & 1][first][0][lane];
+      y = part[i & 1][first][1][lane];
+#pragma unroll
+      for (int q = 1; q < kKeyWaves; ++q) {
+        rhs += part[i & 1][first + q][0][lane];
+        y += part[i & 1][first + q][1][lane];
+      }
+    }
+    f32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = to_f32<T>(o.v[j]);
+    rhs = mm16(o.lak, v, rhs);
+    const f32x4 sa = mm16(o.t, rhs, zero4());
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] = mm16(o.kt[kb], v, S[kb]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] = mm16(o.bt[kb], sa, S[kb]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] *= decay[kb];
+    if (kq == 0) {
+      y = mm16(o.ark, v, y);
+      y = mm16(o.arb, sa, y);
+      const int64_t base = (static_cast<int64_t>(o.start) * heads + head) * D;
+      const auto ys = buffer_rsrc(static_cast<S16*>(p.out) + base,
+                                  static_cast<uint32_t>(o.ntok) * row_bytes);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b16(
+            from_f32<T>(p.scale * y[j]), ys,
+            static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
+      }
+      if constexpr (kTrain) {
+        const auto sas = buffer_rsrc(p.state_dot_a + base,
+                                     static_cast<uint32_t>(o.ntok) * 2 * row_bytes);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          __builtin_amdgcn_raw_buffer_store_b32(
+              __float_as_uint(sa[j]), sas,
+              static_cast<uint32_t>(4 * g + j) * 2 * row_bytes + 4 * col, 0, 0);
+        }
+      }
+    }
+  };
+
+  Ops even, odd;
+  if (walk.count > 0) load(even, 0);
+  for (int i = 0; i < walk.count; i += 2) {
+    step(even, odd, i);
+    if (i + 1 < walk.count) step(odd, even, i + 1);
+  }
+  if (state != nullptr) store_state(state);
+}
+
+// The adjoint chain (head size 256), pieces in reverse. Same wave layout as the
+// forward: dS[kb][j] is dL/dS of key 64q + 16kb + 4g + j, column col0 + n, at
+// the end of the current piece; it goes to p.adjoints for the gradient kernel.
+// Per piece, with dU = g o dS and dYs = scale dY:
+//   dSA = Bh dU + Arb^T dYs,  dZ = T^T dSA,
+//   dV  = Kh dU + Ark^T dYs + Lak^T dZ,  dS <- dU + Rt^T dYs + At^T dZ.
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p) {
+  using L = Tiles<D>;
+  constexpr int kKeyWaves = D / 64;
+  static_assert(kKeyWaves == 4, "one column slab per workgroup");
+  using S16 = typename IoTraits<T>::storage;
+  __shared__ f32x4 part[2][kKeyWaves][2][64];
+  const int heads = p.num_heads;
+  const int units = p.num_sequences * heads;
+  const int unit = static_cast<int>(blockIdx.x) % units;
+  const int seq = unit / heads, head = unit % heads;
+  const int kq = uniform(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int col = 16 * (static_cast<int>(blockIdx.x) / units) + n;
+  const int key0 = 64 * kq + 4 * g;
+  const Walk walk = walk_of(p, seq);
+  constexpr uint32_t kState = D * D;
+  const uint32_t s_off = static_cast<uint32_t>(key0 * D + col) * 4;
+  auto state_rs = [&](const float* base, int64_t index) {
+    return buffer_rsrc(base != nullptr ? base + index * kState : nullptr,
+                       base != nullptr ? kState * 4 : 0u);
+  };
+  f32x4 dS[4];
+  {
+    const auto rs = state_rs(p.dstate_final, unit);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        dS[kb][j] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rs, s_off, (16 * kb + j) * D * 4, 0));
+      }
+    }
+  }
+  auto store_adjoint = [&](float* base, int64_t index) {
+    const auto rs = state_rs(base, index);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dS[kb][j]), rs, s_off,
+                                              (16 * kb + j) * D * 4, 0);
+      }
+    }
+  };
+
+  struct Ops {
+    f32x4 bh[4], kh[4], at[4], rt[4];
+    f32x4 t, lak, arb, ark;
+    uint16_t dy[4];  // dY[4g + j][col]
+    int start, ntok;
+  };
+  const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
+  auto load = [&](Ops& o, int i) {
+    const int4 e = piece_at(p, walk, i);
+    o.start = e.x;
+    o.ntok = e.y;
+    const float* tiles =
+        p.tiles + (static_cast<int64_t>(walk.first + i) * heads + head) * L::kBackward;
+    auto at4 = [&](int offset) { return *reinterpret_cast<const f32x4*>(tiles + offset); };
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      o.bh[kb] = at4(L::kBh + n * D + key0 + 16 * kb);
+      o.kh[kb] = at4(L::kKh + n * D + key0 + 16 * kb);
+    }
+    const bool ok = p.dy != nullptr;
+    const auto ds = buffer_rsrc(ok ? static_cast<const S16*>(p.dy) +
+                                         (static_cast<int64_t>(e.x) * heads + head) * D
+                                   : nullptr,
+                                ok ? static_cast<uint32_t>(e.y) * row_bytes : 0u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o.dy[j] = __builtin_amdgcn_raw_buffer_load_b16(
+          ds, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
+    }
+    const int tri = L::kBackTri + n * kPiece + 4 * g;
+    o.t = at4(tri);
+    o.lak = at4(tri + kTriElems);
+    o.arb = at4(tri + 2 * kTriElems);
+    o.ark = at4(tri + 3 * kTriElems);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      const int key = 64 * kq + 16 * kb + n;
+      o.rt[kb] = at4(L::kRtT + key * kPiece + 4 * g);
+      o.at[kb] = at4(L::kAtT + key * kPiece + 4 * g);
+    }
+  };
+
+  auto step = [&](const Ops& o, Ops& next, int i) {
+    const int64_t ph = static_cast<int64_t>(walk.first + i) * heads + head;
+    f32x4 decay[4];
+    {
+      const float* src = p.tiles + ph * L::kBackward + L::kBackG + key0;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) decay[kb] = *reinterpret_cast<const f32x4*>(src + 16 * kb);
+    }
+    if (i > 0) load(next, i - 1);
+    store_adjoint(p.adjoints, ph);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) dS[kb] *= decay[kb];  // dU
+    f32x4 dsa = zero4(), dsa2 = zero4(), dv = zero4(), dv2 = zero4();
+#pragma unroll
+    for (int kb = 0; kb < 4; kb += 2) {
+      dsa = mm16(o.bh[kb], dS[kb], dsa);
+      dsa2 = mm16(o.bh[kb + 1], dS[kb + 1], dsa2);
+      dv = mm16(o.kh[kb], dS[kb], dv);
+      dv2 = mm16(o.kh[kb + 1], dS[kb + 1], dv2);
+    }
+    part[i & 1][kq][0][lane] = dsa + dsa2;
+    part[i & 1][kq][1][lane] = dv + dv2;
+    __syncthreads();
+    dsa = part[i & 1][0][0][lane];
+    dv = part[i & 1][0][1][lane];
+#pragma unroll
+    for (int q = 1; q < kKeyWaves; ++q) {
+      dsa += part[i & 1][q][0][lane];
+      dv += part[i & 1][q][1][lane];
+    }
+    f32x4 dy;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dy[j] = p.scale * to_f32<T>(o.dy[j]);
+    dsa = mm16(o.arb, dy, dsa);
+    const f32x4 dz = mm16(o.t, dsa, zero4());
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) dS[kb] = mm16(o.rt[kb], dy, dS[kb]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) dS[kb] = mm16(o.at[kb], dz, dS[kb]);
+    if (kq == 0) {
+      dv = mm16(o.ark, dy, dv);
+      dv = mm16(o.lak, dz, dv);
+      const auto vs = buffer_rsrc(static_cast<S16*>(p.dv) +
+                                      (static_cast<int64_t>(o.start) * heads + head) * D,
+                                  static_cast<uint32_t>(o.ntok) * row_bytes);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b16(
+            from_f32<T>(dv[j]), vs, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
+      }
+    } else if (kq == 1) {
+      float* dst = p.dz + ph * (kPiece * D) + (4 * g) * D + col;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[j * D] = dz[j];
+    }
+  };
+
+  Ops even, odd;
+  if (walk.count > 0) load(even, walk.count - 1);
+  for (int i = walk.count - 1; i >= 0; i -= 2) {
+    step(even, odd, i);
+    if (i > 0) step(odd, even, i - 1);
+  }
+  if (p.dstate0 != nullptr) store_adjoint(p.dstate0, unit);
+}
+
+// The gradients of a (piece, head) from its start state S0, the adjoint dS at
+// its end, SA and dZ; every piece at once (head size 256), one workgroup each:
+//   dRt = dYs S0^T + dArb Bh + dArk Kh    dAt = dZ S0^T + dLab Bh + dLak Kh
+//   dBh = dLab^T At + dArb^T Rt           dKh = dLak^T At + dArk^T Rt
+//   dBt = SA dS^T    dKt = V dS^T    dg = rowsum(S0 o dS)
+// and the elementwise chain rules of chunk_bwd.hip. Wave w owns keys 32w ..
+// 32w + 31; products come out with lane (g, n) holding token n, keys 4g .. +3
+// of a 16-key block, the layout of the rows. Bound by reading S0 and dS (512
+// KiB per piece and head) once.
+constexpr int kGradThreads = 512;
+constexpr int kGradStride = 260;  // floats per LDS row: 16-byte aligned, rows 4 banks apart
+constexpr int kGradTriStride = 20;
+
+template <typename T, int D>
+__global__ __launch_bounds__(kGradThreads, 2) void piece32_gradient_kernel(Piece32Params p) {
+  using L = Tiles<D>;
+  static_assert(D == 256, "eight waves of 32 keys");
+  using S16 = typename IoTraits<T>::storage;
+  __shared__ float rows[4][kPiece * kGradStride];         // dYs, dZ, SA, V [t][v]
+  __shared__ float tri[4][kPiece * kGradTriStride];       // dArb, dArk, dLab, dLak [t][i]
+  __shared__ float dgs[D];
+  const int heads = p.num_heads;
+  const int head = static_cast<int>(blockIdx.x) % heads;
+  const int slot = static_cast<int>(blockIdx.x) / heads;
+  const int64_t ph = static_cast<int64_t>(slot) * heads + head;
+  constexpr int64_t kState = static_cast<int64_t>(D) * D;
+  int start, ntok;
+  const float* s0;
+  if (p.seg_offsets != nullptr) {
+    const int4 e = p.table[slot];
+    start = uniform(e.x);
+    ntok = uniform(e.y);
+    const int chunk = uniform(e.z), index = uniform(e.w);
+    s0 = index == 0 ? p.boundary + (static_cast<int64_t>(chunk) * heads + head) * kState
+                    : p.interior + (static_cast<int64_t>(start / kPiece) * heads + head) * kState;
+  } else {
+    const int per = p.dense_t / kPiece;
+    const int seq = slot / per, i = slot % per;
+    start = seq * p.dense_t + kPiece * i;
+    ntok = kPiece;
+    s0 = p.boundary + ((static_cast<int64_t>(seq) * heads + head) * per + i) * kState;
+  }
+  if (ntok <= 0) return;
+  const float* const ds = p.adjoints + ph * kState;
+  const int tid = threadIdx.x;
+  const int wave = uniform(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const bool on = n < ntok;
+  const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
+  const int64_t row0 = (static_cast<int64_t>(start) * heads + head) * D;
+  auto row_rs = [&](const void* x) {
+    return buffer_rsrc(x != nullptr ? static_cast<const S16*>(x) + row0 : nullptr,
+                       x != nullptr ? static_cast<uint32_t>(ntok) * row_bytes : 0u);
+  };
+
+  {
+    // Row t = tid / 32, eight columns: dYs, V; dZ and SA as fp32.
+    const int t = tid >> 5, c = 8 * (tid & 31);
+    const uint32_t off = static_cast<uint32_t>(t) * row_bytes + 2 * c;
+    const auto dys = row_rs(p.dy), vs = row_rs(p.v);
+    const auto sas = buffer_rsrc(p.state_dot_a + row0, static_cast<uint32_t>(ntok) * 2 * row_bytes);
+    const float* dz = p.dz + ph * (kPiece * D) + t * D + c;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = t * kGradStride + c + 4 * h;
+      *reinterpret_cast<f32x4*>(&rows[0][at]) = widen4<T>(load4(dys, off + 8 * h)) * p.scale;
+      *reinterpret_cast<f32x4*>(&rows[1][at]) = *reinterpret_cast<const f32x4*>(dz + 4 * h);
+      const u32x4 sa = __builtin_amdgcn_raw_buffer_load_b128(sas, 2 * off + 16 * h, 0, 0);
+      *reinterpret_cast<f32x4*>(&rows[2][at]) = __builtin_bit_cast(f32x4, sa);
+      *reinterpret_cast<f32x4*>(&rows[3][at]) = widen4<T>(load4(vs, off + 8 * h));
+    }
+  }
+  __syncthreads();
+  auto row4 = [&](int m, int c) {
+    return *reinterpret_cast<const f32x4*>(&rows[m][n * kGradStride + c + 4 * g]);
+  };
+
+  // Sums over the value columns, 16 at a time: S0 and dS rows as A operands.
+  f32x4 acc_r[2], acc_a[2], acc_b[2], acc_k[2];
+  float dg[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) acc_r[kt] = acc_a[kt] = acc_b[kt] = acc_k[kt] = zero4();
+  const float* const s_row = s0 + (32 * wave + n) * D + 4 * g;
+  const float* const d_row = ds + (32 * wave + n) * D + 4 * g;
+#pragma unroll 4
+  for (int vb = 0; vb < D / 16; ++vb) {
+    f32x4 s[2], d[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      s[kt] = *reinterpret_cast<const f32x4*>(s_row + 16 * kt * D + 16 * vb);
+      d[kt] = *reinterpret_cast<const f32x4*>(d_row + 16 * kt * D + 16 * vb);
+    }
+    const f32x4 xdy = row4(0, 16 * vb), xdz = row4(1, 16 * vb);
+    const f32x4 xsa = row4(2, 16 * vb), xv = row4(3, 16 * vb);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      acc_r[kt] = mm16(s[kt], xdy, acc_r[kt]);
+      acc_a[kt] = mm16(s[kt], xdz, acc_a[kt]);
+      acc_b[kt] = mm16(d[kt], xsa, acc_b[kt]);
+      acc_k[kt] = mm16(d[kt], xv, acc_k[kt]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dg[kt] += s[kt][j] * d[kt][j];
+    }
+  }
+  // The gradient triangles: waves 0-3, X[t][i] = sum_v A[t][v] B[i][v].
+  if (wave < 4) {
+    f32x4 x = zero4();
+    const int am = wave >> 1, bm = 2 + (wave & 1);
+#pragma unroll 4
+    for (int vb = 0; vb < D / 16; ++vb) x = mm16(row4(am, 16 * vb), row4(bm, 16 * vb), x);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = 4 * g + j;
+      const bool keep = n < t || (n == t && wave < 2);
+      tri[wave][t * kGradTriStride + n] = keep ? x[j] : 0.0f;
+    }
+  }
+  // dg of key 32w + 16kt + n: the lanes of the four column groups.
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    dg[kt] += __shfl_xor(dg[kt], 16);
+    dg[kt] += __shfl_xor(dg[kt], 32);
+    if (g == 0) dgs[32 * wave + 16 * kt + n] = dg[kt];
+  }
+  __syncthreads();
+
+  auto tri_r = [&](int m) {  // [t = n][i = 4g + j]
+    return *reinterpret_cast<const f32x4*>(&tri[m][n * kGradTriStride + 4 * g]);
+  };
+  auto tri_c = [&](int m) {  // [t = 4g + j][i = n]
+    f32x4 x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = tri[m][(4 * g + j) * kGradTriStride + n];
+    return x;
+  };
+  const float* const tiles = p.tiles + ph * L::kBackward;
+  const auto rr = row_rs(p.r), rw = row_rs(p.decay), rk = row_rs(p.k), ra = row_rs(p.a),
+             rb = row_rs(p.b);
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    const int keyt = 32 * wave + 16 * kt;
+    auto col4 = [&](int tile) {  // [key = n][t or i = 4g + j]
+      return *reinterpret_cast<const f32x4*>(tiles + tile + (keyt + n) * kPiece + 4 * g);
+    };
+    const f32x4 atT = col4(L::kAtT), rtT = col4(L::kRtT), bhT = col4(L::kBackBhT),
+                khT = col4(L::kBackKhT);
+    const int key = keyt + 4 * g;
+    const uint32_t off = static_cast<uint32_t>(n) * row_bytes + 2 * key;
+    const u32x2 qw = load4(rw, off), qr = load4(rr, off), qk = load4(rk, off),
+                qa = load4(ra, off), qb = load4(rb, off);
+    acc_r[kt] = mm16(bhT, tri_r(0), acc_r[kt]);
+    acc_r[kt] = mm16(khT, tri_r(1), acc_r[kt]);
+    acc_a[kt] = mm16(bhT, tri_r(2), acc_a[kt]);
+    acc_a[kt] = mm16(khT, tri_r(3), acc_a[kt]);
+    f32x4 db = mm16(atT, tri_c(2), zero4());
+    db = mm16(rtT, tri_c(0), db);
+    f32x4 dk = mm16(atT, tri_c(3), zero4());
+    dk = mm16(rtT, tri_c(1), dk);
+    const f32x4 total = *reinterpret_cast<const f32x4*>(tiles + L::kBackG + key);
+    const f32x4 dgv = *reinterpret_cast<const f32x4*>(&dgs[key]);
+    f32x4 x = widen4<T>(qw);
+    if (p.bias != nullptr) {
+      const S16* bias = static_cast<const S16*>(p.bias) + static_cast<int64_t>(head) * D + key;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] += to_f32<T>(bias[j]);
+    }
+    const f32x4 rv = widen4<T>(qr), kv = widen4<T>(qk), av = widen4<T>(qa), bv = widen4<T>(qb);
+    f32x4 gr, gw, gk, ga, gb;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const Decay dec = piece_decay(x[j], on);
+      const float dbt = total[j] * acc_b[kt][j], dkt = total[j] * acc_k[kt][j];
+      const float dbc = db[j] + dbt, dkc = dk[j] + dkt;
+      gr[j] = acc_r[kt][j] * dec.incl;
+      ga[j] = acc_a[kt][j] * dec.excl;
+      gb[j] = dbc * dec.inv;
+      gk[j] = dkc * dec.inv;
+      // Lanes past the piece hold zero rows (their loads are out of range).
+      const float bh = bv[j] * dec.inv, kh = kv[j] * dec.inv;
+      const float e2 = ga[j] * av[j];
+      const float e1 = gr[j] * rv[j] - dbc * bh - dkc * kh;
+      const float e3 = dbt * bh + dkt * kh;
+      const float later = suffix16(e1 + e2) - e2;
+      // The sum of e3 over the tokens, in every lane of the row.
+      const float all3 = __shfl(suffix16(e3), lane & 48);
+      const float dlg = later + all3 + dgv[j] * total[j];
+      gw[j] = dlg * (-kExpNegHalf) * dec.sig * (1.0f - dec.sig);
+    }
+    auto store = [&](void* dst, f32x4 y) {
+      const auto rs = buffer_rsrc(static_cast<S16*>(dst) + row0,
+                                  static_cast<uint32_t>(ntok) * row_bytes);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])}, rs,
+                                            off, 0, 0);
+    };
+    store(p.dr, gr);
+    store(p.ddecay, gw);
+    store(p.dk, gk);
+    store(p.da, ga);
+    store(p.db, gb);
+  }
+}
+
+constexpr size_t round256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
+
+int64_t lists_of(const Piece32Params& p) {
+  return p.seg_offsets != nullptr ? p.num_segments : p.num_sequences;
+}
+
+size_t tile_bytes(int head_size, int64_t heads, int64_t slots, bool backward) {
+  const int64_t floats = head_size == 64    ? Tiles<64>::kForward
+                         : head_size == 128 ? Tiles<128>::kForward
+                         : backward         ? Tiles<256>::kBackward
+                                            : Tiles<256>::kForward;
+  return round256(static_cast<size_t>(slots) * heads * floats * sizeof(float));
+}
+
+// Scratch: the piece table, the chunks' first pieces, the tiles, then the
+// backward's adjoints and dZ.
+size_t table_bytes(int64_t slots) { return round256(static_cast<size_t>(slots) * sizeof(int4)); }
+size_t base_bytes(int64_t lists) {
+  return round256((static_cast<size_t>(lists) + 1) * sizeof(int32_t));
+}
+
+void lay_out(Piece32Params& p, int head_size, bool backward, void* scratch) {
+  const int64_t slots = piece32_slots(p.total_tokens, lists_of(p));
+  char* at = static_cast<char*>(scratch);
+  p.table = reinterpret_cast<int4*>(at);
+  at += table_bytes(slots);
+  p.base = reinterpret_cast<int32_t*>(at);
+  at += base_bytes(lists_of(p));
+  p.tiles = reinterpret_cast<float*>(at);
+  at += tile_bytes(head_size, p.num_heads, slots, backward);
+  p.adjoints = reinterpret_cast<float*>(at);
+  at += static_cast<size_t>(slots) * p.num_heads * head_size * head_size * sizeof(float);
+  p.dz = reinterpret_cast<float*>(at);
+}
+
+// Pieces the parallel kernels run, after the piece table where one is needed.
+int launch_table(const Piece32Params& p, int& pieces, hipStream_t stream) {
+  const int slots = static_cast<int>(piece32_slots(p.total_tokens, lists_of(p)));
+  pieces = p.dense_t > 0 ? p.num_sequences * (p.dense_t / kPiece) : slots;
+  if (p.seg_offsets == nullptr) return FRWKV_OK;
+  hipLaunchKernelGGL(piece32_table, dim3(1), dim3(kTableThreads), 0, stream, p, slots);
+  return check_launch("piece32_table");
+}
+
+template <typename T, int D>
+int launch_forward(const Piece32Params& p, hipStream_t stream) {
+  int pieces = 0;
+  int rc = launch_table(p, pieces, stream);
+  if (rc != FRWKV_OK) return rc;
+  hipLaunchKernelGGL((piece32_prepare<T, D, false>), dim3(pieces * p.num_heads), dim3(D), 0,
+                     stream, p);
+  rc = check_launch("piece32_prepare");
+  if (rc != FRWKV_OK) return rc;
+  constexpr int kBlocks = D / 16 / (4 / (D / 64));  // workgroups per unit
+  const dim3 grid(p.num_sequences * p.num_heads * kBlocks);
+  if constexpr (D == 256) {
+    if (p.boundary != nullptr) {
+      hipLaunchKernelGGL((piece32_forward_kernel<T, D, true>), grid, dim3(256), 0, stream, p);
+      return check_launch("piece32_forward_kernel");
+    }
+  }
+  hipLaunchKernelGGL((piece32_forward_kernel<T, D, false>), grid, dim3(256), 0, stream, p);
+  return check_launch("piece32_forward_kernel");
+}
+
+template <typename T>
+int dispatch_forward(const Piece32Params& p, int head_size, hipStream_t stream) {
+  switch (head_size) {
+    case 64:
+      return launch_forward<T, 64>(p, stream);
+    case 128:
+      return launch_forward<T, 128>(p, stream);
+    default:
+      return launch_forward<T, 256>(p, stream);
+  }
+}
+
+template <typename T>
+int launch_backward(const Piece32Params& p, hipStream_t stream) {
+  constexpr int D = 256;
+  int pieces = 0;
+  int rc = launch_table(p, pieces, stream);
+  if (rc != FRWKV_OK) return rc;
+  hipLaunchKernelGGL((piece32_prepare<T, D, true>), dim3(pieces * p.num_heads), dim3(D), 0,
+                     stream, p);
+  rc = check_launch("piece32_prepare");
+  if (rc != FRWKV_OK) return rc;
+  hipLaunchKernelGGL((piece32_adjoint_kernel<T, D>), dim3(p.num_sequences * p.num_heads * (D / 16)),
+                     dim3(256), 0, stream, p);
+  rc = check_launch("piece32_adjoint_kernel");
+  if (rc != FRWKV_OK) return rc;
+  hipLaunchKernelGGL((piece32_gradient_kernel<T, D>), dim3(pieces * p.num_heads),
+                     dim3(kGradThreads), 0, stream, p);
+  return check_launch("piece32_gradient_kernel");
+}
+
+}  // namespace
+
+size_t piece32_forward_bytes(int head_size, int64_t heads, int64_t tokens, int64_t lists) {
+  if (heads <= 0 || tokens <= 0 || lists <= 0) return 0;
+  const int64_t slots = piece32_slots(tokens, lists);
+  return table_bytes(slots) + base_bytes(lists) + tile_bytes(head_size, heads, slots, false);
+}
+
+size_t piece32_backward_bytes(int64_t heads, int64_t tokens, int64_t lists) {
+  if (heads <= 0 || tokens <= 0 || lists <= 0) return 0;
+  const int64_t slots = piece32_slots(tokens, lists);
+  return table_bytes(slots) + base_bytes(lists) + tile_bytes(256, heads, slots, true) +
+         static_cast<size_t>(slots) * heads * (256 + kPiece) * 256 * sizeof(float);
+}
+
+int piece32_forward(Piece32Params p, int head_size, int io_dtype, void* scratch,
+                    hipStream_t stream) {
+  lay_out(p, head_size, false, scratch);
+  return io_dtype == FRWKV_DTYPE_BF16 ? dispatch_forward<Bf16>(p, head_size, stream)
+                                      : dispatch_forward<F16>(p, head_size, stream);
+}
+
+int piece32_backward(Piece32Params p, int io_dtype, void* scratch, hipStream_t stream) {
+  lay_out(p, 256, true, scratch);
+  return io_dtype == FRWKV_DTYPE_BF16 ? launch_backward<Bf16>(p, stream)
+                                      : launch_backward<F16>(p, stream);
+}
+
+}  // namespace frwkv

@@ -36,6 +36,7 @@
 // nontemporal and decode launches one wave per workgroup: on MI355X that pair
 // measured fastest (6.07 TB/s at B=256, H=40, above a plain 168 MB copy).
 #include "capi_internal.h"
+#include "piece32.h"
 #include "wkv7_device.h"
 #include "wkv7_mfma.h"
 
@@ -1050,6 +1051,30 @@ extern "C" int frwkv_recurrent_forward_split(
                                            metadata_status, state_pool, r, decay, decay_bias,
                                            k, v, a, b, output, scale, max_seqlen, scratch,
                                            scratch_bytes, stream);
+  }
+  // Other long 16-bit calls take the fp32 matrix form, given its scratch.
+  if (scratch != nullptr && piece32_recurrent(io_dtype, decay_mode, head_size, max_seqlen) &&
+      scratch_bytes >= piece32_forward_bytes(head_size, num_heads, total_tokens, num_sequences)) {
+    Piece32Params q{};
+    q.num_heads = num_heads;
+    q.num_sequences = num_sequences;
+    q.total_tokens = total_tokens;
+    q.cu_seqlens = cu_seqlens;
+    q.state = state_pool;
+    q.slots = state_indices;
+    q.state_slots = state_pool_size;
+    q.status = metadata_status;
+    q.r = r;
+    q.decay = decay;
+    q.bias = decay_bias;
+    q.k = k;
+    q.v = v;
+    q.a = a;
+    q.b = b;
+    q.out = output;
+    q.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
+    q.scale = scale;
+    return piece32_forward(q, head_size, io_dtype, scratch, static_cast<hipStream_t>(stream));
   }
   RecurrentArgs p{num_sequences, num_heads, head_size, total_tokens, max_seqlen,
                   state_pool_size, cu_seqlens, state_indices, metadata_status,

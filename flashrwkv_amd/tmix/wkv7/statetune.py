@@ -121,7 +121,12 @@ class _StateTune(torch.autograd.Function):
         C.native().statetune_forward_internal(offsets, starts, ends, state, r, decay, k, v, a, b,
                                               output, boundary, state_dot_a, interior,
                                               float(scale), int(decay_mode))
-        ctx.save_for_backward(offsets, starts, ends, r, decay, k, v, a, b, boundary, interior)
+        # Head size 256: the backward reads a^T S; a private copy, so that the
+        # caller may write to the output.
+        saved_sda = (state_dot_a.clone() if d == 256 and int(decay_mode) == DECAY_LOGITS
+                     and interior is not None else None)
+        ctx.save_for_backward(offsets, starts, ends, r, decay, k, v, a, b, boundary, interior,
+                              saved_sda)
         ctx.scale, ctx.decay_mode = float(scale), int(decay_mode)
         ctx.mark_non_differentiable(boundary, state_dot_a)
         # Outputs without a gradient reach backward as None instead of zero
@@ -134,7 +139,8 @@ class _StateTune(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, grad_final_state, _grad_boundary, _grad_state_dot_a):
-        offsets, starts, ends, r, decay, k, v, a, b, boundary, interior = ctx.saved_tensors
+        (offsets, starts, ends, r, decay, k, v, a, b, boundary, interior,
+         state_dot_a) = ctx.saved_tensors
         grads = [torch.empty_like(t) for t in (r, decay, k, v, a, b)]
         d = r.shape[2]
         grad_state = torch.empty((offsets.numel() - 1, r.shape[1], d, d), device=r.device,
@@ -143,7 +149,7 @@ class _StateTune(torch.autograd.Function):
         ds = None if grad_final_state is None else grad_final_state.contiguous().float()
         C.native().statetune_backward_internal(offsets, starts, ends, r, decay, k, v, a, b, dy,
                                                ds, boundary, *grads, grad_state, interior,
-                                               ctx.scale, ctx.decay_mode)
+                                               ctx.scale, ctx.decay_mode, state_dot_a)
         return (grad_state, None, None, None, *grads, None, None, None)
 
 

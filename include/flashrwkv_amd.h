@@ -135,10 +135,23 @@ int frwkv_recurrent_forward(int io_dtype, int decay_mode, int32_t num_sequences,
  * FRWKV_SPLIT_CHUNK (frwkv_chunk_forward_split, frwkv_pretrain_forward_split)
  * and FRWKV_SPLIT_RECURRENT (frwkv_recurrent_forward_split); for
  * FRWKV_SPLIT_CALLER_CHUNKS (frwkv_statetune_forward_split) total is
- * num_chunks and longest is not used. No counterpart in the reference.
+ * num_chunks and longest the call's total tokens. The _BACKWARD kinds are the
+ * same for frwkv_pretrain_backward_split and frwkv_statetune_backward_split.
+ * With decay logits, scratch also opens the fp32 matrix form over 16-token
+ * pieces where the unsplit call runs the per-token kernel: the recurrent entry
+ * with fp16 tokens, or at head sizes 128 and 256, on sequences of at least 32
+ * tokens, and training at head size 256. Same fp32 arithmetic, other order of
+ * sums. No counterpart in the reference.
  */
-enum { FRWKV_SPLIT_CHUNK = 0, FRWKV_SPLIT_RECURRENT = 1, FRWKV_SPLIT_CALLER_CHUNKS = 2 };
-size_t frwkv_split_scratch_bytes(int kernel, int32_t num_sequences, int32_t num_heads,
+enum {
+  FRWKV_SPLIT_CHUNK = 0,
+  FRWKV_SPLIT_RECURRENT = 1,
+  FRWKV_SPLIT_CALLER_CHUNKS = 2,
+  FRWKV_SPLIT_PRETRAIN_BACKWARD = 3,
+  FRWKV_SPLIT_CALLER_CHUNKS_BACKWARD = 4
+};
+size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_mode,
+                                 int32_t num_sequences, int32_t num_heads,
                                  int32_t head_size, int32_t total, int32_t longest);
 int frwkv_recurrent_forward_split(int io_dtype, int decay_mode, int32_t num_sequences,
                                   int32_t num_heads, int32_t head_size,
@@ -297,6 +310,21 @@ int frwkv_statetune_forward_split(int io_dtype, int decay_mode, int32_t num_sequ
                                   float scale, void* scratch, size_t scratch_bytes,
                                   void* stream);
 
+/* frwkv_statetune_backward with the forward's state_dot_a (or NULL) and scratch
+ * for a split call (see frwkv_split_scratch_bytes). At head size 256, given
+ * state_dot_a and interior and that scratch, the workspace is not used. */
+int frwkv_statetune_backward_split(
+    int io_dtype, int decay_mode, int32_t num_sequences, int32_t num_heads,
+    int32_t head_size, int32_t total_tokens, int32_t num_chunks,
+    const int32_t* sequence_chunk_offsets, const int32_t* chunk_token_starts,
+    const int32_t* chunk_token_ends, const float* boundary, const float* interior,
+    const void* r, const void* decay, const void* decay_bias, const void* k,
+    const void* v, const void* a, const void* b, const void* grad_output,
+    const float* grad_final_state, void* grad_r, void* grad_decay, void* grad_k,
+    void* grad_v, void* grad_a, void* grad_b, float* grad_initial_state,
+    void* workspace, size_t workspace_bytes, float scale, const float* state_dot_a,
+    void* scratch, size_t scratch_bytes, void* stream);
+
 /* Bytes of the interior-state buffer of frwkv_statetune_forward /
  * frwkv_statetune_backward: ceil(total_tokens / P) x H x D x D elements of
  * 4 bytes (fp32; 2 bytes, bf16, at head size 128). */
@@ -427,6 +455,19 @@ int frwkv_pretrain_forward_split(int io_dtype, int decay_mode, int32_t batch, in
                                  const void* a, const void* b, void* output,
                                  float* boundary, float* state_dot_a, void* scratch,
                                  size_t scratch_bytes, void* stream);
+
+/* frwkv_pretrain_backward with the forward's state_dot_a (or NULL) and scratch
+ * for a split call (see frwkv_split_scratch_bytes). At head size 256, given
+ * both, the workspace is not used. */
+int frwkv_pretrain_backward_split(int io_dtype, int decay_mode, int32_t batch, int32_t tokens,
+                                  int32_t num_heads, int32_t head_size, const void* r,
+                                  const void* decay, const void* k, const void* v,
+                                  const void* a, const void* b, const void* grad_output,
+                                  const float* boundary, void* grad_r, void* grad_decay,
+                                  void* grad_k, void* grad_v, void* grad_a, void* grad_b,
+                                  void* workspace, size_t workspace_bytes,
+                                  const float* state_dot_a, void* scratch,
+                                  size_t scratch_bytes, void* stream);
 
 /*
  * Pretraining backward: recomputes every chunk from the boundary written by

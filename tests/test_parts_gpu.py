@@ -34,8 +34,9 @@ def _require_native():
         pytest.fail("flashrwkv_amd native library is not built (no fallback exists)")
 
 
-def _scratch(kernel, sequences, heads, total, longest):
-    size = capi.library().frwkv_split_scratch_bytes(kernel, sequences, heads, 64, total, longest)
+def _scratch(kernel, io, sequences, heads, total, longest):
+    size = capi.library().frwkv_split_scratch_bytes(kernel, io, 1, sequences, heads, 64, total,
+                                                    longest)
     assert size > 0, "the case is meant to split"
     # Filled with NaN: nothing of it may be read before it is written.
     return torch.full((max(size // 4, 1),), float("nan"), device=DEV), size
@@ -71,7 +72,7 @@ def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
     lib = capi.library()
     status, cu, idx = capi.metadata_validate(d["cu_seqlens"], d["state_indices"], n,
                                              len(lengths) + 1)
-    scratch, size = _scratch(kernel, len(lengths), h, n, max(lengths))
+    scratch, size = _scratch(kernel, capi.DTYPE[dtype], len(lengths), h, n, max(lengths))
     out = []
     for split in (True, False):
         pool = d["state_pool"].to(pool_dtype, copy=True)
@@ -101,3 +102,92 @@ def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
     parity.check("y against unsplit", y, y1.double().cpu(), SAME)
     parity.check("state against unsplit", pool, pool1.double().cpu(), SAME)
     assert torch.equal(pool[-1], d["state_pool"].to(pool_dtype)[-1])  # the slot of no sequence
+
+
+# Head sizes and lengths around the 16-token pieces of the fp32 matrix form,
+# which the public entries take with fp16 tokens or wide heads (decay logits):
+# one piece and a token, ragged, a sequence in the middle shorter than a piece.
+# Expected against the oracle: the fp32 state as the per-token kernels (the
+# sums' order alone differs, about 1e-6 normwise over these lengths), outputs
+# at the io type's rounding (2^-9 bf16, 2^-11 fp16, of the largest entry).
+@pytest.mark.parametrize("dtype,d,lengths", [
+    (torch.float16, 64, (33,)),
+    (torch.float16, 64, (1, 48, 7, 65, 16)),
+    (torch.float16, 128, (40, 3)),
+    (torch.bfloat16, 128, (32, 95)),
+    (torch.float16, 256, (17, 50)),
+    (torch.bfloat16, 256, (64,)),
+])
+def test_fp32_matrix_recurrence(dtype, d, lengths):
+    heads = 2
+    case = workloads.make_case(lengths=lengths, heads=heads, head_size=d, dtype=dtype, seed=5,
+                               state_std=0.1, pool_slots=len(lengths) + 1,
+                               slots=list(range(len(lengths)))[::-1])
+    gen = torch.Generator().manual_seed(6)
+    logits = (torch.randn(case["r"].shape, generator=gen) * 3.0).to(dtype)
+    bias = torch.randn((heads, d), generator=gen).to(dtype)
+    dev = {k: v.to(DEV) if isinstance(v, torch.Tensor) else v for k, v in case.items()}
+    y = flashrwkv_amd.infer_recurrent_fp32io16_forward_varlen(
+        dev["r"], logits.to(DEV), dev["k"], dev["v"], dev["a"], dev["b"],
+        state_pool=dev["state_pool"], cu_seqlens=dev["cu_seqlens"],
+        state_indices=dev["state_indices"], scale=0.5, decay_bias=bias.to(DEV))
+    torch.cuda.synchronize()
+    w = oracle.retention_from_logits(logits.double().numpy(), bias.double().numpy())
+    y_ref, pool_ref = oracle.forward_varlen(
+        case["r"].double().numpy(), w, *(case[x].double().numpy() for x in "kvab"),
+        case["state_pool"].double().numpy(), case["cu_seqlens"].numpy(),
+        case["state_indices"].numpy(), scale=0.5)
+    parity.check("y", y, y_ref, 4e-3 if dtype == torch.bfloat16 else 1e-3)
+    parity.check("state", dev["state_pool"], pool_ref, 1e-5)
+
+
+# Head size 256 training: caller chunks of one piece, of a piece and a token,
+# longer ones and an empty one, and no upstream gradient of y or of the state.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("chunks,with_dy,with_ds", [
+    ([[16, 17, 40], [1]], True, True),
+    ([[33], [0, 64, 15]], True, False),
+    ([[70]], False, True),
+])
+def test_fp32_matrix_training(dtype, chunks, with_dy, with_ds):
+    heads, d = 2, 256
+    ends = np.cumsum([c for seq in chunks for c in seq])
+    starts = np.concatenate([[0], ends[:-1]])
+    offsets = np.concatenate([[0], np.cumsum([len(seq) for seq in chunks])])
+    meta = [np.asarray(x, dtype=np.int32) for x in (offsets, starts, ends)]
+    n = int(ends[-1])
+    case = workloads.make_case(lengths=(n,), heads=heads, head_size=d, dtype=dtype, seed=9,
+                               state_std=0.1)
+    gen = torch.Generator().manual_seed(10)
+    tok = {x: case[x] for x in "rkvab"}
+    tok["w"] = (torch.randn(case["r"].shape, generator=gen) * 3.0).to(dtype)
+    s0 = torch.randn((len(chunks), heads, d, d), generator=gen) * 0.1
+    dy = torch.randn(case["r"].shape, generator=gen).to(dtype)
+    ds = torch.randn(s0.shape, generator=gen) * 0.05
+    leaves = [tok[x].to(DEV).requires_grad_() for x in NAMES]
+    state = s0.to(DEV).requires_grad_()
+    y, final, boundary, sda = flashrwkv_amd.statetune_recurrent_fp32io16(
+        state, *(torch.from_numpy(x).to(DEV) for x in meta), *leaves, scale=0.7)
+    grads = torch.autograd.grad([t for t, on in ((y, with_dy), (final, with_ds)) if on],
+                                [*leaves, state],
+                                [t.to(DEV) for t, on in ((dy, with_dy), (ds, with_ds)) if on])
+    torch.cuda.synchronize()
+    x64 = {x: tok[x].double().numpy() for x in NAMES}
+    logits = x64["w"]
+    x64["w"] = oracle.retention_from_logits(logits)
+    kw = dict(seg_offsets=meta[0], seg_starts=meta[1], seg_ends=meta[2],
+              state_slots=np.arange(len(chunks), dtype=np.int32), scale=0.7)
+    args = [x64[x] for x in NAMES] + [s0.double().numpy()]
+    y_ref, final_ref, boundary_ref, sda_ref = oracle.forward(
+        *args, **kw, want_boundary=True, want_state_dot_a=True)
+    ref = oracle.backward(*args, dy=dy.double().numpy() * with_dy,
+                          dstate_final=ds.double().numpy() * with_ds, **kw)
+    ref["dw"] = ref["dw"] * x64["w"] * oracle.retention_log_derivative(logits)
+    tol = 4e-3 if dtype == torch.bfloat16 else 1e-3
+    parity.check("y", y, y_ref, tol)
+    parity.check("final", final, final_ref, 1e-5)
+    parity.check("boundary", boundary, boundary_ref, 1e-5)
+    parity.check("state_dot_a", sda, sda_ref, 1e-5)
+    for name, got in zip(NAMES, grads):
+        parity.check("d" + name, got, ref["d" + name], tol)
+    parity.check("dS0", grads[-1], ref["dstate0"], 1e-5)
