@@ -53,6 +53,38 @@ __device__ __forceinline__ f32x4 mm16(f32x4 a, f32x4 b, f32x4 c) {
   return c;
 }
 
+// Sum over a wave's 64 keys (A operands x, B operands s): four chains, so that
+// consecutive matrix instructions do not depend on each other.
+__device__ __forceinline__ f32x4 over_keys(const f32x4 (&x)[4], const f32x4 (&s)[4]) {
+  f32x4 c[4] = {zero4(), zero4(), zero4(), zero4()};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) c[kb] = mfma4(x[kb][j], s[kb][j], c[kb]);
+  }
+  return (c[0] + c[1]) + (c[2] + c[3]);
+}
+// s[kb] += x[kb] b: 64 keys (rows of the A operands) by one 16-token block.
+__device__ __forceinline__ void add_columns(const f32x4 (&x)[4], f32x4 b, f32x4 (&s)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) s[kb] = mfma4(x[kb][j], b[j], s[kb]);
+  }
+}
+
+// Schedule of a chain step: one load of the next piece after every two matrix
+// instructions. Issued as one burst at the top of the step, the loads of a
+// CU's waves fill the address unit, and no wave reaches its first product
+// before its last load is accepted.
+__device__ __forceinline__ void spread_loads() {
+#pragma unroll
+  for (int i = 0; i < 28; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // MFMA
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // vector memory read
+  }
+}
+
 // Tiles of one (piece, head), in floats.
 template <int D>
 struct Tiles {
@@ -71,6 +103,28 @@ struct Tiles {
   static constexpr int kBackward = kBackTri + 4 * kTriElems;
 };
 
+// Read-only metadata through scalar loads, which do not wait for the vector
+// memory operations in flight.
+__device__ __forceinline__ int32_t meta_at(const int32_t* a, int64_t i) {
+  return ((const __attribute__((address_space(4))) int32_t*)a)[i];
+}
+
+// A pointer known to be the same in every lane, in scalar registers.
+template <typename P>
+__device__ __forceinline__ P* uniform_pointer(P* x) {
+  const uint64_t bits = reinterpret_cast<uint64_t>(x);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32));
+  return reinterpret_cast<P*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+// x[q] for a wave-uniform q by selects (a branch would end the scheduling
+// region).
+__device__ __forceinline__ float pick4(f32x4 x, int q) {
+  const float a = q & 1 ? x[1] : x[0], b = q & 1 ? x[3] : x[2];
+  return q & 2 ? b : a;
+}
+
 // Pieces of sequence `seq`: slots first .. first + count - 1; with the packed
 // and dense layouts, piece i holds tokens begin + 16 i .. of [begin, end).
 struct Walk {
@@ -79,10 +133,10 @@ struct Walk {
 __device__ __forceinline__ Walk walk_of(const Piece32Params& p, int seq) {
   Walk w{0, 0, 0, 0};
   if (p.seg_offsets != nullptr) {
-    const int lo = min(max(p.seg_offsets[seq], 0), p.num_segments);
-    const int hi = min(max(p.seg_offsets[seq + 1], lo), p.num_segments);
-    w.first = p.base[lo];
-    w.count = p.base[hi] - w.first;
+    const int lo = min(max(meta_at(p.seg_offsets, seq), 0), p.num_segments);
+    const int hi = min(max(meta_at(p.seg_offsets, seq + 1), lo), p.num_segments);
+    w.first = meta_at(p.base, lo);
+    w.count = meta_at(p.base, hi) - w.first;
   } else if (p.dense_t > 0) {
     w.begin = seq * p.dense_t;
     w.end = w.begin + p.dense_t;
@@ -91,8 +145,8 @@ __device__ __forceinline__ Walk walk_of(const Piece32Params& p, int seq) {
   } else {
     // floor(begin / 16) + seq: sequences of ascending, disjoint ranges then
     // have disjoint slots.
-    w.begin = max(p.cu_seqlens[seq], 0);
-    w.end = min(p.cu_seqlens[seq + 1], p.total_tokens);
+    w.begin = max(meta_at(p.cu_seqlens, seq), 0);
+    w.end = min(meta_at(p.cu_seqlens, seq + 1), p.total_tokens);
     w.first = w.begin / kPiece + seq;
     w.count = (max(w.end - w.begin, 0) + kPiece - 1) / kPiece;
   }
@@ -105,8 +159,8 @@ __device__ __forceinline__ Walk walk_of(const Piece32Params& p, int seq) {
 // Piece i of a walk: {first token, tokens, caller chunk, piece of the chunk}.
 __device__ __forceinline__ int4 piece_at(const Piece32Params& p, const Walk& w, int i) {
   if (p.seg_offsets != nullptr) {
-    const int4 e = p.table[w.first + i];
-    return make_int4(uniform(e.x), uniform(e.y), uniform(e.z), uniform(e.w));
+    const int32_t* e = reinterpret_cast<const int32_t*>(p.table + w.first + i);
+    return make_int4(meta_at(e, 0), meta_at(e, 1), meta_at(e, 2), meta_at(e, 3));
   }
   const int start = w.begin + kPiece * i;
   return make_int4(start, min(kPiece, w.end - start), 0, i);
@@ -409,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
     }
   }
   auto store_state = [&](float* dst) {
-    const auto rs = buffer_rsrc(dst, static_cast<uint32_t>(kState) * 4);
+    const auto rs = buffer_rsrc(dst, dst != nullptr ? static_cast<uint32_t>(kState) * 4 : 0u);
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -420,16 +474,20 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
     }
   };
 
-  // A piece's operands: registers in operand layout.
+  // A piece's operands: registers in operand layout. The triangles' products
+  // with V and SA (four steps of four tokens) are shared out over the waves
+  // that add up a sum anyway: wave q takes steps kSteps q .. of each.
+  constexpr int kSteps = 4 / kKeyWaves;
+  const int step0 = kSteps * kq;
+  const int lane_step0 = kSteps * ((static_cast<int>(threadIdx.x) >> 6) % kKeyWaves);
   struct Ops {
-    f32x4 at[4], rt[4], bt[4], kt[4];
-    f32x4 t, lak, arb, ark;
+    f32x4 at[4], rt[4], bt[4], kt[4], t;
+    float lak[kSteps], arb[kSteps], ark[kSteps];
     uint16_t v[4];  // V[4g + j][col]
     int start, ntok, chunk, index;
   };
   const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
-  auto load = [&](Ops& o, int i) {
-    const int4 e = piece_at(p, walk, i);
+  auto load = [&](Ops& o, int i, const int4& e) {
     o.start = e.x;
     o.ntok = e.y;
     o.chunk = e.z;
@@ -451,10 +509,13 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
           vs, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
     }
     const int tri = L::kTri + n * kPiece + 4 * g;
-    o.lak = at4(tri + kTriElems);
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      o.lak[j] = tiles[tri + kTriElems + step0 + j];
+      o.arb[j] = tiles[tri + 2 * kTriElems + step0 + j];
+      o.ark[j] = tiles[tri + 3 * kTriElems + step0 + j];
+    }
     o.t = at4(tri);
-    o.arb = at4(tri + 2 * kTriElems);
-    o.ark = at4(tri + 3 * kTriElems);
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       const int key = 64 * kq + 16 * kb + n;
@@ -463,7 +524,49 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
     }
   };
 
+  // Rows 4g + step0 .. of a token block of the column, from its C layout.
+  auto store_y = [&](int start, int ntok, const float (&y)[kSteps]) {
+    const auto ys = buffer_rsrc(
+        static_cast<S16*>(p.out) + (static_cast<int64_t>(start) * heads + head) * D,
+        static_cast<uint32_t>(ntok) * row_bytes);
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      __builtin_amdgcn_raw_buffer_store_b16(
+          from_f32<T>(p.scale * y[j]), ys,
+          static_cast<uint32_t>(4 * g + step0 + j) * row_bytes + 2 * col, 0, 0);
+    }
+  };
+  // The wave's rows of the output of piece i from the key waves' sums, after
+  // the barrier that follows them.
+  auto finish_y = [&](int i, int start, int ntok) {
+    const int first = wave - kq;
+    float y[kSteps];
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      y[j] = 0.0f;
+#pragma unroll
+      for (int q = 0; q < kKeyWaves; ++q) {
+        y[j] += reinterpret_cast<const float*>(&part[i & 1][first + q][1][lane])[step0 + j];
+      }
+    }
+    store_y(start, ntok, y);
+  };
+  int done_start = 0, done_ntok = 0;  // the piece whose output is still in LDS
   auto step = [&](const Ops& o, Ops& next, int i) {
+    // Everything with a branch first: one scheduling region follows.
+    const int following = min(i + 1, walk.count - 1);
+    const int4 e = piece_at(p, walk, following);
+    float* boundary = nullptr;
+    if constexpr (kTrain) {
+      int64_t at = (static_cast<int64_t>(seq) * heads + head) * (p.dense_t / kPiece) + i;
+      float* base = p.boundary;
+      if (p.dense_t == 0) {
+        const bool first = o.index == 0;
+        at = static_cast<int64_t>(first ? o.chunk : o.start / kPiece) * heads + head;
+        base = first ? p.boundary : p.interior;
+      }
+      boundary = uniform_pointer(base != nullptr ? base + at * kState : nullptr);
+    }
     f32x4 decay[4];  // read at the end of the step
     {
       const float* src = p.tiles +
@@ -472,87 +575,78 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) decay[kb] = *reinterpret_cast<const f32x4*>(src + 16 * kb);
     }
-    if (i + 1 < walk.count) load(next, i + 1);
-    if constexpr (kTrain) {
-      if (p.dense_t > 0) {
-        store_state(p.boundary +
-                    ((static_cast<int64_t>(seq) * heads + head) * (p.dense_t / kPiece) + i) *
-                        kState);
-      } else if (o.index == 0) {
-        store_state(p.boundary + (static_cast<int64_t>(o.chunk) * heads + head) * kState);
-      } else if (p.interior != nullptr) {
-        store_state(p.interior +
-                    (static_cast<int64_t>(o.start / kPiece) * heads + head) * kState);
-      }
-    }
-    // Sums over the keys: two accumulators per product, so that consecutive
-    // matrix instructions do not wait for each other.
-    f32x4 rhs = zero4(), rhs2 = zero4(), y = zero4(), y2 = zero4();
-#pragma unroll
-    for (int kb = 0; kb < 4; kb += 2) {
-      rhs = mm16(o.at[kb], S[kb], rhs);
-      rhs2 = mm16(o.at[kb + 1], S[kb + 1], rhs2);
-      y = mm16(o.rt[kb], S[kb], y);
-      y2 = mm16(o.rt[kb + 1], S[kb + 1], y2);
-    }
-    rhs += rhs2;
-    y += y2;
-    if constexpr (kKeyWaves > 1) {
-      // Double-buffered: the next piece's barrier separates this read from
-      // the write after it.
-      part[i & 1][wave][0][lane] = rhs;
-      part[i & 1][wave][1][lane] = y;
-      __syncthreads();
-      const int first = wave - kq;
-      rhs = part[i & 1][first][0][lane];
-      y = part[i & 1][first][1][lane];
-#pragma unroll
-      for (int q = 1; q < kKeyWaves; ++q) {
-        rhs += part[i & 1][first + q][0][lane];
-        y += part[i & 1][first + q][1][lane];
-      }
-    }
+    // Loads and stores are unconditional (the last piece again at the end; a
+    // null resource drops its stores): past a branch the compiler waits for
+    // everything in flight instead of the loads it needs.
+    load(next, following, e);
+    if constexpr (kTrain) store_state(boundary);
+    spread_loads();
+    // The chain is rhs -> SA -> S; everything else is placed where it fills
+    // the chain's waits (the exchange of the key sums, the triangle products).
     f32x4 v;
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = to_f32<T>(o.v[j]);
-    rhs = mm16(o.lak, v, rhs);
+    auto pick = [&](f32x4 x, int j) {  // x[step0 + j]
+      return kKeyWaves == 1 ? x[j] : pick4(x, lane_step0 + j);
+    };
+    f32x4 rhs = over_keys(o.at, S);
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) rhs = mfma4(o.lak[j], pick(v, j), rhs);
+    if constexpr (kKeyWaves > 1) part[i & 1][wave][0][lane] = rhs;
+    f32x4 y = over_keys(o.rt, S);
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) y = mfma4(o.ark[j], pick(v, j), y);
+    if constexpr (kKeyWaves > 1) {
+      // Double-buffered by piece: the next barrier separates these reads from
+      // the writes after it.
+      __syncthreads();
+      const int first = wave - kq;
+      rhs = part[i & 1][first][0][lane];
+#pragma unroll
+      for (int q = 1; q < kKeyWaves; ++q) rhs += part[i & 1][first + q][0][lane];
+    }
+    add_columns(o.kt, v, S);
     const f32x4 sa = mm16(o.t, rhs, zero4());
+    add_columns(o.bt, sa, S);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) S[kb] = mm16(o.kt[kb], v, S[kb]);
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) S[kb] = mm16(o.bt[kb], sa, S[kb]);
+    for (int j = 0; j < kSteps; ++j) y = mfma4(o.arb[j], pick(sa, j), y);
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) S[kb] *= decay[kb];
-    if (kq == 0) {
-      y = mm16(o.ark, v, y);
-      y = mm16(o.arb, sa, y);
-      const int64_t base = (static_cast<int64_t>(o.start) * heads + head) * D;
-      const auto ys = buffer_rsrc(static_cast<S16*>(p.out) + base,
-                                  static_cast<uint32_t>(o.ntok) * row_bytes);
+    if constexpr (kKeyWaves > 1) {
+      finish_y(i - 1, done_start, done_ntok);
+      done_start = o.start;
+      done_ntok = o.ntok;
+      part[i & 1][wave][1][lane] = y;  // read after the next barrier
+    } else {
+      const float rows[4] = {y[0], y[1], y[2], y[3]};
+      store_y(o.start, o.ntok, rows);
+    }
+    if constexpr (kTrain) {
+      const auto sas = buffer_rsrc(
+          p.state_dot_a + (static_cast<int64_t>(o.start) * heads + head) * D,
+          static_cast<uint32_t>(o.ntok) * 2 * row_bytes);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        __builtin_amdgcn_raw_buffer_store_b16(
-            from_f32<T>(p.scale * y[j]), ys,
-            static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
-      }
-      if constexpr (kTrain) {
-        const auto sas = buffer_rsrc(p.state_dot_a + base,
-                                     static_cast<uint32_t>(o.ntok) * 2 * row_bytes);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          __builtin_amdgcn_raw_buffer_store_b32(
-              __float_as_uint(sa[j]), sas,
-              static_cast<uint32_t>(4 * g + j) * 2 * row_bytes + 4 * col, 0, 0);
-        }
+      for (int j = 0; j < kSteps; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(
+            __float_as_uint(pick(sa, j)), sas,
+            static_cast<uint32_t>(4 * g + step0 + j) * 2 * row_bytes + 4 * col, 0, 0);
       }
     }
   };
 
-  Ops even, odd;
-  if (walk.count > 0) load(even, 0);
-  for (int i = 0; i < walk.count; i += 2) {
-    step(even, odd, i);
-    if (i + 1 < walk.count) step(odd, even, i + 1);
+  if (walk.count > 0) {
+    Ops even, odd;
+    load(even, 0, piece_at(p, walk, 0));
+    for (int i = 0;; i += 2) {
+      step(even, odd, i);
+      if (i + 1 >= walk.count) break;
+      step(odd, even, i + 1);
+      if (i + 2 >= walk.count) break;
+    }
+    if constexpr (kKeyWaves > 1) {
+      __syncthreads();
+      finish_y(walk.count - 1, done_start, done_ntok);
+    }
   }
   if (state != nullptr) store_state(state);
 }
@@ -564,7 +658,7 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
 //   dSA = Bh dU + Arb^T dYs,  dZ = T^T dSA,
 //   dV  = Kh dU + Ark^T dYs + Lak^T dZ,  dS <- dU + Rt^T dYs + At^T dZ.
 template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p) {
+__global__ __launch_bounds__(256, 1) void piece32_adjoint_kernel(Piece32Params p) {
   using L = Tiles<D>;
   constexpr int kKeyWaves = D / 64;
   static_assert(kKeyWaves == 4, "one column slab per workgroup");
@@ -611,14 +705,13 @@ __global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p
   };
 
   struct Ops {
-    f32x4 bh[4], kh[4], at[4], rt[4];
-    f32x4 t, lak, arb, ark;
-    uint16_t dy[4];  // dY[4g + j][col]
+    f32x4 bh[4], kh[4], at[4], rt[4], decay[4], t;
+    float lak, arb, ark;  // the wave's step of the triangles' products
+    uint16_t dy[4];       // dY[4g + j][col]
     int start, ntok;
   };
   const uint32_t row_bytes = static_cast<uint32_t>(heads) * D * 2;
-  auto load = [&](Ops& o, int i) {
-    const int4 e = piece_at(p, walk, i);
+  auto load = [&](Ops& o, int i, const int4& e) {
     o.start = e.x;
     o.ntok = e.y;
     const float* tiles =
@@ -628,6 +721,7 @@ __global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p
     for (int kb = 0; kb < 4; ++kb) {
       o.bh[kb] = at4(L::kBh + n * D + key0 + 16 * kb);
       o.kh[kb] = at4(L::kKh + n * D + key0 + 16 * kb);
+      o.decay[kb] = at4(L::kBackG + key0 + 16 * kb);
     }
     const bool ok = p.dy != nullptr;
     const auto ds = buffer_rsrc(ok ? static_cast<const S16*>(p.dy) +
@@ -640,10 +734,10 @@ __global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p
           ds, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
     }
     const int tri = L::kBackTri + n * kPiece + 4 * g;
+    o.lak = tiles[tri + kTriElems + kq];
+    o.arb = tiles[tri + 2 * kTriElems + kq];
+    o.ark = tiles[tri + 3 * kTriElems + kq];
     o.t = at4(tri);
-    o.lak = at4(tri + kTriElems);
-    o.arb = at4(tri + 2 * kTriElems);
-    o.ark = at4(tri + 3 * kTriElems);
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       const int key = 64 * kq + 16 * kb + n;
@@ -652,68 +746,66 @@ __global__ __launch_bounds__(256, 2) void piece32_adjoint_kernel(Piece32Params p
     }
   };
 
-  auto step = [&](const Ops& o, Ops& next, int i) {
-    const int64_t ph = static_cast<int64_t>(walk.first + i) * heads + head;
-    f32x4 decay[4];
-    {
-      const float* src = p.tiles + ph * L::kBackward + L::kBackG + key0;
+  // The wave's rows (4g + kq) of dV of piece i from the key waves' sums, after
+  // the barrier that follows them.
+  auto finish_dv = [&](int i, int start, int ntok) {
+    float dv = 0.0f;
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) decay[kb] = *reinterpret_cast<const f32x4*>(src + 16 * kb);
+    for (int q = 0; q < kKeyWaves; ++q) {
+      dv += reinterpret_cast<const float*>(&part[i & 1][q][1][lane])[kq];
     }
-    if (i > 0) load(next, i - 1);
+    const auto vs = buffer_rsrc(static_cast<S16*>(p.dv) +
+                                    (static_cast<int64_t>(start) * heads + head) * D,
+                                static_cast<uint32_t>(ntok) * row_bytes);
+    __builtin_amdgcn_raw_buffer_store_b16(
+        from_f32<T>(dv), vs, static_cast<uint32_t>(4 * g + kq) * row_bytes + 2 * col, 0, 0);
+  };
+  int done_start = 0, done_ntok = 0;  // the piece whose dV is still in LDS
+  auto step = [&](const Ops& o, Ops& next, int i) {
+    const int following = max(i - 1, 0);
+    const int4 e = piece_at(p, walk, following);
+    const int64_t ph = static_cast<int64_t>(walk.first + i) * heads + head;
+    load(next, following, e);  // unconditional, as in the forward
     store_adjoint(p.adjoints, ph);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) dS[kb] *= decay[kb];  // dU
-    f32x4 dsa = zero4(), dsa2 = zero4(), dv = zero4(), dv2 = zero4();
-#pragma unroll
-    for (int kb = 0; kb < 4; kb += 2) {
-      dsa = mm16(o.bh[kb], dS[kb], dsa);
-      dsa2 = mm16(o.bh[kb + 1], dS[kb + 1], dsa2);
-      dv = mm16(o.kh[kb], dS[kb], dv);
-      dv2 = mm16(o.kh[kb + 1], dS[kb + 1], dv2);
-    }
-    part[i & 1][kq][0][lane] = dsa + dsa2;
-    part[i & 1][kq][1][lane] = dv + dv2;
-    __syncthreads();
-    dsa = part[i & 1][0][0][lane];
-    dv = part[i & 1][0][1][lane];
-#pragma unroll
-    for (int q = 1; q < kKeyWaves; ++q) {
-      dsa += part[i & 1][q][0][lane];
-      dv += part[i & 1][q][1][lane];
-    }
+    for (int kb = 0; kb < 4; ++kb) dS[kb] *= o.decay[kb];  // dU
+    spread_loads();
+    // The chain is dSA -> dZ -> dS; the rest fills its waits (see the forward).
     f32x4 dy;
 #pragma unroll
     for (int j = 0; j < 4; ++j) dy[j] = p.scale * to_f32<T>(o.dy[j]);
-    dsa = mm16(o.arb, dy, dsa);
+    auto pick = [&](f32x4 x) { return pick4(x, static_cast<int>(threadIdx.x) >> 6); };
+    const float dyq = pick(dy);
+    f32x4 dsa = mfma4(o.arb, dyq, over_keys(o.bh, dS));
+    part[i & 1][kq][0][lane] = dsa;
+    f32x4 dv = mfma4(o.ark, dyq, over_keys(o.kh, dS));
+    __syncthreads();
+    dsa = part[i & 1][0][0][lane];
+#pragma unroll
+    for (int q = 1; q < kKeyWaves; ++q) dsa += part[i & 1][q][0][lane];
+    add_columns(o.rt, dy, dS);
     const f32x4 dz = mm16(o.t, dsa, zero4());
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) dS[kb] = mm16(o.rt[kb], dy, dS[kb]);
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) dS[kb] = mm16(o.at[kb], dz, dS[kb]);
-    if (kq == 0) {
-      dv = mm16(o.ark, dy, dv);
-      dv = mm16(o.lak, dz, dv);
-      const auto vs = buffer_rsrc(static_cast<S16*>(p.dv) +
-                                      (static_cast<int64_t>(o.start) * heads + head) * D,
-                                  static_cast<uint32_t>(o.ntok) * row_bytes);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        __builtin_amdgcn_raw_buffer_store_b16(
-            from_f32<T>(dv[j]), vs, static_cast<uint32_t>(4 * g + j) * row_bytes + 2 * col, 0, 0);
-      }
-    } else if (kq == 1) {
-      float* dst = p.dz + ph * (kPiece * D) + (4 * g) * D + col;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) dst[j * D] = dz[j];
-    }
+    add_columns(o.at, dz, dS);
+    const float dzq = pick(dz);
+    dv = mfma4(o.lak, dzq, dv);
+    finish_dv(i + 1, done_start, done_ntok);
+    done_start = o.start;
+    done_ntok = o.ntok;
+    part[i & 1][kq][1][lane] = dv;  // read after the next barrier
+    p.dz[ph * (kPiece * D) + (4 * g + kq) * D + col] = dzq;
   };
 
-  Ops even, odd;
-  if (walk.count > 0) load(even, walk.count - 1);
-  for (int i = walk.count - 1; i >= 0; i -= 2) {
-    step(even, odd, i);
-    if (i > 0) step(odd, even, i - 1);
+  if (walk.count > 0) {
+    Ops even, odd;
+    load(even, walk.count - 1, piece_at(p, walk, walk.count - 1));
+    for (int i = walk.count - 1;; i -= 2) {
+      step(even, odd, i);
+      if (i < 1) break;
+      step(odd, even, i - 1);
+      if (i < 2) break;
+    }
+    __syncthreads();
+    finish_dv(0, done_start, done_ntok);
   }
   if (p.dstate0 != nullptr) store_adjoint(p.dstate0, unit);
 }
@@ -792,8 +884,10 @@ __global__ __launch_bounds__(kGradThreads, 2) void piece32_gradient_kernel(Piece
     }
   }
   __syncthreads();
+  // Step j of half h of columns c .. c + 31 takes column c + 8g + 4h + j, so
+  // that a lane reads 32 and a group of lanes 128 consecutive bytes of a row.
   auto row4 = [&](int m, int c) {
-    return *reinterpret_cast<const f32x4*>(&rows[m][n * kGradStride + c + 4 * g]);
+    return *reinterpret_cast<const f32x4*>(&rows[m][n * kGradStride + c + 8 * g]);
   };
 
   // Sums over the value columns, 16 at a time: S0 and dS rows as A operands.
@@ -801,26 +895,34 @@ __global__ __launch_bounds__(kGradThreads, 2) void piece32_gradient_kernel(Piece
   float dg[2] = {0.0f, 0.0f};
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt) acc_r[kt] = acc_a[kt] = acc_b[kt] = acc_k[kt] = zero4();
-  const float* const s_row = s0 + (32 * wave + n) * D + 4 * g;
-  const float* const d_row = ds + (32 * wave + n) * D + 4 * g;
-#pragma unroll 4
-  for (int vb = 0; vb < D / 16; ++vb) {
-    f32x4 s[2], d[2];
+  const float* const s_row = s0 + (32 * wave + n) * D + 8 * g;
+  const float* const d_row = ds + (32 * wave + n) * D + 8 * g;
+#pragma unroll 2
+  for (int c = 0; c < D; c += 32) {
+    f32x4 s[2][2], d[2][2];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      s[kt] = *reinterpret_cast<const f32x4*>(s_row + 16 * kt * D + 16 * vb);
-      d[kt] = *reinterpret_cast<const f32x4*>(d_row + 16 * kt * D + 16 * vb);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        s[kt][h] = *reinterpret_cast<const f32x4*>(s_row + 16 * kt * D + c + 4 * h);
+        d[kt][h] = *reinterpret_cast<const f32x4*>(d_row + 16 * kt * D + c + 4 * h);
+      }
     }
-    const f32x4 xdy = row4(0, 16 * vb), xdz = row4(1, 16 * vb);
-    const f32x4 xsa = row4(2, 16 * vb), xv = row4(3, 16 * vb);
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      acc_r[kt] = mm16(s[kt], xdy, acc_r[kt]);
-      acc_a[kt] = mm16(s[kt], xdz, acc_a[kt]);
-      acc_b[kt] = mm16(d[kt], xsa, acc_b[kt]);
-      acc_k[kt] = mm16(d[kt], xv, acc_k[kt]);
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 xdy = row4(0, c + 4 * h), xdz = row4(1, c + 4 * h);
+      const f32x4 xsa = row4(2, c + 4 * h), xv = row4(3, c + 4 * h);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dg[kt] += s[kt][j] * d[kt][j];
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+          acc_r[kt] = mfma4(s[kt][h][j], xdy[j], acc_r[kt]);
+          acc_a[kt] = mfma4(s[kt][h][j], xdz[j], acc_a[kt]);
+          acc_b[kt] = mfma4(d[kt][h][j], xsa[j], acc_b[kt]);
+          acc_k[kt] = mfma4(d[kt][h][j], xv[j], acc_k[kt]);
+          dg[kt] += s[kt][h][j] * d[kt][h][j];
+        }
+      }
     }
   }
   // The gradient triangles: waves 0-3, X[t][i] = sum_v A[t][v] B[i][v].
@@ -828,7 +930,10 @@ __global__ __launch_bounds__(kGradThreads, 2) void piece32_gradient_kernel(Piece
     f32x4 x = zero4();
     const int am = wave >> 1, bm = 2 + (wave & 1);
 #pragma unroll 4
-    for (int vb = 0; vb < D / 16; ++vb) x = mm16(row4(am, 16 * vb), row4(bm, 16 * vb), x);
+    for (int c = 0; c < D; c += 32) {
+      x = mm16(row4(am, c), row4(bm, c), x);
+      x = mm16(row4(am, c + 4), row4(bm, c + 4), x);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int t = 4 * g + j;
