@@ -11,10 +11,14 @@ RuntimeError.
 
 from __future__ import annotations
 
+import sys
+
 import torch
 
 from ... import _contract as C
 from ..._contract import Each, check, is_tensor
+
+_package = sys.modules[__name__.split(".")[0]]
 
 DECAY_LOGITS = 0
 DECAY_RAW_W = 1
@@ -121,6 +125,16 @@ ADD_VEC = (
 
 
 # ------------------------------------------------------------------ entries
+def _whole_call(name: str):
+    """The native whole call of a decode-chain entry (checks, output and launch
+    at once; it declines what its checks do not pass), or None without the
+    native library."""
+    facade = getattr(_package, "_C", None)
+    if facade is None or torch.compiler.is_compiling():
+        return None
+    return getattr(facade.direct, name)
+
+
 def _max_seqlen_arg(max_seqlen: int | None) -> int:
     return -1 if max_seqlen is None else int(max_seqlen)
 
@@ -225,6 +239,11 @@ def infer_recurrent_fp32io16_forward_varlen(
     ``[slots,H,D,D]`` pool ([K,V]) updated at ``state_indices``; returns the
     output shaped like ``v``.
     """
+    if validated_metadata is not None and (call := _whole_call("recurrent_fp32_call")):
+        output = call(r, decay_logits, k, v, a, b, state_pool, cu_seqlens, state_indices, scale,
+                      decay_bias, max_seqlen, validated_metadata)
+        if output is not None:
+            return output
     return _recurrent_fp32(dict(locals()), None)
 
 
@@ -281,6 +300,11 @@ def infer_recurrent_fp16_forward_varlen(
     the fp16 output shaped like ``v``. Without ``max_seqlen`` the ticket
     infers it, so a launch never reads the offsets on the host.
     """
+    if validated_metadata is not None and (call := _whole_call("recurrent_fp16_call")):
+        output = call(r, decay_logits, k, v, a, b, state_pool, elapsed_state_pool, cu_seqlens,
+                      state_indices, scale, decay_bias, max_seqlen, validated_metadata)
+        if output is not None:
+            return output
     ns = dict(locals())
     C.enforce(RECURRENT_FP16, ns)
     ticket = _ticket_for(validated_metadata, cu_seqlens, state_indices, r.shape[0],
@@ -314,6 +338,9 @@ def infer_recurrent_fp16_advance_i32_varlen(
 
     Reference ``__init__.py:83-130``.
     """
+    if validated_metadata is not None and (call := _whole_call("advance_varlen_call")):
+        if call(elapsed_state_pool, cu_seqlens, state_indices, total_tokens, validated_metadata):
+            return
     C.enforce(ADVANCE_VARLEN, dict(locals()))
     ticket = _ticket_for(validated_metadata, cu_seqlens, state_indices, total_tokens,
                          elapsed_state_pool.shape[0], None)

@@ -7,13 +7,14 @@ dense bf16 ``[B,T,C]`` tokens with decay logits ``w`` (retention
 
 Both directions run through ``torch.ops.rwkv7_clampw_v3``: head size 64 on
 the chunked bf16-MFMA kernels, 128 on the bf16-MFMA kernels over 16-token
-pieces, 256 on the per-token fp32 training kernels. The forward saves the state every 16 tokens; the backward recomputes
-from those states and never divides by the decay.
+pieces, 256 on the fp32 matrix kernels over 16-token pieces. The forward saves
+the state every 16 tokens; the backward recomputes from those states and never
+divides by the decay.
 """
 
 from __future__ import annotations
 
-from dataclasses import dataclass
+import sys
 
 import torch
 
@@ -57,76 +58,66 @@ PRETRAIN = (
 )
 
 
-@dataclass(frozen=True)
-class _Layout:
-    """Shapes of one pretraining call: dense [B,T,C] seen as [B,T,H,D]."""
-
-    batch: int
-    tokens: int
-    heads: int
-    head_size: int
-
-    @classmethod
-    def of(cls, tensors: tuple, head_size: int) -> "_Layout":
-        ns = {"tensors": tensors, "head_size": head_size, "r": tensors[0] if tensors else None}
-        ns.update(zip(_DECAY_AND_FRIENDS, tensors[1:]))
-        C.enforce(PRETRAIN, ns)
-        batch, tokens, channels = tensors[0].shape
-        return cls(batch, tokens, channels // head_size, head_size)
-
-    def heads_view(self, x: torch.Tensor) -> torch.Tensor:
-        return x.view(self.batch, self.tokens, self.heads, self.head_size)
-
-    def dense_view(self, x: torch.Tensor) -> torch.Tensor:
-        return x.view(self.batch, self.tokens, self.heads * self.head_size)
-
-    def fp32(self, *shape: int, like: torch.Tensor) -> torch.Tensor:
-        return torch.empty(shape, device=like.device, dtype=torch.float32)
-
-    def checkpoints(self, like: torch.Tensor) -> torch.Tensor:
-        """State before every 16th token: [B, H, T/16, D, D]."""
-        d = self.head_size
-        return self.fp32(self.batch, self.heads, self.tokens // CHUNK_LEN, d, d, like=like)
-
-    def state_dot_a(self, like: torch.Tensor) -> torch.Tensor:
-        return self.fp32(self.batch, self.tokens, self.heads, self.head_size, like=like)
+def _check(tensors: tuple, head_size: int) -> None:
+    ns = {"tensors": tensors, "head_size": head_size, "r": tensors[0] if tensors else None}
+    ns.update(zip(_DECAY_AND_FRIENDS, tensors[1:]))
+    C.enforce(PRETRAIN, ns)
 
 
 class _ClampwV3(torch.autograd.Function):
     """Autograd node over the two ``rwkv7_clampw_v3`` ops (forward saves the
-    16-token checkpoints, backward recomputes from them)."""
+    state before every 16th token, [B,H,T/16,D,D], and a^T S, [B,T,H,D];
+    backward recomputes from them). ``direct``: plain tensors outside of modes,
+    tracing and compiling take the native calls that allocate the buffers too;
+    others go through the registered ops."""
 
     @staticmethod
-    def forward(ctx, layout: _Layout, *tensors):
-        split = tuple(layout.heads_view(t) for t in tensors)
-        y = torch.empty_like(split[3])
-        ckpt = layout.checkpoints(y)
-        sda = layout.state_dot_a(y)
-        torch.ops.rwkv7_clampw_v3.forward(*split, y, ckpt, sda, layout.head_size)
-        ctx.layout = layout
-        ctx.save_for_backward(*split, ckpt, sda)
-        return layout.dense_view(y)
+    def forward(ctx, direct: bool, head_size: int, *tensors):
+        ctx.direct, ctx.head_size = direct, head_size
+        if direct:
+            y, ckpt, sda = C.native().direct.clampw_forward_call(*tensors, head_size)
+        else:
+            batch, tokens, channels = tensors[0].shape
+            heads = channels // head_size
+            split = [t.view(batch, tokens, heads, head_size) for t in tensors]
+            like = {"device": tensors[0].device, "dtype": torch.float32}
+            y = torch.empty_like(split[3])
+            ckpt = torch.empty((batch, heads, tokens // CHUNK_LEN, head_size, head_size), **like)
+            sda = torch.empty((batch, tokens, heads, head_size), **like)
+            torch.ops.rwkv7_clampw_v3.forward(*split, y, ckpt, sda, head_size)
+            y = y.view(batch, tokens, channels)
+        ctx.save_for_backward(*tensors, ckpt, sda)
+        return y
 
     @staticmethod
     def backward(ctx, dy):
-        layout: _Layout = ctx.layout
-        *split, ckpt, sda = ctx.saved_tensors
+        saved, d = ctx.saved_tensors, ctx.head_size
+        if ctx.direct:
+            grads = C.native().direct.clampw_backward_call(dy, saved, d)
+            if grads is not None:
+                return (None, None, *grads)
+        *tensors, ckpt, sda = saved
+        split = [t.view(*t.shape[:2], -1, d) for t in tensors]
         grads = [torch.empty_like(t) for t in split]
-        torch.ops.rwkv7_clampw_v3.backward(*split, layout.heads_view(dy.contiguous()), ckpt,
-                                           sda, *grads, layout.head_size)
-        return (None, *(layout.dense_view(g) for g in grads))
+        torch.ops.rwkv7_clampw_v3.backward(*split, dy.contiguous().view(split[0].shape), ckpt, sda,
+                                           *grads, d)
+        return (None, None, *(g.view(tensors[0].shape) for g in grads))
 
 
 def pretrain_recurrent_bf16(r: torch.Tensor, w: torch.Tensor, k: torch.Tensor,
                             v: torch.Tensor, a: torch.Tensor, b: torch.Tensor, *,
                             head_size: int = 64) -> torch.Tensor:
     """clampw v3 pretraining recurrence with autograd (reference ``pretrain.py:109-126``)."""
-    layout = _Layout.of((r, w, k, v, a, b), head_size)
+    facade = getattr(sys.modules[__name__.split(".")[0]], "_C", None)
+    direct = (facade is not None and not torch.compiler.is_compiling()
+              and facade.direct.clampw_accepts(r, w, k, v, a, b, head_size))
+    if not direct:
+        _check((r, w, k, v, a, b), head_size)
     C.native()
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("pretrain_recurrent_bf16 does not run under HIP graph capture: "
                            "its chunked kernels are not validated inside a captured graph")
-    return _ClampwV3.apply(layout, r, w, k, v, a, b)
+    return _ClampwV3.apply(direct, int(head_size), r, w, k, v, a, b)
 
 
 __all__ = ["pretrain_recurrent_bf16"]

@@ -1,0 +1,150 @@
+"""The native whole calls of the decode chain and of pretraining against the
+contract tables: every form of a call has the same outcome on both, the same
+result or an error of the same type and text."""
+
+import pytest
+import torch
+
+from flashrwkv_amd.tmix import wkv7
+from flashrwkv_amd.tmix.wkv7 import pretrain
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+class Wrapped(torch.Tensor):
+    """A subclass, which the whole calls leave to the tables."""
+
+
+def _tokens(dtype, tokens=5, heads=2, d=64):
+    g = torch.Generator().manual_seed(3)
+    return [(torch.randn(tokens, heads, d, generator=g) * 0.2).to(DEV, dtype) for _ in range(6)]
+
+
+def _metadata():
+    cu = torch.tensor([0, 1, 5], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([2, 0], dtype=torch.int32, device=DEV)
+    return cu, slots, wkv7.prepare_recurrent_metadata(
+        cu, slots, total_tokens=5, state_pool_size=3)
+
+
+def _strided(x):
+    return torch.cat([x, x], -1)[..., :x.shape[-1]]
+
+
+FORMS = {
+    "as given": lambda c: c,
+    "no ticket": lambda c: {**c, "validated_metadata": None},
+    "a ticket of another type": lambda c: {**c, "validated_metadata": object()},
+    "longest 4": lambda c: {**c, "max_seqlen": 4},
+    "longest 0": lambda c: {**c, "max_seqlen": 0},
+    "longest -3": lambda c: {**c, "max_seqlen": -3},
+    "longest 5": lambda c: {**c, "max_seqlen": 5},
+    "longest True": lambda c: {**c, "max_seqlen": True},
+    "longest 4.0": lambda c: {**c, "max_seqlen": 4.0},
+    "longest 2^80": lambda c: {**c, "max_seqlen": 1 << 80},
+    "scale 2": lambda c: {**c, "scale": 2},
+    "scale as text": lambda c: {**c, "scale": "2"},
+    "scale as a tensor": lambda c: {**c, "scale": torch.tensor(0.5)},
+    "bias": lambda c: {**c, "decay_bias": c["r"][0].clone()},
+    "bias of another size": lambda c: {**c, "decay_bias": c["r"][0, :, :7].clone()},
+    "bias no tensor": lambda c: {**c, "decay_bias": 1.0},
+    "r no tensor": lambda c: {**c, "r": [1.0]},
+    "r of two dimensions": lambda c: {**c, "r": c["r"][0]},
+    "k strided": lambda c: {**c, "k": _strided(c["k"])},
+    "v of another size": lambda c: {**c, "v": c["v"][:4]},
+    "v empty": lambda c: {**c, "v": c["v"][:0]},
+    "a double": lambda c: {**c, "a": c["a"].double()},
+    "b on the host": lambda c: {**c, "b": c["b"].cpu()},
+    "b a subclass": lambda c: {**c, "b": c["b"].as_subclass(Wrapped)},
+    "k a parameter": lambda c: {**c, "k": torch.nn.Parameter(c["k"])},
+    "pool strided": lambda c: {**c, "state_pool": _strided(c["state_pool"])},
+    "pool of another type": lambda c: {**c, "state_pool": c["state_pool"].bfloat16()},
+    "pool on the host": lambda c: {**c, "state_pool": c["state_pool"].cpu()},
+    "pool of no dimension": lambda c: {**c, "state_pool": c["state_pool"].sum()},
+    "offsets of 64 bits": lambda c: {**c, "cu_seqlens": c["cu_seqlens"].long()},
+    "offsets of two dimensions": lambda c: {**c, "cu_seqlens": c["cu_seqlens"][None]},
+    "offsets of one sequence": lambda c: {**c, "cu_seqlens": c["cu_seqlens"][:2]},
+    "slots no tensor": lambda c: {**c, "state_indices": [2, 0]},
+    "slots of 64 bits": lambda c: {**c, "state_indices": c["state_indices"].long()},
+    "phases of 64 bits": lambda c: {**c, "elapsed_state_pool": c["elapsed_state_pool"].long()},
+    "phases on the host": lambda c: {**c, "elapsed_state_pool": c["elapsed_state_pool"].cpu()},
+    "phases too few": lambda c: {**c, "elapsed_state_pool": c["elapsed_state_pool"][:2]},
+    "total 4": lambda c: {**c, "total_tokens": 4},
+    "total True": lambda c: {**c, "total_tokens": True},
+    "total 0": lambda c: {**c, "total_tokens": 0},
+    "8 tokens": lambda c: {**{n: c[n][:, :8] for n in "rwkvab"}, "head_size": c["head_size"]},
+    "head size 128": lambda c: {**c, "head_size": 128},
+    "head size 32": lambda c: {**c, "head_size": 32},
+    "head size 64.0": lambda c: {**c, "head_size": 64.0},
+}
+
+
+def _call(which):
+    cu, slots, ticket = _metadata()
+    pool = torch.arange(3 * 2 * 64 * 64, device=DEV).view(3, 2, 64, 64).remainder(13).div(50)
+    if which == "fp32":
+        r, w, k, v, a, b = _tokens(torch.bfloat16)
+        return wkv7.infer_recurrent_fp32io16_forward_varlen, dict(
+            r=r, decay_logits=w, k=k, v=v, a=a, b=b, state_pool=pool, cu_seqlens=cu,
+            state_indices=slots, validated_metadata=ticket)
+    if which == "fp16":
+        r, w, k, v, a, b = _tokens(torch.float16)
+        return wkv7.infer_recurrent_fp16_forward_varlen, dict(
+            r=r, decay_logits=w, k=k, v=v, a=a, b=b, state_pool=pool.half(),
+            elapsed_state_pool=torch.zeros(3, dtype=torch.int32, device=DEV), cu_seqlens=cu,
+            state_indices=slots, validated_metadata=ticket)
+    if which == "advance":
+        return wkv7.infer_recurrent_fp16_advance_i32_varlen, dict(
+            elapsed_state_pool=torch.zeros(3, dtype=torch.int32, device=DEV), cu_seqlens=cu,
+            state_indices=slots, total_tokens=5, validated_metadata=ticket)
+    r, w, k, v, a, b = (x.view(1, 16, 128).requires_grad_()
+                        for x in _tokens(torch.bfloat16, tokens=16))
+    return pretrain.pretrain_recurrent_bf16, dict(r=r, w=w, k=k, v=v, a=a, b=b, head_size=64)
+
+
+def _outcome(entry, call):
+    try:
+        out = entry(**call) if "w" in call else entry(
+            *(call[n] for n in wkv7.C.PACKED_TOKENS if n in call),
+            **{n: x for n, x in call.items() if n not in wkv7.C.PACKED_TOKENS}) \
+            if "r" in call else entry(call["elapsed_state_pool"], call["cu_seqlens"],
+                                      call["state_indices"],
+                                      total_tokens=call["total_tokens"],
+                                      validated_metadata=call["validated_metadata"])
+    except Exception as error:  # noqa: BLE001 - the outcome itself is compared
+        return type(error), str(error)
+    if out is not None and out.requires_grad:
+        return [out.detach(), *torch.autograd.grad((out.float() * 0.25).sum(),
+                                                   [call[n] for n in "rwkvab"])]
+    return [x for x in (out, call.get("state_pool"), call.get("elapsed_state_pool"))
+            if x is not None]
+
+
+@pytest.mark.parametrize("which", ["fp32", "fp16", "advance", "pretrain"])
+def test_whole_call_and_tables_agree(which, monkeypatch):
+    for form, change in FORMS.items():
+        outcomes = []
+        for direct in (True, False):
+            entry, call = _call(which)
+            try:
+                changed = change(call)
+            except KeyError:  # an argument that this entry has not
+                break
+            if set(changed) != set(call):
+                break
+            with monkeypatch.context() as patch:
+                if not direct:
+                    patch.setattr(wkv7, "_whole_call", lambda name: None)
+                    patch.setattr(torch.compiler, "is_compiling", lambda: True)
+                outcomes.append(_outcome(entry, changed))
+            torch.cuda.synchronize()
+        if not outcomes:
+            continue
+        here, tables = outcomes
+        if isinstance(tables, tuple):
+            assert here == tables, form
+            continue
+        assert isinstance(here, list), (form, here)
+        for x, y in zip(here, tables, strict=True):
+            assert x.dtype == y.dtype and torch.equal(x, y), form
