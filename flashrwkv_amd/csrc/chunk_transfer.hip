@@ -119,10 +119,13 @@ __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>
     spans.whole = __builtin_amdgcn_ballot_w64(!(prod >= kSpanFloor)) == 0;
   }
 
-  float fa[8], fd[8];  // 2^Gp and 2^-G, zero outside [lo, hi)
+  // 2^Gp and 2^-G, zero outside [lo, hi). The shift runs in all lanes: the
+  // first token of a sub-range reads the lane before it, which is outside.
+  float fa[8], fd[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    fa[e] = on ? exclusive16(up[e], n) * carry[e] : 0.0f;
+    const float gp = exclusive16(up[e], n) * carry[e];
+    fa[e] = on ? gp : 0.0f;
     fd[e] = on ? __builtin_amdgcn_rcpf(up[e] * carry[e]) : 0.0f;
   }
   const int o = t * kOpStride + f0;

@@ -42,9 +42,21 @@ def _scratch(kernel, io, sequences, heads, total, longest):
     return torch.full((max(size // 4, 1),), float("nan"), device=DEV), size
 
 
+MIXED = 9.0  # in place of u_low: _mixed_decay
+
+
+def _mixed_decay(w):
+    """Retention 1e-3 on 30% of the entries, about 190 log2 units per 64 tokens
+    (such chunks run as sub-chunks) with the others as given, so that states
+    still reach over sub-chunks."""
+    weak = torch.rand(w.shape, generator=torch.Generator().manual_seed(19)) >= 0.3
+    return torch.where(weak, w, torch.full_like(w, 1e-3))
+
+
 def _case(lengths, dtype, u_low=-5.0, heads=3):
     case = workloads.make_case(lengths=lengths, heads=heads, head_size=64, dtype=dtype, seed=31,
-                               state_std=0.1, u_low=u_low, pool_slots=len(lengths) + 1,
+                               state_std=0.1, u_low=-5.0 if u_low == MIXED else u_low,
+                               pool_slots=len(lengths) + 1,
                                slots=list(range(len(lengths)))[::-1])
     return case, {k: v.to(DEV) if isinstance(v, torch.Tensor) else v for k, v in case.items()}
 
@@ -59,6 +71,8 @@ def _case(lengths, dtype, u_low=-5.0, heads=3):
     ((2111, 65), torch.bfloat16, torch.float32, -5.0),
     ((4100,), torch.float16, torch.bfloat16, -5.0),
     ((640, 70), torch.bfloat16, torch.float32, 3.0),
+    ((640, 70), torch.bfloat16, torch.float32, MIXED),
+    ((640, 70), torch.float16, torch.float32, MIXED),
 ])
 @pytest.mark.parametrize("kernel", (CHUNK, RECURRENT))
 def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
@@ -66,7 +80,10 @@ def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
         pytest.skip("the split-precision variant takes bf16 tokens and an fp32 pool")
     case, d = _case(lengths, dtype, u_low)
     n, h, _ = d["r"].shape
-    if u_low > 0:  # strong decay: retentions down to 2^-20
+    if u_low == MIXED:
+        case["w"] = _mixed_decay(case["w"])
+        d["w"] = case["w"].to(DEV)
+    elif u_low > 0:  # strong decay: retentions down to 2^-20
         case["w"] = case["w"].float().clamp_min(2.0 ** -20).to(dtype)
         d["w"] = case["w"].to(DEV)
     lib = capi.library()
