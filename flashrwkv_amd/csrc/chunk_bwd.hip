@@ -66,6 +66,7 @@
 
 #include "capi_internal.h"
 #include "chunk_common.h"
+#include "chunk_parts.h"
 #include "piece32.h"
 
 namespace frwkv {
@@ -108,37 +109,6 @@ static_assert(sizeof(BwdSmem) <= 160 * 1024, "one workgroup per CU");
 
 enum FwdTri { kLab = 0, kLak = 1, kArb = 2, kArk = 3 };
 enum GradTri { kGArb = 0, kGArk = 1, kGLab = 2, kGLak = 3 };
-
-struct ChunkBwdParams {
-  int32_t num_heads;
-  int32_t total_tokens;
-  int32_t num_segments;
-  const int32_t* seg_offsets;
-  const int32_t* seg_starts;
-  const int32_t* seg_ends;
-  const float* checkpoint;      // [num_segments, H, 64, 64]: state at each segment start
-  const float* interior;        // [ceil(N/64), H, 64, 64] piece-start states, or null
-  const void* r;
-  const void* decay;
-  const void* bias;
-  const void* k;
-  const void* v;
-  const void* a;
-  const void* b;
-  const void* dy;               // or null (zero)
-  const float* dstate_final;    // or null (zero)
-  void* dr;
-  void* ddecay;
-  void* dk;
-  void* dv;
-  void* da;
-  void* db;
-  float* dstate0;               // or null (not needed)
-  float scale;
-  // Dense layout: > 0 means every sequence has dense_t tokens (one segment)
-  // and checkpoint is [B, H, dense_t / 16, D, D], the state every 16 tokens.
-  int32_t dense_t;
-};
 
 __device__ __forceinline__ const __attribute__((address_space(4))) ChunkBwdParams& args() {
   return kernel_args<ChunkBwdParams>();
@@ -1091,7 +1061,9 @@ __device__ void run_backward_step(BwdSmem& sm, const ChunkBwdParams& p, const To
 // kDense: the pretraining layout (dense_t > 0), a separate instantiation so
 // that the StateTune path's piece walk carries no dense-layout branches (18
 // fewer SGPRs spilled to VGPR lanes; 2% faster at config 4, same bits).
-template <typename T, DecayMode M, bool kDense>
+// kParts: one workgroup per part of a sequence's segments (dense: chunks),
+// from the end (chunk_parts.h).
+template <typename T, DecayMode M, bool kDense, bool kParts>
 __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParams p) {
   __shared__ BwdSmem sm;
 
@@ -1103,12 +1075,30 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   const int cs = wave & 3;                  // column slab (columns phase)
   const bool adjoint = wave >= 4;
   const int heads = p.num_heads;
-  const int seq = blockIdx.x / heads;
-  const int head = blockIdx.x % heads;
+  const int units = kParts ? static_cast<int>(gridDim.x) / p.parts : 0;
+  const int part = kParts ? static_cast<int>(blockIdx.x) / units : 0;
+  const int unit = kParts ? static_cast<int>(blockIdx.x) % units : static_cast<int>(blockIdx.x);
+  const int seq = unit / heads;
+  const int head = unit % heads;
   const int f0 = 32 * hf + 8 * g;
   constexpr bool dense = kDense;
-  const int seg_lo = dense ? 0 : uniform(max(p.seg_offsets[seq], 0));
-  const int seg_hi = dense ? 1 : uniform(min(p.seg_offsets[seq + 1], p.num_segments));
+  int seg_lo = dense ? 0 : uniform(max(p.seg_offsets[seq], 0));
+  int seg_hi = dense ? 1 : uniform(min(p.seg_offsets[seq + 1], p.num_segments));
+  int dense_lo = 0, dense_hi = p.dense_t;  // dense: the part's tokens of the sequence
+  bool first_part = true;                  // the part with the sequence's start
+  if constexpr (kParts) {
+    const int count = dense ? (p.dense_t + kChunk - 1) / kChunk : max(seg_hi - seg_lo, 0);
+    const PartRange pr = part_range(p, count, part);
+    if (!pr.exists) return;
+    first_part = pr.last;
+    if constexpr (dense) {
+      dense_lo = (count - pr.end) * kChunk;
+      dense_hi = min((count - pr.begin) * kChunk, p.dense_t);
+    } else if (count > 0) {
+      seg_lo = seg_hi - pr.end;
+      seg_hi = seg_hi - pr.begin;
+    }
+  }
 
   // Decay bias of the lane's 8 features, packed (zero: no bias).
   uint4 bias = make_uint4(0u, 0u, 0u, 0u);
@@ -1126,7 +1116,16 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
 
   // dS: dL/dS at the end of the current piece, kept by the adjoint waves in
   // the LDS stash (each lane reads back only what it wrote).
-  if (adjoint) {
+  if constexpr (kParts) {
+    static_assert(sizeof(BwdSmem) - sizeof(sm.dstash) >= kComposeBytes,
+                  "the maps fit the tiles before the stash");
+    f32x4 x[4];
+    compose_start<kBwdThreads>(&sm, p, unit, part, x);
+    if (adjoint) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) sm.dstash[cs][kb][lane] = x[kb];
+    }
+  } else if (adjoint) {
     const auto rs = buffer_rsrc(p.dstate_final != nullptr ? p.dstate_final + unit_state : nullptr,
                                 p.dstate_final != nullptr ? kHead * kHead * 4 : 0);
 #pragma unroll
@@ -1148,8 +1147,8 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   int starts_v = 0, ends_v = 0;
   auto seg_bounds = [&](int seg, int& tb, int& te) {
     if (dense) {
-      tb = seq * p.dense_t;
-      te = tb + p.dense_t;
+      tb = seq * p.dense_t + dense_lo;
+      te = seq * p.dense_t + dense_hi;
       return;
     }
     if (seg < cache_base) {
@@ -1168,8 +1167,8 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
     pc.ntok = uniform(max(min(te - pc.c0, kChunk), 0));
     pc.from_interior = j > 0 && !dense;
     if (dense) {
-      pc.ckpt = ((static_cast<int64_t>(seq) * heads + head) * (p.dense_t / 16) + 4 * j) *
-                kHead * kHead;
+      pc.ckpt = ((static_cast<int64_t>(seq) * heads + head) * (p.dense_t / 16) + dense_lo / 16 +
+                 4 * j) * kHead * kHead;
     } else if (j == 0) {
       pc.ckpt = (static_cast<int64_t>(seg) * heads + head) * kHead * kHead;
     } else {
@@ -1313,7 +1312,7 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   }
 
   // Gradient of the initial state (the adjoint waves' stash).
-  if (p.dstate0 != nullptr && adjoint) {
+  if (p.dstate0 != nullptr && adjoint && first_part) {
     const auto rs0 = buffer_rsrc(p.dstate0 + unit_state, kHead * kHead * 4);
     const float kNaN = __int_as_float(0x7fc00000);
 #pragma unroll
@@ -1333,11 +1332,22 @@ int launch_bwd(const ChunkBwdParams& p, int units, hipStream_t stream) {
     return set_error(FRWKV_ERR_UNSUPPORTED, "chunked kernels take at most %d heads, got %d",
                      kMaxChunkHeads, p.num_heads);
   }
-  if (p.dense_t > 0) {
-    hipLaunchKernelGGL((chunk_bwd_kernel<T, M, true>), dim3(units), dim3(kBwdThreads), 0,
+  if (p.parts > 1) {
+    const int rc = launch_chunk_adjoint<T, M>(p, units, stream);
+    if (rc != FRWKV_OK) return rc;
+    const dim3 grid(units * p.parts);
+    if (p.dense_t > 0) {
+      hipLaunchKernelGGL((chunk_bwd_kernel<T, M, true, true>), grid, dim3(kBwdThreads), 0, stream,
+                         p);
+    } else {
+      hipLaunchKernelGGL((chunk_bwd_kernel<T, M, false, true>), grid, dim3(kBwdThreads), 0,
+                         stream, p);
+    }
+  } else if (p.dense_t > 0) {
+    hipLaunchKernelGGL((chunk_bwd_kernel<T, M, true, false>), dim3(units), dim3(kBwdThreads), 0,
                        stream, p);
   } else {
-    hipLaunchKernelGGL((chunk_bwd_kernel<T, M, false>), dim3(units), dim3(kBwdThreads), 0,
+    hipLaunchKernelGGL((chunk_bwd_kernel<T, M, false, false>), dim3(units), dim3(kBwdThreads), 0,
                        stream, p);
   }
   return check_launch("chunk_bwd_kernel");
@@ -1522,6 +1532,9 @@ extern "C" int frwkv_statetune_backward_split(
   p.db = grad_b;
   p.dstate0 = grad_initial_state;
   p.scale = scale;
+  use_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
+            plan_caller_chunks(num_sequences, num_heads, num_chunks, kBackwardTime, kAdjointTime),
+            scratch, scratch_bytes);
   return dispatch_bwd(p, io_dtype, decay_mode, num_sequences * num_heads,
                       static_cast<hipStream_t>(stream));
 }
@@ -1635,6 +1648,10 @@ extern "C" int frwkv_pretrain_backward_split(int io_dtype, int decay_mode, int32
   p.da = grad_a;
   p.db = grad_b;
   p.scale = 1.0f;
+  use_parts(p, static_cast<int64_t>(batch) * num_heads,
+            plan_parts(batch, num_heads, batch * chunks_of(tokens), chunks_of(tokens),
+                       kBackwardTime, kAdjointTime),
+            scratch, scratch_bytes);
   return dispatch_bwd(p, io_dtype, decay_mode, batch * num_heads,
                       static_cast<hipStream_t>(stream));
 }

@@ -685,100 +685,6 @@ __device__ void state_pass(const ChunkSmem& sm, const ExtraTiles<kPrecise>& ext,
   }
 }
 
-// Start state of part `part`, wave w's columns in C layout (S[kb][j]: row
-// 16kb + 4g + j, column 16w + n): part 0 takes the kept start state, part j the
-// first part's end state through the maps of parts 1 .. j - 1,
-// S <- M_i S + N_i. The four waves need all of each map, so maps go through
-// LDS, four at a time (the chunk tiles' space, not yet in use), split into
-// bf16 hi + lo there: M S is the three products hi hi + hi lo + lo hi, about
-// 2^-16 relative error per step, on an fp32 state. The next four maps are
-// loaded while these are applied. (Every wave reading the maps from memory as
-// fp32 MFMA operands took 3.2 us per step; this takes 0.5.)
-constexpr int kComposeMaps = 4;
-__device__ __forceinline__ void compose_start(ChunkSmem& sm, const ChunkFwdParams& p, int unit,
-                                              int part, f32x4 (&S)[4]) {
-  const int tid = threadIdx.x;
-  const int w = uniform(tid >> 6);
-  const int lane = tid & 63;
-  const int g = lane >> 4, n = lane & 15;
-  uint16_t* const tiles = reinterpret_cast<uint16_t*>(&sm);  // [map][hi, lo][row][col]
-  static_assert(sizeof(ChunkSmem) >= kComposeMaps * 2 * kOpTile * sizeof(uint16_t),
-                "the maps fit the chunk tiles");
-  const int col = (4 * g) * kHead + 16 * w + n;
-  auto load_slab = [&](int i, int which, f32x4 (&x)[4]) {
-    const float* src = part_state(p, unit, i, which) + col;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[kb][j] = src[(16 * kb + j) * kHead];
-    }
-  };
-  load_slab(0, part > 0 ? 1 : 0, S);
-  if (part < 2) return;
-  // The thread's share of a map: row tid / 4, 16 columns.
-  const int share = (tid >> 2) * kHead + 16 * (tid & 3);
-  const int place = (tid >> 2) * kOpStride + 16 * (tid & 3);
-  f32x4 m[kComposeMaps][4], off[kComposeMaps][4];
-  auto load_maps = [&](int first) {
-#pragma unroll
-    for (int u = 0; u < kComposeMaps; ++u) {
-      if (first + u < part) {
-        const float* src = part_state(p, unit, first + u, 0) + share;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) m[u][c] = *reinterpret_cast<const f32x4*>(src + 4 * c);
-      }
-    }
-  };
-  load_maps(1);
-  for (int first = 1; first < part; first += kComposeMaps) {
-#pragma unroll
-    for (int u = 0; u < kComposeMaps; ++u) {
-      if (first + u < part) load_slab(first + u, 1, off[u]);
-    }
-    if (first > 1) __syncthreads();  // the maps before these are applied
-#pragma unroll
-    for (int u = 0; u < kComposeMaps; ++u) {
-      if (first + u < part) {
-        uint16_t* hi = tiles + 2 * u * kOpTile + place;
-#pragma unroll
-        for (int c = 0; c < 4; c += 2) {
-          const float x[8] = {m[u][c][0],     m[u][c][1],     m[u][c][2],     m[u][c][3],
-                              m[u][c + 1][0], m[u][c + 1][1], m[u][c + 1][2], m[u][c + 1][3]};
-          store8_bf16_split(hi + 4 * c, hi + kOpTile + 4 * c, x);
-        }
-      }
-    }
-    __syncthreads();
-    load_maps(first + kComposeMaps);
-#pragma unroll
-    for (int u = 0; u < kComposeMaps; ++u) {
-      if (first + u < part) {
-        const uint16_t* hi = tiles + 2 * u * kOpTile;
-        const uint16_t* lo = hi + kOpTile;
-        i16x4 sh[4], sl[4];
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) to_operand_split(S[kb], sh[kb], sl[kb]);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) S[kb] = off[u][kb];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const i16x8 bh = cat(sh[2 * kk], sh[2 * kk + 1]);
-          const i16x8 bl = cat(sl[2 * kk], sl[2 * kk + 1]);
-#pragma unroll
-          for (int rb = 0; rb < 4; ++rb) {
-            const i16x8 ah = lds_operand32<kOpStride>(hi, 16 * rb + n, 32 * kk, g);
-            const i16x8 al = lds_operand32<kOpStride>(lo, 16 * rb + n, 32 * kk, g);
-            S[rb] = mfma32(al, bh, S[rb]);
-            S[rb] = mfma32(ah, bl, S[rb]);
-            S[rb] = mfma32(ah, bh, S[rb]);
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();  // before the chunk tiles are written
-}
-
 // The sequence of the given rank in order of decreasing length (ties in
 // index order), for batches of at most 64 sequences: lane s holds sequence
 // s's length, counts the sequences ahead of it, and the lane whose count is
@@ -908,7 +814,8 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   // A null state means S0 = 0 and no final state (the pretraining layout).
   f32x4 S[4];
   if constexpr (kParts) {
-    compose_start(sm, p, unit, part, S);
+    static_assert(sizeof(ChunkSmem) >= kComposeBytes, "the maps fit the chunk tiles");
+    compose_start<256>(&sm, p, unit, part, S);
   } else {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
@@ -1277,6 +1184,14 @@ extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_
                                           chunks_of(longest), kPreciseTime, kTransferTime));
     case FRWKV_SPLIT_CALLER_CHUNKS:
       return part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total));
+    case FRWKV_SPLIT_PRETRAIN_BACKWARD:
+      return part_bytes(units, plan_parts(num_sequences, num_heads,
+                                          num_sequences * chunks_of(total / num_sequences),
+                                          chunks_of(total / num_sequences), kBackwardTime,
+                                          kAdjointTime));
+    case FRWKV_SPLIT_CALLER_CHUNKS_BACKWARD:
+      return part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total,
+                                                  kBackwardTime, kAdjointTime));
     default:
       return 0;
   }

@@ -16,6 +16,11 @@
 //      1 .. j - 1 in fp32 (compose_start), then walks its chunks.
 // The work is about twice that of the unsplit kernel, over `parts` times the
 // workgroups.
+//
+// The backward's state adjoint is affine in the adjoint behind it, so it is
+// split the same way from the end: part 0 is a sequence's last run of chunks,
+// chunk_adjoint_kernel gives dS_start = M dS_end + N of each part, and the
+// backward kernel composes the adjoint at its part's end.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -79,6 +84,41 @@ struct ChunkFwdParams {
   float* part_states;
 };
 
+struct ChunkBwdParams {
+  int32_t num_heads;
+  int32_t total_tokens;
+  int32_t num_segments;
+  const int32_t* seg_offsets;
+  const int32_t* seg_starts;
+  const int32_t* seg_ends;
+  const float* checkpoint;      // [num_segments, H, 64, 64]: state at each segment start
+  const float* interior;        // [ceil(N/64), H, 64, 64] piece-start states, or null
+  const void* r;
+  const void* decay;
+  const void* bias;
+  const void* k;
+  const void* v;
+  const void* a;
+  const void* b;
+  const void* dy;               // or null (zero)
+  const float* dstate_final;    // or null (zero)
+  void* dr;
+  void* ddecay;
+  void* dk;
+  void* dv;
+  void* da;
+  void* db;
+  float* dstate0;               // or null (not needed)
+  float scale;
+  // Dense layout: > 0 means every sequence has dense_t tokens (one segment)
+  // and checkpoint is [B, H, dense_t / 16, D, D], the state every 16 tokens.
+  int32_t dense_t;
+  // Sequence parts (see above): part 0 is a sequence's last run of chunks.
+  int32_t parts;
+  int32_t part_len;
+  float* part_states;
+};
+
 constexpr int kMinParts = 3;
 constexpr int kMaxParts = 16;
 
@@ -88,8 +128,8 @@ constexpr int kStateElems = kHead * kHead;
 // each, row-major over keys. Part 0 keeps the sequence's start state in place
 // of M (the pool is overwritten by the last part while the first one still
 // needs it) and its end state in place of N. The last part has none.
-__device__ __forceinline__ float* part_state(const ChunkFwdParams& p, int unit, int part,
-                                             int which) {
+template <typename P>
+__device__ __forceinline__ float* part_state(const P& p, int unit, int part, int which) {
   return p.part_states +
          ((static_cast<int64_t>(unit) * (p.parts - 1) + part) * 2 + which) * kStateElems;
 }
@@ -101,7 +141,8 @@ struct PartRange {
   int begin, end;
   bool exists, last;
 };
-__device__ __forceinline__ PartRange part_range(const ChunkFwdParams& p, int count, int part) {
+template <typename P>
+__device__ __forceinline__ PartRange part_range(const P& p, int count, int part) {
   const int per = max((count + p.parts - 1) / p.parts, p.part_len);
   PartRange r;
   r.begin = min(part * per, count);
@@ -111,12 +152,108 @@ __device__ __forceinline__ PartRange part_range(const ChunkFwdParams& p, int cou
   return r;
 }
 
+// Start state of part `part`, columns 16w .. of the wave (w = wave % 4) in C
+// layout (S[kb][j]: row 16kb + 4g + j, column 16w + n): part 0 takes the kept
+// start state, part j the first part's end state through the maps of parts
+// 1 .. j - 1, S <- M_i S + N_i. All waves need all of each map, so maps go
+// through LDS (tiles: kComposeBytes, not yet in use), four at a time, split
+// into bf16 hi + lo there: M S is the three products hi hi + hi lo + lo hi,
+// about 2^-16 relative error per step, on an fp32 state. The next four maps
+// are loaded while these are applied. (Every wave reading the maps from memory
+// as fp32 MFMA operands took 3.2 us per step; this takes 1.1.)
+constexpr int kComposeMaps = 4;
+constexpr size_t kComposeBytes = kComposeMaps * 2 * kOpTile * sizeof(uint16_t);
+template <int kThreads, typename P>
+__device__ __forceinline__ void compose_start(void* space, const P& p, int unit, int part,
+                                              f32x4 (&S)[4]) {
+  constexpr int kShare = kStateElems / kThreads;  // a thread's elements of a map
+  constexpr int kPerRow = kHead / kShare;
+  const int tid = threadIdx.x;
+  const int w = uniform(tid >> 6) & 3;
+  const int lane = tid & 63;
+  const int g = lane >> 4, n = lane & 15;
+  uint16_t* const tiles = static_cast<uint16_t*>(space);  // [map][hi, lo][row][col]
+  const int col = (4 * g) * kHead + 16 * w + n;
+  auto load_slab = [&](int i, int which, f32x4 (&x)[4]) {
+    const float* src = part_state(p, unit, i, which) + col;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[kb][j] = src[(16 * kb + j) * kHead];
+    }
+  };
+  load_slab(0, part > 0 ? 1 : 0, S);
+  if (part < 2) return;
+  const int share = kShare * tid;
+  const int place = (tid / kPerRow) * kOpStride + kShare * (tid % kPerRow);
+  f32x4 m[kComposeMaps][kShare / 4], off[kComposeMaps][4];
+  auto load_maps = [&](int first) {
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        const float* src = part_state(p, unit, first + u, 0) + share;
+#pragma unroll
+        for (int c = 0; c < kShare / 4; ++c) m[u][c] = *reinterpret_cast<const f32x4*>(src + 4 * c);
+      }
+    }
+  };
+  load_maps(1);
+  for (int first = 1; first < part; first += kComposeMaps) {
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) load_slab(first + u, 1, off[u]);
+    }
+    if (first > 1) __syncthreads();  // the maps before these are applied
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        uint16_t* hi = tiles + 2 * u * kOpTile + place;
+#pragma unroll
+        for (int c = 0; c < kShare / 4; c += 2) {
+          const float x[8] = {m[u][c][0],     m[u][c][1],     m[u][c][2],     m[u][c][3],
+                              m[u][c + 1][0], m[u][c + 1][1], m[u][c + 1][2], m[u][c + 1][3]};
+          store8_bf16_split(hi + 4 * c, hi + kOpTile + 4 * c, x);
+        }
+      }
+    }
+    __syncthreads();
+    load_maps(first + kComposeMaps);
+#pragma unroll
+    for (int u = 0; u < kComposeMaps; ++u) {
+      if (first + u < part) {
+        const uint16_t* hi = tiles + 2 * u * kOpTile;
+        const uint16_t* lo = hi + kOpTile;
+        i16x4 sh[4], sl[4];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) to_operand_split(S[kb], sh[kb], sl[kb]);
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) S[kb] = off[u][kb];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const i16x8 bh = cat(sh[2 * kk], sh[2 * kk + 1]);
+          const i16x8 bl = cat(sl[2 * kk], sl[2 * kk + 1]);
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) {
+            const i16x8 ah = lds_operand32<kOpStride>(hi, 16 * rb + n, 32 * kk, g);
+            const i16x8 al = lds_operand32<kOpStride>(lo, 16 * rb + n, 32 * kk, g);
+            S[rb] = mfma32(al, bh, S[rb]);
+            S[rb] = mfma32(ah, bl, S[rb]);
+            S[rb] = mfma32(ah, bh, S[rb]);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();  // before the chunk tiles are written
+}
+
 // How a call is split: at most `parts` parts of `len` chunks each.
 struct PartPlan {
   int32_t parts, len;
 };
 
-// Measured time of one chunk step of a kernel (us): with at most one workgroup
+// Measured time of one chunk step of a kernel (us; the adjoint transfer kernel
+// takes 5.9 + 4.9 per chunk): with at most one workgroup
 // per CU (256 CUs), and with two on each, in proportion between. Further
 // workgroups wait for a place, and the last round of them fills the GPU only
 // in part (768 workgroups of equal length took 1.8 times as long as 512, 1024
@@ -134,15 +271,20 @@ struct ChunkTime {
 constexpr ChunkTime kForwardTime{5.2, 7.2, false};
 constexpr ChunkTime kPreciseTime{6.4, 12.8, true};
 constexpr ChunkTime kTransferTime{5.2, 8.3, false};
+constexpr ChunkTime kBackwardTime{11.5, 23.0, true};
+constexpr ChunkTime kAdjointTime{5.2, 8.3, false};
 
 // The split of a call of `heads` heads whose sequences have `chunks` chunks in
 // all and at most `longest` each: the part length with the least estimated
 // time of both launches (every chunk is walked by each, and composing a part's
-// start state costs about a fifth of a chunk per part), if that beats the
-// unsplit kernel. Measured, one sequence of 32 heads (unsplit / split): 4
+// start state costs about a fifth of a forward chunk per part), if that beats
+// the unsplit kernel. Measured, one sequence of 32 heads (unsplit / split): 4
 // chunks 29 / 22 us (split-precision), 16 chunks 89 / 39, 64 chunks 331 / 88;
 // two parts never paid (170 / 162), four paid up to 128 units (64 chunks
-// 337 / 237), and at 256 units no split did (32 chunks 177 / 204).
+// 337 / 237), and at 256 units no split did (32 chunks 177 / 204). Backward
+// (unsplit / split): 32 units of 4 chunks 46 / 26, of 16 chunks 170 / 51, of
+// 64 chunks 702 / 160; 96 units of 16 chunks 174 / 120, 128 units 182 / 134;
+// from 192 units on the estimate keeps it whole.
 inline PartPlan plan_parts(int64_t sequences, int64_t heads, int64_t chunks, int64_t longest,
                            const ChunkTime& main, const ChunkTime& transfer) {
   PartPlan best{1, 0};
@@ -156,11 +298,12 @@ inline PartPlan plan_parts(int64_t sequences, int64_t heads, int64_t chunks, int
     const int64_t len = (longest + parts - 1) / parts;
     if ((longest + len - 1) / len != parts) continue;
     // The last part of a sequence of a ragged batch is half full on average.
-    const bool ragged = len > 1 && chunks < longest * sequences;
-    const double groups = heads * (static_cast<double>(chunks) / len +
-                                   (ragged ? 0.5 * (sequences - 1) : 0.0));
-    const double time =
-        5.0 + (len + 0.2 * parts) * main.of(groups) + len * transfer.of(groups - units);
+    const bool ragged = chunks < longest * sequences;
+    const double groups =
+        ragged ? heads * (static_cast<double>(chunks) / len + (len > 1 ? 0.5 * (sequences - 1) : 0))
+               : units * parts;
+    const double time = 5.0 + len * main.of(groups) + 0.2 * parts * kForwardTime.of(groups) +
+                        len * transfer.of(groups - units);
     if (time < least) {
       least = time;
       best = PartPlan{parts, static_cast<int32_t>(len)};
@@ -177,7 +320,8 @@ inline size_t part_bytes(int64_t units, const PartPlan& plan) {
 }
 
 // Splits the call when the caller's scratch holds its part states.
-inline void use_parts(ChunkFwdParams& p, int64_t units, const PartPlan& plan, void* scratch,
+template <typename P>
+inline void use_parts(P& p, int64_t units, const PartPlan& plan, void* scratch,
                       size_t scratch_bytes) {
   const bool split = plan.parts > 1 && scratch != nullptr &&
                      scratch_bytes >= part_bytes(units, plan);
@@ -192,14 +336,19 @@ inline int64_t chunks_of(int64_t tokens) {
 
 // The plan of a call with caller chunks, whose lengths are on the device: by
 // the mean chunk count (a longer sequence gets as many, longer parts).
-inline PartPlan plan_caller_chunks(int64_t sequences, int64_t heads, int64_t chunks) {
+inline PartPlan plan_caller_chunks(int64_t sequences, int64_t heads, int64_t chunks,
+                                   const ChunkTime& main = kForwardTime,
+                                   const ChunkTime& transfer = kTransferTime) {
   if (sequences <= 0) return PartPlan{1, 0};
-  return plan_parts(sequences, heads, chunks, (chunks + sequences - 1) / sequences, kForwardTime,
-                    kTransferTime);
+  return plan_parts(sequences, heads, chunks, (chunks + sequences - 1) / sequences, main,
+                    transfer);
 }
 
 // Launches chunk_transfer_kernel (chunk_transfer.hip) for p.parts > 1.
 template <typename T, DecayMode M, typename PoolT, bool kPrecise>
 int launch_chunk_transfer(const ChunkFwdParams& p, int units, hipStream_t stream);
+// Launches chunk_adjoint_kernel for p.parts > 1.
+template <typename T, DecayMode M>
+int launch_chunk_adjoint(const ChunkBwdParams& p, int units, hipStream_t stream);
 
 }  // namespace frwkv

@@ -30,11 +30,11 @@ template <bool kPrecise>
 struct TransferSmem {
   uint16_t at[kOpTile];  // [t][k]
   uint16_t bh[kOpTile];  // [t][k]
-  uint16_t kh[kOpTile];  // [t][k]
-  uint16_t vt[kOpTile];  // [t][v]
+  uint16_t kh[kOpTile];  // [t][k] (adjoint: Rt)
+  uint16_t vt[kOpTile];  // [t][v] (adjoint: dYs)
   uint16_t kh_lo[kPrecise ? kOpTile : 4];  // low half of Kh (split_bf16x2)
   uint16_t lab[kTriBlocks * kTriBlock];    // [t][i]
-  uint16_t lak[kTriBlocks * kTriBlock];    // [t][i]
+  uint16_t lak[kTriBlocks * kTriBlock];    // [t][i] (adjoint: Arb)
   uint16_t tinv[4][kTriBlock];             // (I - Lab_pp)^{-1}, [t][i]
   float blk[4][kHead];  // decay product of each 16-token block
   float gc[kHead];      // 2^GC
@@ -44,7 +44,7 @@ static_assert(sizeof(TransferSmem<true>) <= 80 * 1024, "two workgroups per CU");
 // A thread's token rows: token 16p + n, features 32h + 8g .. +7 of its wave
 // (p = wave % 4, h = wave / 4, lane (g, n)).
 struct TransferRows {
-  uint4 w, a, b, k, v;
+  uint4 w, a, b, k, v;  // adjoint: r and dy in place of k and v
 };
 
 // Decay-span verdicts of a prepared range (see chunk_fwd.hip), uniform over
@@ -61,11 +61,11 @@ struct TransferSpans {
 // scans the decay and writes the operand tiles. The first barrier frees the
 // tiles (every wave is past its previous state update) and publishes the
 // block products; the second publishes the tiles.
-template <typename T, DecayMode M, bool kPrecise>
+template <typename T, DecayMode M, bool kPrecise, bool kAdjoint = false>
 __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>& sm,
                                                           const TransferRows& rows,
                                                           const float (&bias)[8], int lo,
-                                                          int hi) {
+                                                          int hi, float scale = 1.0f) {
   const int tid = lane_tid();
   const int wave = uniform(tid >> 6);
   const int lane = tid & 63;
@@ -140,7 +140,7 @@ __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>
   store8_bf16(sm.bh + o, x);
   unpack8<T>(rows.k, x);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] *= fd[e];
+  for (int e = 0; e < 8; ++e) x[e] *= kAdjoint ? (on ? up[e] * carry[e] : 0.0f) : fd[e];
   if constexpr (kPrecise) {
     store8_bf16_split(sm.kh + o, sm.kh_lo + o, x);
   } else {
@@ -148,7 +148,7 @@ __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>
   }
   unpack8<T>(rows.v, x);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = on ? x[e] : 0.0f;
+  for (int e = 0; e < 8; ++e) x[e] = on ? (kAdjoint ? scale * x[e] : x[e]) : 0.0f;
   store8_bf16(sm.vt + o, x);
   if (p == 0 && n == 0) {
     *reinterpret_cast<float4*>(&sm.gc[f0]) = make_float4(total[0], total[1], total[2], total[3]);
@@ -162,19 +162,20 @@ __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>
 // Lab, Lak ([t][i] blocks) and the diagonal inverses: waves 0-3 the diagonal
 // block of their index and its inverse, waves 4-7 three of the twelve
 // off-diagonal blocks each. Blocks are computed transposed (A operand = Y
-// rows), as in chunk_fwd.hip. Ends with a barrier.
-template <bool kPrecise>
+// rows), as in chunk_fwd.hip. The adjoint's second matrix is Arb (Rt Bh^T, with
+// its diagonal) in place of Lak. Ends with a barrier.
+template <bool kPrecise, bool kAdjoint = false>
 __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
   const int tid = lane_tid();
   const int wave = uniform(tid >> 6);
   const int lane = tid & 63;
   const int g = lane >> 4, n = lane & 15;
 
-  auto block = [&](const uint16_t* y, const uint16_t* y_lo, int p, int q) {
+  auto block = [&](const uint16_t* x, const uint16_t* y, const uint16_t* y_lo, int p, int q) {
     f32x4 acc = zero4();
 #pragma unroll
     for (int c = 0; c < 64; c += 32) {
-      const i16x8 xa = lds_operand32<kOpStride>(sm.at, 16 * p + n, c, g);
+      const i16x8 xa = lds_operand32<kOpStride>(x, 16 * p + n, c, g);
       acc = mfma32(lds_operand32<kOpStride>(y, 16 * q + n, c, g), xa, acc);
       if constexpr (kPrecise) {
         if (y_lo != nullptr) {
@@ -185,6 +186,8 @@ __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
     return acc;
   };
   const uint16_t* kh_lo = kPrecise ? sm.kh_lo : nullptr;
+  const uint16_t* x2 = kAdjoint ? sm.kh : sm.at;  // factors of the second matrix
+  const uint16_t* y2 = kAdjoint ? sm.bh : sm.kh;
   if (wave < 4) {
     f32x4 l_r = zero4(), l_c = zero4();
 #pragma unroll
@@ -194,12 +197,12 @@ __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
       l_r = mfma32(yb, xa, l_r);  // lane (g, n): L[n][4g + j]
       l_c = mfma32(xa, yb, l_c);  // lane (g, n): L[4g + j][n]
     }
-    f32x4 lak = block(sm.kh, kh_lo, wave, wave);
+    f32x4 lak = block(x2, y2, kh_lo, wave, wave);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       l_r[j] = (4 * g + j < n) ? l_r[j] : 0.0f;
       l_c[j] = (n < 4 * g + j) ? l_c[j] : 0.0f;
-      lak[j] = (4 * g + j < n) ? lak[j] : 0.0f;
+      lak[j] = (4 * g + j < n || (kAdjoint && 4 * g + j == n)) ? lak[j] : 0.0f;
     }
     const int at = tri_index(wave, wave) * kTriBlock;
     lds_store_transposed(sm.lab + at, kTriStride, g, n, l_r);
@@ -227,7 +230,8 @@ __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
       const int p = pair < 1 ? 1 : (pair < 3 ? 2 : 3);
       const int q = pair - (p * (p - 1)) / 2;
       const bool with_k = (item & 1) != 0;
-      const f32x4 acc = with_k ? block(sm.kh, kh_lo, p, q) : block(sm.bh, nullptr, p, q);
+      const f32x4 acc =
+          with_k ? block(x2, y2, kh_lo, p, q) : block(sm.at, sm.bh, nullptr, p, q);
       lds_store_transposed((with_k ? sm.lak : sm.lab) + tri_index(p, q) * kTriBlock, kTriStride,
                            g, n, acc);
     }
@@ -481,6 +485,231 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
   }
 }
 
+// One chunk's adjoint step of a column slab, dS at the chunk's end to dS at its
+// start (C layout): with U = g o dS,
+//   dSA = Bh U + Arb^T dYs,  dZ = T^T dSA,  dS0 = U + Rt^T dYs + At^T dZ
+// (chunk_bwd.hip). kWithDy: the slab belongs to N, else to M (dY = 0).
+template <bool kWithDy>
+__device__ __forceinline__ void adjoint_step(const TransferSmem<false>& sm, f32x4 (&S)[4],
+                                             int cs) {
+  const int lane = lane_tid() & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const i16x4 z4 = {0, 0, 0, 0};
+  auto lo32 = [&](i16x4 x) { return cat(x, z4); };
+  auto lt = [&](const uint16_t* m, int p, int q) {  // block (p, q) transposed
+    return lds_operand_tr<kTriStride>(m + tri_index(p, q) * kTriBlock, 0, 0, g, n);
+  };
+  auto tr32 = [&](const uint16_t* tile, int kb, int t) {
+    return cat(lds_operand_tr<kOpStride>(tile, t, 16 * kb, g, n),
+               lds_operand_tr<kOpStride>(tile, t + 16, 16 * kb, g, n));
+  };
+  auto half = [](const i16x8& x, int h) {
+    return h == 0 ? __builtin_shufflevector(x, x, 0, 1, 2, 3)
+                  : __builtin_shufflevector(x, x, 4, 5, 6, 7);
+  };
+  i16x8 y01, y23;
+  if constexpr (kWithDy) {
+    y01 = tr32(sm.vt, cs, 0);
+    y23 = tr32(sm.vt, cs, 32);
+  }
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    const float4 gc = *reinterpret_cast<const float4*>(&sm.gc[16 * kb + 4 * g]);
+    S[kb] = f32x4{S[kb][0] * gc.x, S[kb][1] * gc.y, S[kb][2] * gc.z, S[kb][3] * gc.w};
+  }
+  f32x4 dsa[4];
+  {
+    const i16x8 u01 = cat(to_operand(S[0]), to_operand(S[1]));
+    const i16x8 u23 = cat(to_operand(S[2]), to_operand(S[3]));
+#pragma unroll
+    for (int pb = 0; pb < 4; ++pb)
+      dsa[pb] = mfma32(lds_operand32<kOpStride>(sm.bh, 16 * pb + n, 0, g), u01, zero4());
+#pragma unroll
+    for (int pb = 0; pb < 4; ++pb)
+      dsa[pb] = mfma32(lds_operand32<kOpStride>(sm.bh, 16 * pb + n, 32, g), u23, dsa[pb]);
+  }
+  if constexpr (kWithDy) {
+    const uint16_t* arb = sm.lak;
+    dsa[3] = mfma32(lo32(lt(arb, 3, 3)), lo32(half(y23, 1)), dsa[3]);
+    dsa[2] = mfma32(cat(lt(arb, 2, 2), lt(arb, 3, 2)), y23, dsa[2]);
+    dsa[1] = mfma32(lo32(lt(arb, 1, 1)), lo32(half(y01, 1)), dsa[1]);
+    dsa[1] = mfma32(cat(lt(arb, 2, 1), lt(arb, 3, 1)), y23, dsa[1]);
+    dsa[0] = mfma32(cat(lt(arb, 0, 0), lt(arb, 1, 0)), y01, dsa[0]);
+    dsa[0] = mfma32(cat(lt(arb, 2, 0), lt(arb, 3, 0)), y23, dsa[0]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] = mfma32(tr32(sm.kh, kb, 0), y01, S[kb]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S[kb] = mfma32(tr32(sm.kh, kb, 32), y23, S[kb]);
+  }
+  // dZ_p = T_pp^T (dSA_p + sum_{q>p} Lab^T(q, p) dZ_q).
+  auto solve = [&](int pb) {
+    return to_operand(mfma32(lo32(lds_operand_tr<kTriStride>(sm.tinv[pb], 0, 0, g, n)),
+                             lo32(to_operand(dsa[pb])), zero4()));
+  };
+  const i16x4 dz3 = solve(3);
+  dsa[2] = mfma32(lo32(lt(sm.lab, 3, 2)), lo32(dz3), dsa[2]);
+  const i16x4 dz2 = solve(2);
+  const i16x8 dz23 = cat(dz2, dz3);
+  dsa[1] = mfma32(cat(lt(sm.lab, 2, 1), lt(sm.lab, 3, 1)), dz23, dsa[1]);
+  dsa[0] = mfma32(cat(lt(sm.lab, 2, 0), lt(sm.lab, 3, 0)), dz23, dsa[0]);
+  const i16x4 dz1 = solve(1);
+  dsa[0] = mfma32(lo32(lt(sm.lab, 1, 0)), lo32(dz1), dsa[0]);
+  const i16x8 dz01 = cat(solve(0), dz1);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) S[kb] = mfma32(tr32(sm.at, kb, 32), dz23, S[kb]);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) S[kb] = mfma32(tr32(sm.at, kb, 0), dz01, S[kb]);
+}
+
+// The adjoint's transfer states: chunks from the last to the first, segments
+// likewise (backward part 0 is a sequence's last run). Same bound, split and
+// tiles as chunk_transfer_kernel. Measured: 1 chunk per part 10.6 us, 3 chunks
+// 20.6, 5 chunks 30.4 (192 workgroups); the backward of 2 x 17 chunks in 32
+// heads takes 95 us with it and 185 without, of 2 x 8 chunks in 12 heads 35
+// and 88.
+template <typename T, DecayMode M>
+__global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(ChunkBwdParams p) {
+  __shared__ TransferSmem<false> sm;
+  const int tid = threadIdx.x;
+  const int wave = uniform(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int cs = wave & 3;
+  const bool map = wave >= 4;
+  const int heads = p.num_heads;
+  const int units = static_cast<int>(gridDim.x) / (p.parts - 1);
+  const int part = static_cast<int>(blockIdx.x) / units;
+  const int unit = static_cast<int>(blockIdx.x) % units;
+  const int seq = unit / heads;
+  const int head = unit % heads;
+
+  // The part's segments, or its run of chunks of the dense sequence; chunks
+  // start at c_begin + 64 j.
+  int seg = 0, seg_lo = 0, c_begin = 0, c_end = 0;
+  bool last;
+  if (p.seg_offsets != nullptr) {
+    const int lo = uniform(max(p.seg_offsets[seq], 0));
+    const int hi = uniform(min(p.seg_offsets[seq + 1], p.num_segments));
+    const PartRange r = part_range(p, max(hi - lo, 0), part);
+    if (!r.exists) return;
+    seg = hi - r.begin;
+    seg_lo = hi - r.end;
+    last = r.last;
+  } else {
+    const int count = (p.dense_t + kChunk - 1) / kChunk;
+    const PartRange r = part_range(p, count, part);
+    if (!r.exists) return;
+    c_begin = seq * p.dense_t + (count - r.end) * kChunk;
+    c_end = seq * p.dense_t + min((count - r.begin) * kChunk, p.dense_t);
+    seg = r.end > r.begin ? 1 : 0;
+    last = r.last;
+  }
+  if (last && part > 0) return;  // no part follows
+
+  f32x4 S[4];
+  const uint32_t s_off = static_cast<uint32_t>((4 * g) * kHead + 16 * cs + n);
+  {
+    const float* src = part == 0 ? p.dstate_final : nullptr;
+    if (src != nullptr) src += (static_cast<int64_t>(seq) * heads + head) * kStateElems + s_off;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        S[kb][j] = src != nullptr ? src[(16 * kb + j) * kHead]
+                   : (part > 0 && map && 16 * kb + 4 * g + j == 16 * cs + n) ? 1.0f
+                                                                             : 0.0f;
+      }
+    }
+  }
+
+  float bias[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) bias[e] = 0.0f;
+  const int f0 = 32 * (wave >> 2) + 8 * g;
+  if constexpr (M == DecayMode::kLogits) {
+    if (p.bias != nullptr) {
+      unpack8<T>(load_row8<T>(p.bias, static_cast<int64_t>(head) * kHead + f0), bias);
+    }
+  }
+
+  using S16 = typename IoTraits<T>::storage;
+  const uint32_t row_bytes = static_cast<uint32_t>(heads) * kHead * 2;
+  const uint32_t row_off = static_cast<uint32_t>(16 * (wave & 3) + n) * row_bytes + 2 * f0;
+  auto load = [&](const void* src, int first, int ntok) {
+    const int64_t base = (static_cast<int64_t>(first) * heads + head) * kHead;
+    const auto rs = buffer_rsrc(static_cast<const S16*>(src) + base,
+                                src != nullptr ? static_cast<uint32_t>(ntok) * row_bytes : 0u);
+    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, row_off, 0, 0);
+    return make_uint4(x.x, x.y, x.z, x.w);
+  };
+  auto load_rows = [&](TransferRows& rows, int first, int ntok) {
+    rows.w = load(p.decay, first, ntok);
+    rows.a = load(p.a, first, ntok);
+    rows.b = load(p.b, first, ntok);
+    rows.k = load(p.r, first, ntok);
+    rows.v = load(p.dy, first, ntok);
+  };
+
+  // The chunk before: [c0, c_end) within the current segment, else the last
+  // one of the nearest earlier segment with tokens.
+  int c0 = c_end;
+  auto previous = [&]() {
+    c_end = c0;
+    while (c0 <= c_begin) {
+      if (--seg < seg_lo) return false;
+      if (p.seg_offsets != nullptr) {
+        c_begin = uniform(max(p.seg_starts[seg], 0));
+        c0 = c_end = uniform(min(p.seg_ends[seg], p.total_tokens));
+      }
+    }
+    c0 = c_begin + (c_end - c_begin - 1) / kChunk * kChunk;
+    return true;
+  };
+  // A part that is its sequence's first and last only keeps the end adjoint.
+  bool more = !(part == 0 && last) && seg > seg_lo && previous();
+  TransferRows rows;
+  if (more) load_rows(rows, c0, c_end - c0);
+  while (more) {
+    const int ntok = c_end - c0;
+    more = previous();
+    // As in the transfer kernel, sub-chunks from the last to the first.
+    TransferSpans spans{};
+    bool whole = true, probe = true;
+    int lo = 0, hi = ntok;
+    for (;;) {
+      const TransferSpans cur =
+          transfer_prepare<T, M, false, true>(sm, rows, bias, lo, hi, p.scale);
+      if (probe) {
+        probe = false;
+        spans = cur;
+        whole = cur.whole;
+        if (!whole) {
+          lo = (hi - 1) & (spans.block_ok((hi - 1) >> 4) ? ~15 : ~3);
+          continue;
+        }
+        if (more) load_rows(rows, c0, c_end - c0);
+      }
+      transfer_intra<false, true>(sm);
+      if (!map) {
+        adjoint_step<true>(sm, S, cs);
+      } else if (part > 0) {
+        adjoint_step<false>(sm, S, cs);
+      }
+      if (whole || lo == 0) break;
+      hi = lo;
+      lo = (hi - 1) & (spans.block_ok((hi - 1) >> 4) ? ~15 : ~3);
+    }
+    if (!whole && more) load_rows(rows, c0, c_end - c0);
+  }
+
+  float* dst = part_state(p, unit, part, map ? 0 : 1) + s_off;
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dst[(16 * kb + j) * kHead] = S[kb][j];
+  }
+}
+
 }  // namespace
 
 template <typename T, DecayMode M, typename PoolT, bool kPrecise>
@@ -489,6 +718,21 @@ int launch_chunk_transfer(const ChunkFwdParams& p, int units, hipStream_t stream
                      dim3(units * (p.parts - 1)), dim3(kTransferThreads), 0, stream, p);
   return check_launch("chunk_transfer_kernel");
 }
+
+template <typename T, DecayMode M>
+int launch_chunk_adjoint(const ChunkBwdParams& p, int units, hipStream_t stream) {
+  hipLaunchKernelGGL((chunk_adjoint_kernel<T, M>), dim3(units * (p.parts - 1)),
+                     dim3(kTransferThreads), 0, stream, p);
+  return check_launch("chunk_adjoint_kernel");
+}
+template int launch_chunk_adjoint<Bf16, DecayMode::kLogits>(const ChunkBwdParams&, int,
+                                                            hipStream_t);
+template int launch_chunk_adjoint<Bf16, DecayMode::kRawW>(const ChunkBwdParams&, int,
+                                                          hipStream_t);
+template int launch_chunk_adjoint<F16, DecayMode::kLogits>(const ChunkBwdParams&, int,
+                                                           hipStream_t);
+template int launch_chunk_adjoint<F16, DecayMode::kRawW>(const ChunkBwdParams&, int,
+                                                         hipStream_t);
 
 #define FRWKV_TRANSFER(T, M, PoolT, P) \
   template int launch_chunk_transfer<T, M, PoolT, P>(const ChunkFwdParams&, int, hipStream_t);
