@@ -35,7 +35,7 @@ HIP_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    # Packed fp32 VALU ops stay disabled for all device code on this pool.
+    # Packed fp32 VALU ops stay disabled for all device code.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", str(REPO / "include"),
 ]

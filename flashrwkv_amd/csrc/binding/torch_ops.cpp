@@ -1645,8 +1645,8 @@ std::optional<TicketPtr> ticket_arg(const pybind11::object& obj) {
 // wrapper runs its tables, which raise the contract's errors in the contract's
 // order. Time of a one-token call, bounded by the host: fp32 state 10.3 us
 // through the tables and 6.1 through this, fp16 state with the advance 17.6
-// and 10.6; forward and backward of a pretraining block of 512 tokens in 8
-// heads 274 and 211 us.
+// and 10.6. The pretraining forward takes 31 us of host time through the
+// registered op and 17 through this.
 struct PlainArgs {
   bool ok = !at::impl::torch_function_mode_enabled() &&
             !c10::impl::TorchDispatchModeTLS::any_modes_set() &&

@@ -1075,9 +1075,9 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   const int cs = wave & 3;                  // column slab (columns phase)
   const bool adjoint = wave >= 4;
   const int heads = p.num_heads;
-  const int units = kParts ? static_cast<int>(gridDim.x) / p.parts : 0;
-  const int part = kParts ? static_cast<int>(blockIdx.x) / units : 0;
-  const int unit = kParts ? static_cast<int>(blockIdx.x) % units : static_cast<int>(blockIdx.x);
+  const uint32_t units = kParts ? gridDim.x / p.parts : 1;
+  const int part = kParts ? blockIdx.x / units : 0;
+  const uint32_t unit = kParts ? blockIdx.x % units : blockIdx.x;
   const int seq = unit / heads;
   const int head = unit % heads;
   const int f0 = 32 * hf + 8 * g;

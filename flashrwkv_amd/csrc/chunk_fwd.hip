@@ -730,9 +730,9 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   const int heads = p.num_heads;
   // Parts: block part * units + unit, so that (for a unit count divisible by
   // the 8 XCDs) a unit's parts share an XCD, and its L2, in both launches.
-  const int units = kParts ? static_cast<int>(gridDim.x) / p.parts : 0;
-  const int part = kParts ? static_cast<int>(blockIdx.x) / units : 0;
-  const int unit = kParts ? static_cast<int>(blockIdx.x) % units : static_cast<int>(blockIdx.x);
+  const uint32_t units = kParts ? gridDim.x / p.parts : 1;
+  const int part = kParts ? blockIdx.x / units : 0;
+  const uint32_t unit = kParts ? blockIdx.x % units : blockIdx.x;
   int seq = unit / heads;
   if (!kParts && p.longest_first_sequences > 0) seq = sequence_by_length_rank(p, seq, lane);
   const int head = unit % heads;

@@ -253,19 +253,20 @@ struct PartPlan {
 };
 
 // Measured time of one chunk step of a kernel (us; the adjoint transfer kernel
-// takes 5.9 + 4.9 per chunk): with at most one workgroup
-// per CU (256 CUs), and with two on each, in proportion between. Further
-// workgroups wait for a place, and the last round of them fills the GPU only
-// in part (768 workgroups of equal length took 1.8 times as long as 512, 1024
-// 2.6 times). A kernel whose LDS admits one per CU starts a second round
-// beyond 256 (`rounds`).
+// takes 5.9 + 4.9 per chunk): with at most one workgroup per CU (256 CUs), and
+// with two on each, in proportion between. Further workgroups wait for a place,
+// and the last round of them fills the GPU only in part (768 workgroups of
+// equal length took 1.8 times as long as 512, 1024 2.6 times). A kernel whose
+// LDS admits one per CU runs in rounds of 256 (`rounds`; 576 workgroups of the
+// backward, 2 chunks each, took 82 us, 256 of 5 chunks 64).
 struct ChunkTime {
   double alone, shared;
   bool rounds;
   double of(double workgroups) const {
     if (workgroups <= 256) return alone;
+    if (rounds) return alone * __builtin_ceil(workgroups / 256);
     if (workgroups > 512) return shared * (1.0 + 1.6 * (workgroups / 512 - 1.0));
-    return rounds ? shared : alone + (shared - alone) * (workgroups - 256) / 256;
+    return alone + (shared - alone) * (workgroups - 256) / 256;
   }
 };
 constexpr ChunkTime kForwardTime{5.2, 7.2, false};

@@ -15,7 +15,9 @@
 // the forward's) are spread over all eight, so a chunk of two states takes
 // less time than the forward's chunk of one. 52 KB of LDS (60 KB in the
 // split-precision variant) and at most 128 registers per lane leave two
-// workgroups per CU.
+// workgroups per CU. Measured: 5.2 us per chunk alone on a CU, 8.3 with two
+// (the forward kernel 5.2 and 7.2); with up to 256 registers, one workgroup
+// per CU, 128 units of 4 chunks took 42.4 us instead of 33.2.
 #include "capi_internal.h"
 #include "chunk_parts.h"
 #include "wkv7_device.h"

@@ -72,7 +72,14 @@ inline int64_t piece32_slots(int64_t tokens, int64_t lists) { return tokens / 16
 
 // The recurrent operator's calls on this route: decay logits, 16-bit tokens
 // that the chunk kernel of bf16 tokens at head size 64 does not take, and at
-// least 32 tokens in the longest sequence.
+// least 32 tokens in the longest sequence. Measured (us per token / pieces):
+//                            16 tokens    24 tokens    32 tokens    64 tokens
+//   D = 64,  1 x 32 heads    10.0 / 12.2  12.7 / 14.4  15.4 / 14.1  26.1 / 17.8
+//   D = 64,  9 x 32 heads    18.6 / 18.5  24.7 / 22.9  30.5 / 23.5  54.3 / 35.9
+//   D = 64,  64 x 32 heads   58.2 / 59.9  79.3 / 74.2  99.0 / 76.9   184 / 151
+//   D = 128, 64 x 16 heads   94.5 / 94.1   130 / 122    165 / 125    312 / 218
+//   D = 256, 64 x 8 heads     218 / 179    298 / 279    377 / 286    697 / 458
+// Calls whose tiles would take more than 2 GiB stay on the per-token kernel.
 constexpr int32_t kPiece32MinSeqlen = 32;
 constexpr size_t kPiece32RecurrentBytes = size_t{2} << 30;
 inline bool piece32_recurrent(int io_dtype, int decay_mode, int head_size, int32_t max_seqlen) {

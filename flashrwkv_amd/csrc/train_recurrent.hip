@@ -1,4 +1,6 @@
-// Per-token WKV7 training kernels for head size 256.
+// Per-token WKV7 training kernels for head size 256: raw retentions, callers
+// without scratch or without the forward's a^T S and interior states. Other
+// calls run the fp32 matrix form (piece32.hip).
 //
 // The chunked MFMA kernels (chunk_fwd.hip, chunk_bwd.hip) are built around
 // D = 64 tiles and the piece kernels (piece_train.hip) around D = 128. These

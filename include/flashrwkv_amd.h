@@ -281,7 +281,8 @@ int frwkv_chunk_forward_split(int io_dtype, int decay_mode, int pool_dtype,
  * (csrc/sm90/tmix/wkv7/statetune_recurrent_fp32io16_forward.cu:32-224;
  * binding statetune_recurrent_fp32io16_forward.cpp:26-56). head_size 64
  * runs the chunked MFMA kernel, 128 the MFMA kernel over 16-token pieces,
- * 256 the per-token fp32 kernel.
+ * 256 the per-token fp32 kernel (the _split entry: see
+ * frwkv_split_scratch_bytes).
  */
 int frwkv_statetune_forward(int io_dtype, int decay_mode, int32_t num_sequences,
                             int32_t num_heads, int32_t head_size,
