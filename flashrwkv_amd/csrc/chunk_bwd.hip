@@ -367,15 +367,8 @@ __device__ __forceinline__ void intra_piece(BwdSmem& sm, Issue&& issue) {
       store(kArk, p, q, ark, false);
     }
     if (lab_c != nullptr) {
-      // lab: lane (g, n) holds L[n][4g + j]; labc: L[4g + j][n] (strict lower).
-      f32x4 lr = lab, lc = labc;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        lr[j] = (4 * g + j < n) ? lr[j] : 0.0f;
-        lc[j] = (n < 4 * g + j) ? lc[j] : 0.0f;
-      }
-      lab_c[0] = lr;
-      lab_c[1] = lc;
+      lab_c[0] = lab;   // lane (g, n) holds L[n][4g + j]
+      lab_c[1] = labc;  // L[4g + j][n]
     }
   };
 
@@ -385,22 +378,8 @@ __device__ __forceinline__ void intra_piece(BwdSmem& sm, Issue&& issue) {
     issue(0);
     group(wave, wave, true, true, l);
     issue(1);
-    // (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8) for strictly lower
-    // 16 x 16 L. With X_R "lane (g, n) holds X[n][4g + j]" and X_C the C
-    // layout, Z = X Y is Z_C = mfma(X_R, Y_C) and Z_R = mfma(Y_C, X_R).
-    const i16x4 lr = to_operand(l[0]), lc = to_operand(l[1]);
-    const i16x4 p2c = to_operand(mfma16(lr, lc, zero4()));
-    const i16x4 p2r = to_operand(mfma16(lc, lr, zero4()));
-    const i16x4 p4c = to_operand(mfma16(p2r, p2c, zero4()));
-    const i16x4 p4r = to_operand(mfma16(p2c, p2r, zero4()));
-    const i16x4 p8c = to_operand(mfma16(p4r, p4c, zero4()));
-    f32x4 tt = l[0];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) tt[j] += (4 * g + j == n) ? 1.0f : 0.0f;
-    tt = mfma16(p2c, to_operand(tt), tt);
-    tt = mfma16(p4c, to_operand(tt), tt);
-    tt = mfma16(p8c, to_operand(tt), tt);
-    lds_store_transposed(sm.u.f.tinv[wave], kTriStride, g, n, tt);  // T [t][i]
+    lds_store_transposed(sm.u.f.tinv[wave], kTriStride, g, n,  // T [t][i]
+                         invert_unit_lower(l[0], l[1]));
     issue(2);
   } else {
     // Off-diagonal half-pairs: pair index item / 2 over (1,0) (2,0) (2,1)

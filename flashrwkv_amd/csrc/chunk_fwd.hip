@@ -405,12 +405,8 @@ __device__ __forceinline__ void intra_chunk(ChunkSmem& sm, ExtraTiles<kPrecise>&
   issue(0);
   group(wave, wave, true, true, true);
   issue(1);
-  // T_pp = (I - L)^{-1} for the strictly lower 16 x 16 block L = Lab_pp:
-  // L^16 = 0, so (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8). All
-  // factors are polynomials in L and commute. With X_R the register layout
-  // "lane (g, n) holds X[n][4g + j]" (A operand of X, C layout of X^T) and
-  // X_C the C layout of X (B operand of X), a product Z = X Y is
-  // Z_C = mfma(X_R, Y_C) and Z_R = mfma(Y_C, X_R).
+  // T_pp = (I - L)^{-1} for the strictly lower 16 x 16 block L = Lab_pp, from
+  // its rows and its columns (invert_unit_lower).
   {
     f32x4 l_r = zero4(), l_c = zero4();
 #pragma unroll
@@ -420,24 +416,7 @@ __device__ __forceinline__ void intra_chunk(ChunkSmem& sm, ExtraTiles<kPrecise>&
       l_r = mfma32(yb, xa, l_r);  // lane (g, n): L[n][4g + j]
       l_c = mfma32(xa, yb, l_c);  // lane (g, n): L[4g + j][n]
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      l_r[j] = (4 * g + j < n) ? l_r[j] : 0.0f;
-      l_c[j] = (n < 4 * g + j) ? l_c[j] : 0.0f;
-    }
-    const i16x4 lr = to_operand(l_r), lc = to_operand(l_c);
-    const i16x4 p2c = to_operand(mfma16(lr, lc, zero4()));
-    const i16x4 p2r = to_operand(mfma16(lc, lr, zero4()));
-    const i16x4 p4c = to_operand(mfma16(p2r, p2c, zero4()));
-    const i16x4 p4r = to_operand(mfma16(p2c, p2r, zero4()));
-    const i16x4 p8c = to_operand(mfma16(p4r, p4c, zero4()));
-    f32x4 t = l_r;  // T1 = I + L
-#pragma unroll
-    for (int j = 0; j < 4; ++j) t[j] += (4 * g + j == n) ? 1.0f : 0.0f;
-    t = mfma16(p2c, to_operand(t), t);  // T2 = T1 + P2 T1
-    t = mfma16(p4c, to_operand(t), t);  // T3 = T2 + P4 T2
-    t = mfma16(p8c, to_operand(t), t);  // T  = T3 + P8 T3
-    lds_store_transposed(sm.tinv[wave], kTriStride, g, n, t);
+    lds_store_transposed(sm.tinv[wave], kTriStride, g, n, invert_unit_lower(l_r, l_c));
   }
   issue(2);
 

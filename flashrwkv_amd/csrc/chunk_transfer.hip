@@ -203,26 +203,12 @@ __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       l_r[j] = (4 * g + j < n) ? l_r[j] : 0.0f;
-      l_c[j] = (n < 4 * g + j) ? l_c[j] : 0.0f;
       lak[j] = (4 * g + j < n || (kAdjoint && 4 * g + j == n)) ? lak[j] : 0.0f;
     }
     const int at = tri_index(wave, wave) * kTriBlock;
     lds_store_transposed(sm.lab + at, kTriStride, g, n, l_r);
     lds_store_transposed(sm.lak + at, kTriStride, g, n, lak);
-    // (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8) (see chunk_fwd.hip).
-    const i16x4 lr = to_operand(l_r), lc = to_operand(l_c);
-    const i16x4 p2c = to_operand(mfma16(lr, lc, zero4()));
-    const i16x4 p2r = to_operand(mfma16(lc, lr, zero4()));
-    const i16x4 p4c = to_operand(mfma16(p2r, p2c, zero4()));
-    const i16x4 p4r = to_operand(mfma16(p2c, p2r, zero4()));
-    const i16x4 p8c = to_operand(mfma16(p4r, p4c, zero4()));
-    f32x4 tt = l_r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) tt[j] += (4 * g + j == n) ? 1.0f : 0.0f;
-    tt = mfma16(p2c, to_operand(tt), tt);
-    tt = mfma16(p4c, to_operand(tt), tt);
-    tt = mfma16(p8c, to_operand(tt), tt);
-    lds_store_transposed(sm.tinv[wave], kTriStride, g, n, tt);
+    lds_store_transposed(sm.tinv[wave], kTriStride, g, n, invert_unit_lower(l_r, l_c));
   } else {
     // Block pairs (1,0) (2,0) (2,1) (3,0) (3,1) (3,2), each for Lab and Lak.
 #pragma unroll

@@ -378,25 +378,13 @@ __device__ __forceinline__ void piece_intra(PieceSmem& sm) {
     }
     lds_store_transposed(sm.tri[w], kTriStride, g, n, acc);
     if (w == 0) {
-      // The Neumann product of chunk_fwd.hip's diagonal blocks:
-      // (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8). l_r: lane (g, n)
-      // holds L[n][4g + j]; lc, the B operand of L, is a transpose read of
-      // the block just stored (same wave, in order).
-      const f32x4 l_r = acc;
-      const i16x4 lr = to_operand(l_r);
+      // The columns of L are a transpose read of the block just stored (same
+      // wave, in order).
       const i16x4 lc = lds_operand_tr<kTriStride>(sm.tri[kTLab], 0, 0, g, n);
-      const i16x4 p2c = to_operand(mfma16(lr, lc, zero4()));
-      const i16x4 p2r = to_operand(mfma16(lc, lr, zero4()));
-      const i16x4 p4c = to_operand(mfma16(p2r, p2c, zero4()));
-      const i16x4 p4r = to_operand(mfma16(p2c, p2r, zero4()));
-      const i16x4 p8c = to_operand(mfma16(p4r, p4c, zero4()));
-      f32x4 t = l_r;
+      f32x4 l_c;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) t[j] += (4 * g + j == n) ? 1.0f : 0.0f;
-      t = mfma16(p2c, to_operand(t), t);
-      t = mfma16(p4c, to_operand(t), t);
-      t = mfma16(p8c, to_operand(t), t);
-      lds_store_transposed(sm.tri[kTT], kTriStride, g, n, t);
+      for (int j = 0; j < 4; ++j) l_c[j] = bf16_float(static_cast<uint16_t>(lc[j]));
+      lds_store_transposed(sm.tri[kTT], kTriStride, g, n, invert_unit_lower(acc, l_c));
     }
     __builtin_amdgcn_s_setprio(0);
   }

@@ -119,6 +119,101 @@ __device__ __forceinline__ void to_operand_split(f32x4 c, i16x4& hi, i16x4& lo) 
   lo = __builtin_bit_cast(i16x4, l);
 }
 
+// Inverses of I - L for a strictly lower 16 x 16 L, as every chunk form needs
+// of its diagonal blocks. Registers: X_R "lane (g, n) holds X[n][4g + j]" (A
+// operand of X, C layout of X^T) and X_C the C layout of X (B operand of X); a
+// product Z = X Y is Z_C = mfma(X_R, Y_C) and Z_R = mfma(Y_C, X_R).
+//
+// Block substitution: the four 4 x 4 diagonal blocks by substitution in fp32
+// (a block's rows lie in one quad of lanes), then twice
+//   T <- T + T E T,  E the part of L that joins pairs of inverted blocks
+// (E T E = 0, so this is exact). No power of L is formed: the product
+// (I + L)(I + L^2)(I + L^4)(I + L^8) has intermediate entries up to
+// C(14, 7) = 3432 for the L of repeated keys (every entry near -1) that must
+// cancel to the entries of T, near 1, and in bf16 they do not: states were off
+// by a factor of 1e10 after 256 tokens of one key, and are 2e-3 off with this
+// form; random keys are the same to two digits (3.7e-3).
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_mov_dpp(__float_as_int(x), 0x55 * kLane, 0xf, 0xf, true));
+}
+
+// Lane masks that depend on (g, n) alone are constants. The empty asm has them
+// written to scalar registers where they are used: hoisted out of a chunk loop,
+// as compares or as constants, they spill there (prefill 2 to 3% slower).
+template <typename F>
+constexpr uint64_t lanes_where(F f) {
+  uint64_t mask = 0;
+  for (int lane = 0; lane < 64; ++lane) {
+    if (f(lane >> 4, lane & 15)) mask |= uint64_t{1} << lane;
+  }
+  return mask;
+}
+__device__ __forceinline__ bool in_lanes(uint64_t mask) {
+  uint32_t lo = static_cast<uint32_t>(mask), hi = static_cast<uint32_t>(mask >> 32);
+  asm volatile("" : "+s"(lo), "+s"(hi));
+  return __builtin_amdgcn_inverse_ballot_w64(static_cast<uint64_t>(hi) << 32 | lo);
+}
+// Strict lower triangle of the 4 x 4 diagonal blocks: element j of a lane of
+// X_R (rows i > j) and of X_C (columns i < j), i = n - 4g.
+template <int j>
+constexpr uint64_t kRowBelow = lanes_where([](int g, int n) {
+  return n - 4 * g > j && n - 4 * g < 4;
+});
+template <int j>
+constexpr uint64_t kColumnBelow = lanes_where([](int g, int n) {
+  return n - 4 * g >= 0 && n - 4 * g < j;
+});
+template <int j>
+constexpr uint64_t kOnDiagonal = lanes_where([](int g, int n) { return n == 4 * g + j; });
+// Lanes of X_C that join 4 x 4 blocks to 8 x 8 ones, and those to 16 x 16.
+constexpr uint64_t kJoins8 = lanes_where([](int g, int n) {
+  return g % 2 == 1 && n / 4 == g - 1;
+});
+constexpr uint64_t kJoins16 = lanes_where([](int g, int n) { return g / 2 > n / 8; });
+
+// N with I + N the inverse of the 4 x 4 diagonal blocks, in both layouts, zero
+// elsewhere. Of l_r and l_c only the strict lower triangle is read.
+__device__ __forceinline__ void invert_diagonal4(f32x4 l_r, f32x4 l_c, f32x4& n_r, f32x4& n_c) {
+  // Rows: row i of the block in lane i of the quad, rows before it broadcast.
+  n_r = f32x4{in_lanes(kRowBelow<0>) ? l_r[0] : 0.0f, in_lanes(kRowBelow<1>) ? l_r[1] : 0.0f,
+              in_lanes(kRowBelow<2>) ? l_r[2] : 0.0f, 0.0f};
+  const float c1 = n_r[1], c2 = n_r[2];
+  n_r[0] += c1 * quad_lane<1>(n_r[0]);
+  const float r0 = quad_lane<2>(n_r[0]), r1 = quad_lane<2>(n_r[1]);
+  n_r[0] += c2 * r0;
+  n_r[1] += c2 * r1;
+  // Columns: column c in lane c, L's further columns broadcast.
+  n_c = f32x4{0.0f, in_lanes(kColumnBelow<1>) ? l_c[1] : 0.0f,
+              in_lanes(kColumnBelow<2>) ? l_c[2] : 0.0f,
+              in_lanes(kColumnBelow<3>) ? l_c[3] : 0.0f};
+  const float l2 = n_c[2], l3 = n_c[3];
+  n_c[2] += quad_lane<1>(l2) * n_c[1];
+  n_c[3] += quad_lane<1>(l3) * n_c[1];
+  n_c[3] += quad_lane<2>(l3) * n_c[2];
+}
+
+// T_R of (I - L)^{-1} with bf16 operands (see above), by T <- (I + T E) T: five
+// matrix products, four of them in a chain. The identity goes into operands
+// whose diagonal is zero; of l_r and l_c only the strict lower triangle is read.
+__device__ __forceinline__ f32x4 invert_unit_lower(f32x4 l_r, f32x4 l_c) {
+  f32x4 n_r, n_c;
+  invert_diagonal4(l_r, l_c, n_r, n_c);
+  const u32x2 one = {
+      (in_lanes(kOnDiagonal<0>) ? 0x3f80u : 0u) | (in_lanes(kOnDiagonal<1>) ? 0x3f800000u : 0u),
+      (in_lanes(kOnDiagonal<2>) ? 0x3f80u : 0u) | (in_lanes(kOnDiagonal<3>) ? 0x3f800000u : 0u)};
+  auto plus_one = [&](f32x4 x) {
+    return __builtin_bit_cast(i16x4, __builtin_bit_cast(u32x2, to_operand(x)) | one);
+  };
+  const i16x4 zero = {0, 0, 0, 0};
+  const i16x4 l = to_operand(l_c), t4_r = plus_one(n_r), t4_c = plus_one(n_c);
+  const i16x4 x = plus_one(mfma16(in_lanes(kJoins8) ? l : zero, t4_r, zero4()));
+  const f32x4 t8_r = mfma16(t4_c, x, zero4()), t8_c = mfma16(x, t4_c, zero4());
+  const i16x4 y = plus_one(mfma16(in_lanes(kJoins16) ? l : zero, to_operand(t8_r), zero4()));
+  return mfma16(to_operand(t8_c), y, zero4());
+}
+
 // Operand read from an LDS tile: 4 consecutive bf16 of row `row` starting at
 // column `col` (8-byte aligned). Serves as A operand (row = m, col = k0) or
 // as B operand of a tile stored [n][k] (row = n, col = k0).
