@@ -382,35 +382,31 @@ __global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
       for (int m = 0; m < 5; ++m) tri[m] += part[q][m][lane];
     }
   }
-  f32x4 lab_r = tri[0], lab_c = tri[1], lak = tri[2], arb = tri[3], ark = tri[4];
+  const f32x4 lab_r = tri[0], lab_c = tri[1];
+  f32x4 lak = tri[2], arb = tri[3], ark = tri[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int i = 4 * g + j;
-    lab_r[j] = i < n ? lab_r[j] : 0.0f;
-    lab_c[j] = n < i ? lab_c[j] : 0.0f;
     const bool strict = kBackward ? n < i : i < n;  // source before target
     lak[j] = strict ? lak[j] : 0.0f;
     arb[j] = strict || i == n ? arb[j] : 0.0f;
     ark[j] = strict || i == n ? ark[j] : 0.0f;
   }
-  // L and L^T exchange their layouts: the inverse of I - L^T is T^T.
-  if constexpr (kBackward) {
-    const f32x4 x = lab_r;
-    lab_r = lab_c;
-    lab_c = x;
-  }
-  // (I - L)^{-1} = (I + L)(I + L^2)(I + L^4)(I + L^8) for the strictly lower
-  // L. With X_R "lane (g, n) holds X[n][4g + j]" and X_C the C layout,
-  // Z = X Y is Z_C = X_R Y_C and Z_R = Y_C X_R.
-  const f32x4 p2c = mm16(lab_r, lab_c, zero4()), p2r = mm16(lab_c, lab_r, zero4());
-  const f32x4 p4c = mm16(p2r, p2c, zero4()), p4r = mm16(p2c, p2r, zero4());
-  const f32x4 p8c = mm16(p4r, p4c, zero4());
-  f32x4 t = lab_r;
+  // (I - L)^{-1} by block substitution (wkv7_mfma.h): in fp32 too, products of
+  // powers of L lose up to four digits to cancellation where the keys are
+  // similar (states 1e-5 off fp64 against 2e-7). The backward takes T^T, T_C.
+  f32x4 t_r, t_c;
+  invert_diagonal4(lab_r, lab_c, t_r, t_c);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) t[j] += (4 * g + j == n) ? 1.0f : 0.0f;
-  t = mm16(p2c, t, t);
-  t = mm16(p4c, t, t);
-  t = mm16(p8c, t, t);
+  for (int j = 0; j < 4; ++j) {
+    const float one = 4 * g + j == n ? 1.0f : 0.0f;
+    t_r[j] += one;
+    t_c[j] += one;
+  }
+  const f32x4 x = mm16(in_lanes(kJoins8) ? lab_c : zero4(), t_r, zero4());
+  const f32x4 t8_r = mm16(t_c, x, t_r), t8_c = mm16(x, t_c, t_c);
+  const f32x4 y = mm16(in_lanes(kJoins16) ? lab_c : zero4(), t8_r, zero4());
+  const f32x4 t = kBackward ? mm16(y, t8_c, t8_c) : mm16(t8_c, y, t8_r);
   float* const out = tiles + (kBackward ? L::kBackTri : L::kTri) + n * kPiece + 4 * g;
   *reinterpret_cast<f32x4*>(out) = t;
   *reinterpret_cast<f32x4*>(out + kTriElems) = lak;

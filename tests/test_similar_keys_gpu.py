@@ -57,6 +57,9 @@ def _reference(tok):
     ("chunk", torch.bfloat16, 64, (700,), 2e-2, 2e-2),
     ("recurrent", torch.bfloat16, 64, (130, 70), 2e-2, 2e-3),
     ("recurrent", torch.bfloat16, 64, (700,), 2e-2, 2e-3),
+    ("recurrent", torch.float16, 64, (130, 70), 1e-3, 1e-6),
+    ("recurrent", torch.float16, 128, (256,), 1e-3, 1e-6),
+    ("recurrent", torch.bfloat16, 256, (130, 70), 4e-3, 1e-6),
 ])
 def test_forward(entry, dtype, d, lengths, tol_y, tol_state, spread, rate):
     n = sum(lengths)
@@ -88,6 +91,7 @@ def test_forward(entry, dtype, d, lengths, tol_y, tol_state, spread, rate):
     (64, (130, 70), torch.bfloat16, 2e-2, 2e-2),
     (64, (640,), torch.bfloat16, 2e-2, 2e-2),
     (128, (130, 70), torch.bfloat16, 2e-2, 2e-2),
+    (256, (130, 70), torch.float16, 1e-3, 1e-6),
 ])
 def test_training(d, lengths, dtype, tol, tol_state, spread, rate):
     n = sum(lengths)
