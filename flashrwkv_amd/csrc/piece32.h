@@ -61,6 +61,10 @@ struct Piece32Params {
   // Scratch areas (piece32_forward_bytes / piece32_backward_bytes).
   int4* table;      // caller chunks: {first token, tokens, chunk, piece of chunk} per piece
   int32_t* base;    // caller chunks: first piece of each chunk, [num_segments + 1]
+  // [H, piece slots]: 1 where the piece holds a value that is not finite (or
+  // products of its tokens overflow). Such a unit runs token by token.
+  uint32_t* flags;
+  int32_t slots_total;
   float* tiles;     // operand tiles per (piece, head)
   float* adjoints;  // backward: dS at the piece end per (piece, head), [D, D]
   float* dz;        // backward: dZ per (piece, head), [16, D]

@@ -15,6 +15,13 @@
 // least exp(-e^{-1/2}), so a piece's decay stays above 2^-14 and one reference
 // point serves a piece (raw retentions stay on the per-token kernels).
 //
+// The matrix products spread a NaN or an infinity over a whole piece (a masked
+// zero times NaN is NaN), and to earlier tokens of it. A (sequence, head) with
+// one anywhere in its tokens therefore runs token by token, as the per-token
+// kernels do, so that it reaches later tokens only: the preparation flags its
+// pieces, the forward walks the unit's tokens (token_form) and the backward
+// leaves it to train_recurrent.hip.
+//
 // Several kernels, so that the serial chain over pieces holds nothing but the
 // state products:
 //   piece32_prepare   every piece at once: decodes the rows, scans the decay
@@ -36,11 +43,11 @@
 #include "capi_internal.h"
 #include "chunk_common.h"
 #include "piece32.h"
+#include "train_common.h"
 
 namespace frwkv {
 namespace {
 
-constexpr int kPiece = 16;
 constexpr int kTriElems = kPiece * kPiece;
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
@@ -103,12 +110,6 @@ struct Tiles {
   static constexpr int kBackward = kBackTri + 4 * kTriElems;
 };
 
-// Read-only metadata through scalar loads, which do not wait for the vector
-// memory operations in flight.
-__device__ __forceinline__ int32_t meta_at(const int32_t* a, int64_t i) {
-  return ((const __attribute__((address_space(4))) int32_t*)a)[i];
-}
-
 // A pointer known to be the same in every lane, in scalar registers.
 template <typename P>
 __device__ __forceinline__ P* uniform_pointer(P* x) {
@@ -164,6 +165,15 @@ __device__ __forceinline__ int4 piece_at(const Piece32Params& p, const Walk& w, 
   }
   const int start = w.begin + kPiece * i;
   return make_int4(start, min(kPiece, w.end - start), 0, i);
+}
+
+// True when the unit runs token by token (uniform over its workgroups).
+__device__ __forceinline__ bool unit_flagged(const Piece32Params& p, const Walk& w, int head,
+                                             int lane) {
+  bool bad = false;
+  const uint32_t* flags = p.flags + static_cast<int64_t>(head) * p.slots_total + w.first;
+  for (int i = lane; i < w.count; i += 64) bad |= flags[i] != 0;
+  return __builtin_amdgcn_ballot_w64(bad) != 0;
 }
 
 // The packed sequence that owns a slot (or the last one that starts at or
@@ -231,6 +241,14 @@ __device__ __forceinline__ f32x4 widen4(u32x2 q) {
                to_f32<T>(static_cast<uint16_t>(q.y)), to_f32<T>(static_cast<uint16_t>(q.y >> 16))};
 }
 
+// Whether one of two packed 16-bit values is an infinity or NaN (its exponent
+// bits, five or eight, are all set).
+template <typename T>
+__device__ __forceinline__ bool not_finite(uint32_t x) {
+  constexpr uint32_t kExponent = __is_same(T, Bf16) ? 0x7f80u : 0x7c00u;
+  return (x & kExponent) == kExponent || ((x >> 16) & kExponent) == kExponent;
+}
+
 // Cumulative decay of a piece at token n of the lane's 16-lane row, from the
 // logits' log2 retentions: 2^G, 2^Gp and 2^-G of sums of logs. A sum of small
 // logs keeps the slow channels (the largest states) more exact than a product
@@ -262,6 +280,7 @@ __global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
   constexpr int kWaves = D / 64;
   using L = Tiles<D>;
   __shared__ f32x4 part[kWaves > 1 ? kWaves : 1][5][64];
+  __shared__ bool wave_bad[kWaves];
   if (p.status != nullptr && p.status[0] != 0) return;
   const int heads = p.num_heads;
   const int head = static_cast<int>(blockIdx.x) % heads;
@@ -304,6 +323,20 @@ __global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
     qr[kb] = load4(rr, off + 32 * kb);
     qb[kb] = load4(rb, off + 32 * kb);
     qk[kb] = load4(rk, off + 32 * kb);
+  }
+  // Values that the tiles do not hold: V, and dY in the backward.
+  const auto rv = rows(p.v);
+  const bool with_dy = kBackward && p.dy != nullptr;
+  const auto rdy = with_dy ? rows(p.dy) : buffer_rsrc(static_cast<const S16*>(nullptr), 0u);
+  bool bad = false;
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    const u32x2 x = load4(rv, off + 32 * kb);
+    bad |= not_finite<T>(x.x) || not_finite<T>(x.y);
+    if constexpr (kBackward) {
+      const u32x2 y = load4(rdy, off + 32 * kb);
+      bad |= not_finite<T>(y.x) || not_finite<T>(y.y);
+    }
   }
   float* const tiles = p.tiles + (static_cast<int64_t>(slot) * heads + head) *
                                      (kBackward ? L::kBackward : L::kForward);
@@ -374,13 +407,23 @@ __global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
   if constexpr (kWaves > 1) {
 #pragma unroll
     for (int m = 0; m < 5; ++m) part[wave][m][lane] = tri[m];
+    wave_bad[wave] = __builtin_amdgcn_ballot_w64(bad) != 0;
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
     for (int q = 1; q < kWaves; ++q) {
 #pragma unroll
       for (int m = 0; m < 5; ++m) tri[m] += part[q][m][lane];
+      bad |= wave_bad[q];
     }
+  }
+  // A value of r, w, k, a or b that is not finite makes a sum of Lab or Ark so
+  // (before the masks, every row meets every other).
+  float probe = 0.0f;
+#pragma unroll
+  for (int m = 0; m < 5; ++m) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) probe = fmaf(tri[m][j], 0.0f, probe);
   }
   const f32x4 lab_r = tri[0], lab_c = tri[1];
   f32x4 lak = tri[2], arb = tri[3], ark = tri[4];
@@ -407,11 +450,129 @@ __global__ __launch_bounds__(D) void piece32_prepare(Piece32Params p) {
   const f32x4 t8_r = mm16(t_c, x, t_r), t8_c = mm16(x, t_c, t_c);
   const f32x4 y = mm16(in_lanes(kJoins16) ? lab_c : zero4(), t8_r, zero4());
   const f32x4 t = kBackward ? mm16(y, t8_c, t8_c) : mm16(t8_c, y, t8_r);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) probe = fmaf(t[j], 0.0f, probe);
+  bad |= !(probe == 0.0f);
+  const uint32_t flag = __builtin_amdgcn_ballot_w64(bad) != 0;
+  if (lane == 0) p.flags[static_cast<int64_t>(head) * p.slots_total + slot] = flag;
   float* const out = tiles + (kBackward ? L::kBackTri : L::kTri) + n * kPiece + 4 * g;
   *reinterpret_cast<f32x4*>(out) = t;
   *reinterpret_cast<f32x4*>(out + kTriElems) = lak;
   *reinterpret_cast<f32x4*>(out + 2 * kTriElems) = arb;
   *reinterpret_cast<f32x4*>(out + 3 * kTriElems) = ark;
+}
+
+// A flagged unit's tokens one by one, on the state slab of the forward kernel
+// (wave: keys 64q .. +63, lane: keys 64q + 16kb + 4g + j of column col), with
+// the outputs of the chain:
+//   sa = a^T S,  S <- diag(w) S + b sa^T + k v^T,  y = scale r^T S.
+// red: 8 x 64 floats of LDS for the sums over the waves that share columns.
+template <typename T, int D, bool kTrain, typename Store>
+__device__ __forceinline__ void token_form(const Piece32Params& p, const Walk& walk, int seq,
+                                           int head, int col, f32x4 (&S)[4], f32x4* red,
+                                           Store&& store_state) {
+  constexpr int kKeyWaves = D / 64;
+  using S16 = typename IoTraits<T>::storage;
+  const int wave = uniform(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int kq = wave % kKeyWaves;
+  const int key0 = 64 * kq + 4 * g;
+  constexpr int64_t kState = static_cast<int64_t>(D) * D;
+  // Sum over the keys. Two areas in turn: a wave writes one again only after
+  // the barrier that follows its reads.
+  auto over_waves = [&](float x, int area) {
+    x = add_xor32(add_xor16(x));
+    if constexpr (kKeyWaves > 1) {
+      float* const at = reinterpret_cast<float*>(red) + 64 * area;
+      if (g == 0) at[16 * wave + n] = x;
+      __syncthreads();
+      x = 0.0f;
+#pragma unroll
+      for (int q = 0; q < kKeyWaves; ++q) x += at[16 * (wave - kq + q) + n];
+    }
+    return x;
+  };
+  f32x4 bias[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    bias[kb] = zero4();
+    if (p.bias != nullptr) {
+      const S16* src = static_cast<const S16*>(p.bias) + static_cast<int64_t>(head) * D + key0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bias[kb][j] = to_f32<T>(src[16 * kb + j]);
+    }
+  }
+  auto tokens = [&](int begin, int end) {
+    for (int t = begin; t < end; ++t) {
+      const int64_t row = (static_cast<int64_t>(t) * p.num_heads + head) * D;
+      auto row4 = [&](const void* x, int kb) {
+        return widen4<T>(*reinterpret_cast<const u32x2*>(static_cast<const S16*>(x) + row + key0 +
+                                                         16 * kb));
+      };
+      const float v = to_f32<T>(static_cast<const S16*>(p.v)[row + col]);
+      f32x4 w[4], a[4], b[4], k[4], r[4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        w[kb] = row4(p.decay, kb) + bias[kb];
+        a[kb] = row4(p.a, kb);
+        b[kb] = row4(p.b, kb);
+        k[kb] = row4(p.k, kb);
+        r[kb] = row4(p.r, kb);
+      }
+      float sa = 0.0f, y = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sa = fmaf(a[kb][j], S[kb][j], sa);
+      }
+      sa = over_waves(sa, 0);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float x = decay_retention<DecayMode::kLogits>(w[kb][j]);
+          S[kb][j] = fmaf(x, S[kb][j], fmaf(b[kb][j], sa, k[kb][j] * v));
+          y = fmaf(r[kb][j], S[kb][j], y);
+        }
+      }
+      y = over_waves(y, 1);
+      if (g == 0 && kq == 0) {
+        static_cast<S16*>(p.out)[row + col] = from_f32<T>(p.scale * y);
+        if constexpr (kTrain) p.state_dot_a[row + col] = sa;
+      }
+    }
+  };
+  if constexpr (kTrain) {
+    // The state at every chunk start, and every 16 tokens inside a chunk.
+    auto chunk = [&](int start, int end, float* at_start, bool interior) {
+      store_state(at_start);
+      for (int t = start; t < end; t += kPiece) {
+        if (interior && t > start) {
+          store_state(p.interior +
+                      (static_cast<int64_t>(t / kPiece) * p.num_heads + head) * kState);
+        }
+        tokens(t, min(t + kPiece, end));
+      }
+    };
+    if (p.seg_offsets != nullptr) {
+      const int hi = min(meta_at(p.seg_offsets, seq + 1), p.num_segments);
+      for (int c = max(meta_at(p.seg_offsets, seq), 0); c < hi; ++c) {
+        const int start = min(max(meta_at(p.seg_starts, c), 0), p.total_tokens);
+        const int end = min(meta_at(p.seg_ends, c), p.total_tokens);
+        chunk(start, end, p.boundary + (static_cast<int64_t>(c) * p.num_heads + head) * kState,
+              p.interior != nullptr);
+      }
+      return;
+    }
+    float* at = p.boundary + (static_cast<int64_t>(seq) * p.num_heads + head) *
+                                 (p.dense_t / kPiece) * kState;
+    for (int t = walk.begin; t < walk.end; t += kPiece, at += kState) {
+      chunk(t, t + kPiece, at, false);
+    }
+  } else {
+    tokens(walk.begin, walk.end);
+  }
 }
 
 // The chain over a sequence's pieces. Wave: keys 64q .. +63 (q = wave % (D /
@@ -635,9 +796,17 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
     }
   };
 
+  // At wide heads the first piece's loads fly while the flags are looked at (1%
+  // of a pass); at D = 64 that costs registers and 10%.
+  Ops even{}, odd;
+  if (kKeyWaves > 1 && walk.count > 0) load(even, 0, piece_at(p, walk, 0));
+  if (unit_flagged(p, walk, head, lane)) {
+    token_form<T, D, kTrain>(p, walk, seq, head, col, S, &part[0][0][0][0], store_state);
+    if (state != nullptr) store_state(state);
+    return;
+  }
   if (walk.count > 0) {
-    Ops even, odd;
-    load(even, 0, piece_at(p, walk, 0));
+    if (kKeyWaves == 1) load(even, 0, piece_at(p, walk, 0));
     for (int i = 0;; i += 2) {
       step(even, odd, i);
       if (i + 1 >= walk.count) break;
@@ -798,9 +967,11 @@ __global__ __launch_bounds__(256, 1) void piece32_adjoint_kernel(Piece32Params p
     p.dz[ph * (kPiece * D) + (4 * g + kq) * D + col] = dzq;
   };
 
+  // The first loads fly while the flags are looked at.
+  Ops even{}, odd;
+  if (walk.count > 0) load(even, walk.count - 1, piece_at(p, walk, walk.count - 1));
+  if (unit_flagged(p, walk, head, lane)) return;  // train_recurrent.hip
   if (walk.count > 0) {
-    Ops even, odd;
-    load(even, walk.count - 1, piece_at(p, walk, walk.count - 1));
     for (int i = walk.count - 1;; i -= 2) {
       step(even, odd, i);
       if (i < 1) break;
@@ -1043,11 +1214,14 @@ size_t tile_bytes(int head_size, int64_t heads, int64_t slots, bool backward) {
   return round256(static_cast<size_t>(slots) * heads * floats * sizeof(float));
 }
 
-// Scratch: the piece table, the chunks' first pieces, the tiles, then the
+// Scratch: the piece table, the chunks' first pieces, the flags, the tiles, then the
 // backward's adjoints and dZ.
 size_t table_bytes(int64_t slots) { return round256(static_cast<size_t>(slots) * sizeof(int4)); }
 size_t base_bytes(int64_t lists) {
   return round256((static_cast<size_t>(lists) + 1) * sizeof(int32_t));
+}
+size_t flag_bytes(int64_t heads, int64_t slots) {
+  return round256(static_cast<size_t>(heads) * slots * sizeof(uint32_t));
 }
 
 void lay_out(Piece32Params& p, int head_size, bool backward, void* scratch) {
@@ -1057,6 +1231,9 @@ void lay_out(Piece32Params& p, int head_size, bool backward, void* scratch) {
   at += table_bytes(slots);
   p.base = reinterpret_cast<int32_t*>(at);
   at += base_bytes(lists_of(p));
+  p.flags = reinterpret_cast<uint32_t*>(at);
+  p.slots_total = static_cast<int32_t>(slots);
+  at += flag_bytes(p.num_heads, slots);
   p.tiles = reinterpret_cast<float*>(at);
   at += tile_bytes(head_size, p.num_heads, slots, backward);
   p.adjoints = reinterpret_cast<float*>(at);
@@ -1125,18 +1302,58 @@ int launch_backward(const Piece32Params& p, hipStream_t stream) {
   return check_launch("piece32_gradient_kernel");
 }
 
+// The flagged units' gradients, token by token; their sums over value columns
+// go through the adjoints' area (at least 16 * 256 floats a token and head).
+TrainParams redo_params(const Piece32Params& p) {
+  TrainParams q{};
+  q.num_heads = p.num_heads;
+  q.total_tokens = p.total_tokens;
+  q.num_sequences = p.num_sequences;
+  q.seg_offsets = p.seg_offsets;
+  q.seg_starts = p.seg_starts;
+  q.seg_ends = p.seg_ends;
+  q.num_chunks = p.num_segments;
+  q.dense_t = p.dense_t;
+  q.ckpt = p.boundary;
+  q.interior = p.interior;
+  q.r = p.r;
+  q.decay = p.decay;
+  q.bias = p.bias;
+  q.k = p.k;
+  q.v = p.v;
+  q.a = p.a;
+  q.b = p.b;
+  q.dy = p.dy;
+  q.dstate_final = p.dstate_final;
+  q.dr = p.dr;
+  q.ddecay = p.ddecay;
+  q.dk = p.dk;
+  q.dv = p.dv;
+  q.da = p.da;
+  q.db = p.db;
+  q.dstate0 = p.dstate0;
+  q.accum = p.adjoints;
+  q.scale = p.scale;
+  q.redo_flags = p.flags;
+  q.redo_slots = p.slots_total;
+  q.redo_base = p.seg_offsets != nullptr ? p.base : nullptr;
+  return q;
+}
+
 }  // namespace
 
 size_t piece32_forward_bytes(int head_size, int64_t heads, int64_t tokens, int64_t lists) {
   if (heads <= 0 || tokens <= 0 || lists <= 0) return 0;
   const int64_t slots = piece32_slots(tokens, lists);
-  return table_bytes(slots) + base_bytes(lists) + tile_bytes(head_size, heads, slots, false);
+  return table_bytes(slots) + base_bytes(lists) + flag_bytes(heads, slots) +
+         tile_bytes(head_size, heads, slots, false);
 }
 
 size_t piece32_backward_bytes(int64_t heads, int64_t tokens, int64_t lists) {
   if (heads <= 0 || tokens <= 0 || lists <= 0) return 0;
   const int64_t slots = piece32_slots(tokens, lists);
-  return table_bytes(slots) + base_bytes(lists) + tile_bytes(256, heads, slots, true) +
+  return table_bytes(slots) + base_bytes(lists) + flag_bytes(heads, slots) +
+         tile_bytes(256, heads, slots, true) +
          static_cast<size_t>(slots) * heads * (256 + kPiece) * 256 * sizeof(float);
 }
 
@@ -1149,8 +1366,10 @@ int piece32_forward(Piece32Params p, int head_size, int io_dtype, void* scratch,
 
 int piece32_backward(Piece32Params p, int io_dtype, void* scratch, hipStream_t stream) {
   lay_out(p, 256, true, scratch);
-  return io_dtype == FRWKV_DTYPE_BF16 ? launch_backward<Bf16>(p, stream)
-                                      : launch_backward<F16>(p, stream);
+  const int rc = io_dtype == FRWKV_DTYPE_BF16 ? launch_backward<Bf16>(p, stream)
+                                              : launch_backward<F16>(p, stream);
+  if (rc != FRWKV_OK) return rc;
+  return launch_train_redo(redo_params(p), io_dtype, p.num_sequences * p.num_heads, stream);
 }
 
 }  // namespace frwkv

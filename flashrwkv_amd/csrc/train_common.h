@@ -62,6 +62,12 @@ struct TrainParams {
   // state[c]), only the interior states are written; chunks of at most 16
   // tokens are skipped and a chunk's last piece is not computed.
   int32_t fill_only;
+  // launch_train_redo: the pieces' flags of the fp32 matrix form, [H, slots],
+  // and with caller chunks the first piece of each chunk, [num_chunks + 1]
+  // (Piece32Params::base).
+  const uint32_t* redo_flags;
+  int32_t redo_slots;
+  const int32_t* redo_base;
 };
 
 struct Chunk {
@@ -72,7 +78,7 @@ struct Chunk {
 // Chunk metadata is read-only for a whole launch: read it through the
 // constant address space, so that its (uniform) reads are scalar loads,
 // which do not wait for the vector memory operations in flight.
-__device__ __forceinline__ int32_t meta_at(const int32_t* a, int i) {
+__device__ __forceinline__ int32_t meta_at(const int32_t* a, int64_t i) {
   return ((const __attribute__((address_space(4))) int32_t*)a)[i];
 }
 
@@ -117,5 +123,10 @@ __device__ __forceinline__ Chunk chunk_at(const TrainParams& p, int seq, int hea
 // the per-token kernels (one workgroup per unit); interior states in bf16.
 int launch_piece_train(const TrainParams& p, int io_dtype, int decay_mode, int units,
                        bool backward, hipStream_t stream);
+
+// The per-token backward at head size 256 of the units that the fp32 matrix
+// form flagged (piece32.hip); the others are left as they are. Decay logits;
+// accum holds 5 x N x H x D floats.
+int launch_train_redo(const TrainParams& p, int io_dtype, int units, hipStream_t stream);
 
 }  // namespace frwkv

@@ -420,24 +420,23 @@ struct BwdSmem {
   float red[2][kNW][5][D];
 };
 
-template <int D, typename T, DecayMode M>
-__global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_kernel(TrainParams p) {
+// kRedo: the caller walks a unit's groups in turn with one workgroup, and the
+// sums over columns are added up in one slice; the last group stores them.
+template <int D, typename T, DecayMode M, bool kRedo>
+__device__ __forceinline__ void train_bwd_unit(BwdSmem<D>& sm, const TrainParams& p, int unit,
+                                               int group) {
   using L = Layout<D>;
   using Sg = Staging<D>;
   using St = typename IoTraits<T>::storage;
   constexpr int kRpl = L::kRpl;
   constexpr int kThreads = L::kThreads;
   constexpr int kGroups = L::kGroups;
-  static_assert(sizeof(BwdSmem<D>) <= 160 * 1024, "backward LDS budget");
-  __shared__ BwdSmem<D> sm;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int cg = lane % L::kCg, rg = lane / L::kCg;
   const int row0 = rg * kRpl;
-  const int unit = blockIdx.x / kGroups;
-  const int group = blockIdx.x % kGroups;
   const int col0 = group * L::kCols;
   const int wcol = L::kCW * wave + 4 * cg;
   const int col = col0 + wcol;
@@ -470,9 +469,18 @@ __global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_kernel(TrainPar
 
   // Where this workgroup's per-key gradient gi of element `off` goes.
   auto key_store = [&](int gi, int64_t off, float4 x) {
+    void* const outs[5] = {p.dr, p.dk, p.db, p.ddecay, p.da};
     if constexpr (kGroups == 1) {
-      void* const outs[5] = {p.dr, p.dk, p.db, p.ddecay, p.da};
       store4<T>(static_cast<St*>(outs[gi]) + off, x.x, x.y, x.z, x.w);
+    } else if constexpr (kRedo) {
+      // The same thread holds an element in every group.
+      float4* const sum = reinterpret_cast<float4*>(p.accum + gi * slice + off);
+      if (group > 0) x = make_float4(sum->x + x.x, sum->y + x.y, sum->z + x.z, sum->w + x.w);
+      if (group == kGroups - 1) {
+        store4<T>(static_cast<St*>(outs[gi]) + off, x.x, x.y, x.z, x.w);
+      } else {
+        *sum = x;
+      }
     } else {
       *reinterpret_cast<float4*>(p.accum + (group * 5 + gi) * slice + off) = x;
     }
@@ -717,6 +725,36 @@ __global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_kernel(TrainPar
   }
 }
 
+template <int D, typename T, DecayMode M>
+__global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_kernel(TrainParams p) {
+  static_assert(sizeof(BwdSmem<D>) <= 160 * 1024, "backward LDS budget");
+  __shared__ BwdSmem<D> sm;
+  constexpr int kGroups = Layout<D>::kGroups;
+  train_bwd_unit<D, T, M, false>(sm, p, blockIdx.x / kGroups, blockIdx.x % kGroups);
+}
+
+// The flagged units (launch_train_redo), one workgroup each.
+template <int D, typename T>
+__global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_redo_kernel(TrainParams p) {
+  __shared__ BwdSmem<D> sm;
+  const int seq = blockIdx.x / p.num_heads, head = blockIdx.x % p.num_heads;
+  int first = seq * (p.dense_t / kPiece), count = p.dense_t / kPiece;
+  bool bad = false;
+  if (p.redo_base != nullptr) {
+    const int lo = min(max(meta_at(p.seg_offsets, seq), 0), p.num_chunks);
+    const int hi = min(max(meta_at(p.seg_offsets, seq + 1), lo), p.num_chunks);
+    first = meta_at(p.redo_base, lo);
+    count = meta_at(p.redo_base, hi) - first;
+  }
+  const uint32_t* flags = p.redo_flags + static_cast<int64_t>(head) * p.redo_slots + first;
+  for (int i = threadIdx.x & 63; i < count; i += 64) bad |= flags[i] != 0;
+  if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+  for (int group = 0; group < Layout<D>::kGroups; ++group) {
+    train_bwd_unit<D, T, DecayMode::kLogits, true>(sm, p, blockIdx.x, group);
+    __syncthreads();
+  }
+}
+
 // Per-group fp32 slices [groups, 5, n] -> dr, dk, db, ddecay, da in the io
 // dtype, adding the slices in group order.
 template <typename T, int kGroups>
@@ -822,6 +860,17 @@ int dispatch_train_io(const TrainParams& p, int io_dtype, int decay_mode, int he
 }
 
 }  // namespace
+
+int launch_train_redo(const TrainParams& p, int io_dtype, int units, hipStream_t stream) {
+  const dim3 block(Layout<256>::kThreads);
+  if (io_dtype == FRWKV_DTYPE_BF16) {
+    hipLaunchKernelGGL((train_bwd_redo_kernel<256, Bf16>), dim3(units), block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((train_bwd_redo_kernel<256, F16>), dim3(units), block, 0, stream, p);
+  }
+  return check_launch("train_bwd_redo_kernel");
+}
+
 }  // namespace frwkv
 
 int frwkv_train_recurrent_forward(int io_dtype, int decay_mode, int32_t num_sequences,
