@@ -60,7 +60,8 @@ struct Piece32Params {
   float* dstate0;  // or null
   // Scratch areas (piece32_forward_bytes / piece32_backward_bytes).
   int4* table;      // caller chunks: {first token, tokens, chunk, piece of chunk} per piece
-  int32_t* base;    // caller chunks: first piece of each chunk, [num_segments + 1]
+  int32_t* base;    // caller chunks: first piece of each chunk, [num_segments + 1], then
+                    // 1 if the chunks have more pieces than there are slots
   // [H, piece slots]: 1 where the piece holds a value that is not finite (or
   // products of its tokens overflow). Such a unit runs token by token.
   uint32_t* flags;

@@ -170,7 +170,7 @@ __device__ __forceinline__ int4 piece_at(const Piece32Params& p, const Walk& w, 
 // True when the unit runs token by token (uniform over its workgroups).
 __device__ __forceinline__ bool unit_flagged(const Piece32Params& p, const Walk& w, int head,
                                              int lane) {
-  bool bad = false;
+  bool bad = p.seg_offsets != nullptr && meta_at(p.base, p.num_segments + 1) != 0;
   const uint32_t* flags = p.flags + static_cast<int64_t>(head) * p.slots_total + w.first;
   for (int i = lane; i < w.count; i += 64) bad |= flags[i] != 0;
   return __builtin_amdgcn_ballot_w64(bad) != 0;
@@ -194,8 +194,8 @@ __device__ __forceinline__ int sequence_of_slot(const Piece32Params& p, int slot
 
 // Slots of the caller chunks' pieces in chunk order, one workgroup. Token
 // ranges are clamped to the call's; an empty chunk has one piece of no tokens
-// (its start state is an output too), and pieces beyond the slots (overlapping
-// chunks) are dropped.
+// (its start state is an output too). Overlapping chunks can have more pieces
+// than there are slots; every unit then runs token by token.
 constexpr int kTableThreads = 1024;
 __global__ __launch_bounds__(kTableThreads) void piece32_table(Piece32Params p, int slots) {
   __shared__ int sums[kTableThreads];
@@ -227,7 +227,10 @@ __global__ __launch_bounds__(kTableThreads) void piece32_table(Piece32Params p, 
     before += sums[kTableThreads - 1];
     __syncthreads();
   }
-  if (tid == 0) p.base[p.num_segments] = min(before, slots);
+  if (tid == 0) {
+    p.base[p.num_segments] = min(before, slots);
+    p.base[p.num_segments + 1] = before > slots;
+  }
   for (int i = before + tid; i < slots; i += kTableThreads) p.table[i] = make_int4(0, 0, -1, 0);
 }
 
@@ -1218,7 +1221,7 @@ size_t tile_bytes(int head_size, int64_t heads, int64_t slots, bool backward) {
 // backward's adjoints and dZ.
 size_t table_bytes(int64_t slots) { return round256(static_cast<size_t>(slots) * sizeof(int4)); }
 size_t base_bytes(int64_t lists) {
-  return round256((static_cast<size_t>(lists) + 1) * sizeof(int32_t));
+  return round256((static_cast<size_t>(lists) + 2) * sizeof(int32_t));
 }
 size_t flag_bytes(int64_t heads, int64_t slots) {
   return round256(static_cast<size_t>(heads) * slots * sizeof(uint32_t));

@@ -63,8 +63,8 @@ struct TrainParams {
   // tokens are skipped and a chunk's last piece is not computed.
   int32_t fill_only;
   // launch_train_redo: the pieces' flags of the fp32 matrix form, [H, slots],
-  // and with caller chunks the first piece of each chunk, [num_chunks + 1]
-  // (Piece32Params::base).
+  // and with caller chunks the first piece of each chunk, [num_chunks + 1],
+  // then a word that flags every unit (Piece32Params::base).
   const uint32_t* redo_flags;
   int32_t redo_slots;
   const int32_t* redo_base;

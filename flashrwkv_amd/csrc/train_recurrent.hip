@@ -745,6 +745,7 @@ __global__ __launch_bounds__(Layout<D>::kThreads) void train_bwd_redo_kernel(Tra
     const int hi = min(max(meta_at(p.seg_offsets, seq + 1), lo), p.num_chunks);
     first = meta_at(p.redo_base, lo);
     count = meta_at(p.redo_base, hi) - first;
+    bad = meta_at(p.redo_base, p.num_chunks + 1) != 0;
   }
   const uint32_t* flags = p.redo_flags + static_cast<int64_t>(head) * p.redo_slots + first;
   for (int i = threadIdx.x & 63; i < count; i += 64) bad |= flags[i] != 0;

@@ -210,6 +210,45 @@ def test_fp32_matrix_training(dtype, chunks, with_dy, with_ds):
     parity.check("dS0", grads[-1], ref["dstate0"], 1e-5)
 
 
+# Chunks that overlap have more 16-token pieces than the matrix form has slots
+# for: the final states, the boundaries, y of the last visit of a token and dS0
+# (which depends on no state) are still those of the recurrence. Both sequences
+# visit the same tokens, each four times, so y is checked with one sequence.
+@pytest.mark.parametrize("sequences", (1, 2))
+def test_fp32_matrix_training_overlapping_chunks(sequences):
+    heads, d, n, visits = 2, 256, 64, 4
+    case = workloads.make_case(lengths=(n,), heads=heads, head_size=d, dtype=torch.bfloat16,
+                               seed=11, state_std=0.1)
+    gen = torch.Generator().manual_seed(12)
+    tok = {x: case[x] for x in NAMES}
+    tok["w"] = torch.randn(case["r"].shape, generator=gen).to(torch.bfloat16)
+    s0 = torch.randn((sequences, heads, d, d), generator=gen) * 0.1
+    dy = torch.randn(case["r"].shape, generator=gen).to(torch.bfloat16)
+    ds = torch.randn(s0.shape, generator=gen) * 0.05
+    chunks = sequences * visits
+    meta = [np.asarray(x, dtype=np.int32)
+            for x in (range(0, chunks + 1, visits), [0] * chunks, [n] * chunks)]
+    leaves = [tok[x].to(DEV).requires_grad_() for x in NAMES]
+    state = s0.to(DEV).requires_grad_()
+    y, final, boundary, _ = flashrwkv_amd.statetune_recurrent_fp32io16(
+        state, *(torch.from_numpy(x).to(DEV) for x in meta), *leaves)
+    grad = torch.autograd.grad((y, final), state, (dy.to(DEV), ds.to(DEV)))[0]
+    torch.cuda.synchronize()
+    x64 = {x: tok[x].double().numpy() for x in NAMES}
+    x64["w"] = oracle.retention_from_logits(x64["w"])
+    kw = dict(seg_offsets=meta[0], seg_starts=meta[1], seg_ends=meta[2],
+              state_slots=np.arange(sequences, dtype=np.int32))
+    args = [x64[x] for x in NAMES] + [s0.double().numpy()]
+    y_ref, final_ref, boundary_ref, _ = oracle.forward(
+        *args, **kw, want_boundary=True, want_state_dot_a=True)
+    ref = oracle.backward(*args, dy=dy.double().numpy(), dstate_final=ds.double().numpy(), **kw)
+    parity.check("final", final, final_ref, 1e-5)
+    parity.check("boundary", boundary, boundary_ref, 1e-5)
+    parity.check("dS0", grad, ref["dstate0"], 1e-5)
+    if sequences == 1:
+        parity.check("y", y, y_ref, 4e-3)
+
+
 # Training at head size 64: caller chunks of whole, partial, several and no
 # pieces, sequences shorter than the split and without chunks, a decay that
 # sends pieces through the sub-piece path, no upstream gradient of y or of the
