@@ -1811,6 +1811,9 @@ std::optional<std::vector<Tensor>> clampw_backward_call(
   if (!args.ok || plain.size() != 8) return std::nullopt;
   const Tensor &r = plain[0], &w = plain[1], &k = plain[2], &v = plain[3], &a = plain[4],
                &b = plain[5], &ckpt = plain[6], &sda = plain[7];
+  // The checks are done with Python objects; allocations and launches leave
+  // the interpreter to other threads, as the registered ops do.
+  pybind11::gil_scoped_release release;
   const int64_t batch = r.size(0), tokens = r.size(1), heads = r.size(2) / head_size;
   auto split = [&](const Tensor& x) { return x.view({batch, tokens, heads, head_size}); };
   std::vector<Tensor> grads;
@@ -1879,7 +1882,8 @@ PYBIND11_MODULE(_flashrwkv_amd_ops, m) {
   m.def("recurrent_fp16_call", &recurrent_fp16_call);
   m.def("advance_varlen_call", &advance_varlen_call);
   m.def("clampw_accepts", &clampw_accepts);
-  m.def("clampw_forward_call", &clampw_forward_call);
+  m.def("clampw_forward_call", &clampw_forward_call,
+        py::call_guard<py::gil_scoped_release>());
   m.def("clampw_backward_call", &clampw_backward_call);
   m.def("recurrent_fp16_advance_i32", &recurrent_fp16_advance_i32);
   m.def("recurrent_fp16_advance_i32_varlen",

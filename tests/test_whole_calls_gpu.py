@@ -2,6 +2,10 @@
 contract tables: every form of a call has the same outcome on both, the same
 result or an error of the same type and text."""
 
+import sys
+import threading
+import time
+
 import pytest
 import torch
 
@@ -148,3 +152,38 @@ def test_whole_call_and_tables_agree(which, monkeypatch):
         assert isinstance(here, list), (form, here)
         for x, y in zip(here, tables, strict=True):
             assert x.dtype == y.dtype and torch.equal(x, y), form
+
+
+# With a switch interval of minutes a thread that waits for the interpreter runs
+# only where the calling thread lets go of it.
+@pytest.mark.parametrize("direction", ["forward", "backward"])
+def test_pretraining_calls_release_the_interpreter(direction):
+    native = pretrain.C.native().direct
+    tokens = [x.view(1, 16, 128) for x in _tokens(torch.bfloat16, tokens=16)]
+    y, ckpt, sda = native.clampw_forward_call(*tokens, 64)
+    calls = {"forward": lambda: native.clampw_forward_call(*tokens, 64),
+             "backward": lambda: native.clampw_backward_call(y, [*tokens, ckpt, sda], 64)}
+    ran, kept, stop = [], [], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            ran.append(1)
+            time.sleep(0)
+
+    call, interval = calls[direction], sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    sys.setswitchinterval(600.0)
+    try:
+        thread.start()
+        before = len(ran)
+        for _ in range(2000):
+            kept.append(call())  # freeing a tensor lets go of it too
+            if len(ran) > before:
+                break
+        released = len(ran) > before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
+    torch.cuda.synchronize()
+    assert released
