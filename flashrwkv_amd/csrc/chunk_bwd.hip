@@ -1054,11 +1054,11 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   const int cs = wave & 3;                  // column slab (columns phase)
   const bool adjoint = wave >= 4;
   const int heads = p.num_heads;
-  const uint32_t units = kParts ? gridDim.x / p.parts : 1;
-  const int part = kParts ? blockIdx.x / units : 0;
-  const uint32_t unit = kParts ? blockIdx.x % units : blockIdx.x;
-  const int seq = unit / heads;
-  const int head = unit % heads;
+  PartPlace place{};
+  if constexpr (kParts) place = unit_place<false>(p);
+  const uint32_t unit = blockIdx.x;
+  const int seq = kParts ? place.seq : unit / heads;
+  const int head = kParts ? place.head : unit % heads;
   const int f0 = 32 * hf + 8 * g;
   constexpr bool dense = kDense;
   int seg_lo = dense ? 0 : uniform(max(p.seg_offsets[seq], 0));
@@ -1067,7 +1067,7 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
   bool first_part = true;                  // the part with the sequence's start
   if constexpr (kParts) {
     const int count = dense ? (p.dense_t + kChunk - 1) / kChunk : max(seg_hi - seg_lo, 0);
-    const PartRange pr = part_range(p, count, part);
+    const PartRange pr = part_range(p, count, place.part);
     if (!pr.exists) return;
     first_part = pr.last;
     if constexpr (dense) {
@@ -1095,11 +1095,11 @@ __global__ __launch_bounds__(kBwdThreads, 1) void chunk_bwd_kernel(ChunkBwdParam
 
   // dS: dL/dS at the end of the current piece, kept by the adjoint waves in
   // the LDS stash (each lane reads back only what it wrote).
-  if constexpr (kParts) {
-    static_assert(sizeof(BwdSmem) - sizeof(sm.dstash) >= kComposeBytes,
-                  "the maps fit the tiles before the stash");
+  static_assert(sizeof(BwdSmem) - sizeof(sm.dstash) >= kComposeBytes,
+                "the maps fit the tiles before the stash");
+  if (kParts && !(place.part == 0 && first_part)) {
     f32x4 x[4];
-    compose_start<kBwdThreads>(&sm, p, unit, part, x);
+    compose_start<kBwdThreads>(&sm, place, x);
     if (adjoint) {
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) sm.dstash[cs][kb][lane] = x[kb];
@@ -1511,9 +1511,10 @@ extern "C" int frwkv_statetune_backward_split(
   p.db = grad_b;
   p.dstate0 = grad_initial_state;
   p.scale = scale;
-  use_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
-            plan_caller_chunks(num_sequences, num_heads, num_chunks, kBackwardTime, kAdjointTime),
-            scratch, scratch_bytes);
+  use_unit_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
+                 plan_caller_chunks(num_sequences, num_heads, num_chunks, kBackwardTime,
+                                    kAdjointTime),
+                 scratch, scratch_bytes);
   return dispatch_bwd(p, io_dtype, decay_mode, num_sequences * num_heads,
                       static_cast<hipStream_t>(stream));
 }
@@ -1627,10 +1628,10 @@ extern "C" int frwkv_pretrain_backward_split(int io_dtype, int decay_mode, int32
   p.da = grad_a;
   p.db = grad_b;
   p.scale = 1.0f;
-  use_parts(p, static_cast<int64_t>(batch) * num_heads,
-            plan_parts(batch, num_heads, batch * chunks_of(tokens), chunks_of(tokens),
-                       kBackwardTime, kAdjointTime),
-            scratch, scratch_bytes);
+  use_unit_parts(p, static_cast<int64_t>(batch) * num_heads,
+                 plan_parts(batch, num_heads, batch * chunks_of(tokens), chunks_of(tokens),
+                            kBackwardTime, kAdjointTime),
+                 scratch, scratch_bytes);
   return dispatch_bwd(p, io_dtype, decay_mode, batch * num_heads,
                       static_cast<hipStream_t>(stream));
 }

@@ -707,14 +707,18 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   const int tp = lane & 7;   // token pair
   const int kg = lane >> 3;  // feature group
   const int heads = p.num_heads;
-  // Parts: block part * units + unit, so that (for a unit count divisible by
-  // the 8 XCDs) a unit's parts share an XCD, and its L2, in both launches.
-  const uint32_t units = kParts ? gridDim.x / p.parts : 1;
-  const int part = kParts ? blockIdx.x / units : 0;
-  const uint32_t unit = kParts ? blockIdx.x % units : blockIdx.x;
-  int seq = unit / heads;
-  if (!kParts && p.longest_first_sequences > 0) seq = sequence_by_length_rank(p, seq, lane);
-  const int head = unit % heads;
+  PartPlace place{};
+  int seq, head;
+  if constexpr (kParts) {
+    place = p.part_slots > 0 ? packed_place<false>(p, lane) : unit_place<false>(p);
+    seq = place.seq;
+    head = place.head;
+  } else {
+    const uint32_t unit = blockIdx.x;
+    seq = unit / heads;
+    if (p.longest_first_sequences > 0) seq = sequence_by_length_rank(p, seq, lane);
+    head = unit % heads;
+  }
   // Metadata values are workgroup-uniform; readfirstlane keeps them (and
   // every buffer descriptor derived from them) in scalar registers.
   const int slot = uniform(p.slots != nullptr ? p.slots[seq] : seq);
@@ -745,7 +749,7 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   if constexpr (kParts) {
     PartRange pr;
     if (segmented) {
-      pr = part_range(p, max(seg_hi - seg_lo, 0), part);
+      pr = part_range(p, max(seg_hi - seg_lo, 0), place.part);
       seg_hi = seg_lo + pr.end;
       seg_lo += pr.begin;
     } else {
@@ -753,7 +757,7 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
       if (len == 0) {
         len = min(p.cu_seqlens[seq + 1], p.total_tokens) - max(p.cu_seqlens[seq], 0);
       }
-      pr = part_range(p, (uniform(max(len, 0)) + kChunk - 1) / kChunk, part);
+      pr = part_range(p, (uniform(max(len, 0)) + kChunk - 1) / kChunk, place.part);
       part_lo = pr.begin * kChunk;
       part_hi = pr.end * kChunk;
     }
@@ -792,24 +796,24 @@ __global__ __launch_bounds__(kChunkThreads, kPrecise ? 1 : 2) void chunk_fwd_ker
   const uint32_t s_off = static_cast<uint32_t>((4 * g) * kHead + 16 * wave + n) * kPoolBytes;
   // A null state means S0 = 0 and no final state (the pretraining layout).
   f32x4 S[4];
-  if constexpr (kParts) {
-    static_assert(sizeof(ChunkSmem) >= kComposeBytes, "the maps fit the chunk tiles");
-    compose_start<256>(&sm, p, unit, part, S);
+  static_assert(sizeof(ChunkSmem) >= kComposeBytes, "the maps fit the chunk tiles");
+  if (kParts && !(place.part == 0 && last_part)) {
+    compose_start<256>(&sm, place, S);
   } else {
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int so = (16 * kb + j) * kHead * kPoolBytes;
-      if (!has_state) {
-        S[kb][j] = 0.0f;
-      } else if constexpr (kPoolBytes == 4) {
-        S[kb][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state_rs, s_off, so, 0));
-      } else {
-        S[kb][j] = to_f32<PoolT>(__builtin_amdgcn_raw_buffer_load_b16(state_rs, s_off, so, 0));
+      for (int j = 0; j < 4; ++j) {
+        const int so = (16 * kb + j) * kHead * kPoolBytes;
+        if (!has_state) {
+          S[kb][j] = 0.0f;
+        } else if constexpr (kPoolBytes == 4) {
+          S[kb][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state_rs, s_off, so, 0));
+        } else {
+          S[kb][j] = to_f32<PoolT>(__builtin_amdgcn_raw_buffer_load_b16(state_rs, s_off, so, 0));
+        }
       }
     }
-  }
   }
 
   // Segment bounds, 64 segments at a time in VGPR lanes (lane i: segment
@@ -1067,7 +1071,7 @@ int launch_chunk(const ChunkFwdParams& p, int units, hipStream_t stream) {
   if (p.parts > 1) {
     const int rc = launch_chunk_transfer<T, M, PoolT, kPrecise>(p, units, stream);
     if (rc != FRWKV_OK) return rc;
-    const dim3 grid(units * p.parts);
+    const dim3 grid(p.part_slots > 0 ? units + p.part_slots * p.num_heads : units * p.parts);
     if (lean) {
       hipLaunchKernelGGL((chunk_fwd_kernel<T, M, PoolT, kPrecise, true, true>), grid,
                          dim3(kChunkThreads), 0, stream, p);
@@ -1155,22 +1159,25 @@ extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_
   if (head_size != 64) return 0;
   const int64_t units = static_cast<int64_t>(num_sequences) * num_heads;
   switch (kernel) {
-    case FRWKV_SPLIT_CHUNK:
-      return part_bytes(units, plan_parts(num_sequences, num_heads, chunks_of(total),
+    case FRWKV_SPLIT_CHUNK:  // of equal sequences (pretraining): states by unit
+      return packed_part_bytes(total, num_sequences, num_heads,
+                               plan_parts(num_sequences, num_heads, chunks_of(total),
                                           chunks_of(longest), kForwardTime, kTransferTime));
     case FRWKV_SPLIT_RECURRENT:
-      return part_bytes(units, plan_parts(num_sequences, num_heads, chunks_of(total),
+      return packed_part_bytes(total, num_sequences, num_heads,
+                               plan_parts(num_sequences, num_heads, chunks_of(total),
                                           chunks_of(longest), kPreciseTime, kTransferTime));
     case FRWKV_SPLIT_CALLER_CHUNKS:
-      return part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total));
+      return unit_part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total));
     case FRWKV_SPLIT_PRETRAIN_BACKWARD:
-      return part_bytes(units, plan_parts(num_sequences, num_heads,
-                                          num_sequences * chunks_of(total / num_sequences),
-                                          chunks_of(total / num_sequences), kBackwardTime,
-                                          kAdjointTime));
+      return unit_part_bytes(units,
+                             plan_parts(num_sequences, num_heads,
+                                        num_sequences * chunks_of(total / num_sequences),
+                                        chunks_of(total / num_sequences), kBackwardTime,
+                                        kAdjointTime));
     case FRWKV_SPLIT_CALLER_CHUNKS_BACKWARD:
-      return part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total,
-                                                  kBackwardTime, kAdjointTime));
+      return unit_part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total,
+                                                       kBackwardTime, kAdjointTime));
     default:
       return 0;
   }
@@ -1237,10 +1244,10 @@ extern "C" int frwkv_chunk_forward_split(
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
   const int units = num_sequences * num_heads;
-  use_parts(p, units,
-            plan_parts(num_sequences, num_heads, chunks_of(total_tokens), chunks_of(max_seqlen),
-                       kForwardTime, kTransferTime),
-            scratch, scratch_bytes);
+  use_packed_parts(p, num_sequences,
+                   plan_parts(num_sequences, num_heads, chunks_of(total_tokens),
+                              chunks_of(max_seqlen), kForwardTime, kTransferTime),
+                   scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (pool_dtype == FRWKV_DTYPE_F32) return dispatch_chunk_io<float>(p, io_dtype, decay_mode, units, s);
   if (pool_dtype == FRWKV_DTYPE_BF16) return dispatch_chunk_io<Bf16>(p, io_dtype, decay_mode, units, s);
@@ -1347,8 +1354,9 @@ extern "C" int frwkv_statetune_forward_split(
   p.interior = interior;
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
-  use_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
-            plan_caller_chunks(num_sequences, num_heads, num_chunks), scratch, scratch_bytes);
+  use_unit_parts(p, static_cast<int64_t>(num_sequences) * num_heads,
+                 plan_caller_chunks(num_sequences, num_heads, num_chunks), scratch,
+                 scratch_bytes);
   return dispatch_chunk_io<float>(p, io_dtype, decay_mode, num_sequences * num_heads,
                                   static_cast<hipStream_t>(stream));
 }
@@ -1492,10 +1500,10 @@ extern "C" int frwkv_pretrain_forward_split(
   p.state_dot_a = state_dot_a;
   p.scale = 1.0f;
   p.out_elems = static_cast<int64_t>(batch) * tokens * num_heads * head_size;
-  use_parts(p, static_cast<int64_t>(batch) * num_heads,
-            plan_parts(batch, num_heads, chunks_of(p.total_tokens), chunks_of(tokens),
-                       kForwardTime, kTransferTime),
-            scratch, scratch_bytes);
+  use_unit_parts(p, static_cast<int64_t>(batch) * num_heads,
+                 plan_parts(batch, num_heads, chunks_of(p.total_tokens), chunks_of(tokens),
+                            kForwardTime, kTransferTime),
+                 scratch, scratch_bytes);
   return dispatch_chunk_io<float>(p, io_dtype, decay_mode, batch * num_heads,
                                   static_cast<hipStream_t>(stream));
 }
@@ -1584,10 +1592,10 @@ int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32
   p.scale = scale;
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * kHead;
   const int units = num_sequences * num_heads;
-  use_parts(p, units,
-            plan_parts(num_sequences, num_heads, chunks_of(total_tokens), chunks_of(max_seqlen),
-                       kPreciseTime, kTransferTime),
-            scratch, scratch_bytes);
+  use_packed_parts(p, num_sequences,
+                   plan_parts(num_sequences, num_heads, chunks_of(total_tokens),
+                              chunks_of(max_seqlen), kPreciseTime, kTransferTime),
+                   scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (decay_mode == FRWKV_DECAY_LOGITS) {
     return launch_chunk<Bf16, DecayMode::kLogits, float, true>(p, units, s);

@@ -15,7 +15,7 @@
 //      state from the first part's end state and the maps of parts
 //      1 .. j - 1 in fp32 (compose_start), then walks its chunks.
 // The work is about twice that of the unsplit kernel, over `parts` times the
-// workgroups.
+// workgroups. A sequence of one part takes no transfer and no part states.
 //
 // The backward's state adjoint is affine in the adjoint behind it, so it is
 // split the same way from the end: part 0 is a sequence's last run of chunks,
@@ -82,6 +82,9 @@ struct ChunkFwdParams {
   int32_t parts;
   int32_t part_len;
   float* part_states;
+  // Packed sequences: their number, and the slots of a head (0: states by unit).
+  int32_t packed_sequences;
+  int32_t part_slots;
 };
 
 struct ChunkBwdParams {
@@ -124,14 +127,80 @@ constexpr int kMaxParts = 16;
 
 constexpr int kStateElems = kHead * kHead;
 
-// States of part `part` of unit (sequence, head) `unit`: [M][N], 64 x 64 fp32
-// each, row-major over keys. Part 0 keeps the sequence's start state in place
-// of M (the pool is overwritten by the last part while the first one still
-// needs it) and its end state in place of N. The last part has none.
-template <typename P>
-__device__ __forceinline__ float* part_state(const P& p, int unit, int part, int which) {
-  return p.part_states +
-         ((static_cast<int64_t>(unit) * (p.parts - 1) + part) * 2 + which) * kStateElems;
+// Where a part's workgroup is: its (sequence, head), its part, and the states
+// of the unit's parts. A part's states are [M][N], 64 x 64 fp32 each, row-major
+// over keys. Part 0 keeps the sequence's start state in place of M (the pool is
+// overwritten by the last part while the first one still needs it) and its end
+// state in place of N. The last part has none.
+struct PartPlace {
+  int seq, head, part;
+  float* states;
+  int64_t step;  // from one part's states to the next
+  __device__ __forceinline__ float* state(int i, int which) const {
+    return states + i * step + which * kStateElems;
+  }
+};
+
+// Packed sequences: sequence s has its states at slots part_slot(s) .. of each
+// head. It needs at most ceil(chunks / len) - 1 = floor((tokens - 1) / (64 len))
+// of them, so the slots of disjoint, ascending sequences are disjoint and below
+// floor(total_tokens / (64 len)), and short sequences have none.
+__device__ __forceinline__ int part_slot(const ChunkFwdParams& p, int seq) {
+  return max(p.cu_seqlens[seq], 0) / (kChunk * p.part_len);
+}
+// The sequence that owns a slot (or the last one that starts at or before it).
+// Every lane tries one of 64 equal steps, so 64 sequences take one round.
+__device__ __forceinline__ int sequence_of_part_slot(const ChunkFwdParams& p, int slot,
+                                                     int lane) {
+  int lo = 0, hi = p.packed_sequences;
+  while (hi - lo > 1) {
+    const int stride = (hi - lo + 63) / 64;
+    const int s = lo + lane * stride;
+    const bool before = s < hi && part_slot(p, s) <= slot;
+    const int count = max(__builtin_popcountll(__builtin_amdgcn_ballot_w64(before)), 1);
+    lo = uniform(lo + (count - 1) * stride);
+    hi = min(lo + stride, hi);
+  }
+  return lo;
+}
+// Blocks (slot, head): the parts with a successor (kTransfer) or, in the main
+// launch, those with a predecessor, followed by every sequence's first part.
+template <bool kTransfer>
+__device__ __forceinline__ PartPlace packed_place(const ChunkFwdParams& p, int lane) {
+  PartPlace at;
+  const int blocks = p.part_slots * p.num_heads;
+  const int block = static_cast<int>(blockIdx.x);
+  int first;
+  if (kTransfer || block < blocks) {
+    const int slot = block / p.num_heads;
+    at.head = block % p.num_heads;
+    at.seq = sequence_of_part_slot(p, slot, lane);
+    first = uniform(part_slot(p, at.seq));
+    at.part = slot - first + (kTransfer ? 0 : 1);
+  } else {
+    at.seq = (block - blocks) / p.num_heads;
+    at.head = (block - blocks) % p.num_heads;
+    at.part = 0;
+    first = uniform(part_slot(p, at.seq));
+  }
+  at.step = static_cast<int64_t>(p.num_heads) * 2 * kStateElems;
+  at.states = p.part_states + first * at.step + at.head * 2 * kStateElems;
+  return at;
+}
+// Dense sequences and caller chunks: block part * units + unit, so that (for a
+// unit count divisible by the 8 XCDs) a unit's parts share an XCD, and its L2,
+// in both launches.
+template <bool kTransfer, typename P>
+__device__ __forceinline__ PartPlace unit_place(const P& p) {
+  PartPlace at;
+  const uint32_t units = gridDim.x / (kTransfer ? p.parts - 1 : p.parts);
+  const uint32_t unit = blockIdx.x % units;
+  at.part = blockIdx.x / units;
+  at.seq = unit / p.num_heads;
+  at.head = unit % p.num_heads;
+  at.step = 2 * kStateElems;
+  at.states = p.part_states + static_cast<int64_t>(unit) * (p.parts - 1) * at.step;
+  return at;
 }
 
 // Part `part` of a sequence's `count` items (64-token chunks, or caller
@@ -163,9 +232,10 @@ __device__ __forceinline__ PartRange part_range(const P& p, int count, int part)
 // as fp32 MFMA operands took 3.2 us per step; this takes 1.1.)
 constexpr int kComposeMaps = 4;
 constexpr size_t kComposeBytes = kComposeMaps * 2 * kOpTile * sizeof(uint16_t);
-template <int kThreads, typename P>
-__device__ __forceinline__ void compose_start(void* space, const P& p, int unit, int part,
+template <int kThreads>
+__device__ __forceinline__ void compose_start(void* space, const PartPlace& where,
                                               f32x4 (&S)[4]) {
+  const int part = where.part;
   constexpr int kShare = kStateElems / kThreads;  // a thread's elements of a map
   constexpr int kPerRow = kHead / kShare;
   const int tid = threadIdx.x;
@@ -175,7 +245,7 @@ __device__ __forceinline__ void compose_start(void* space, const P& p, int unit,
   uint16_t* const tiles = static_cast<uint16_t*>(space);  // [map][hi, lo][row][col]
   const int col = (4 * g) * kHead + 16 * w + n;
   auto load_slab = [&](int i, int which, f32x4 (&x)[4]) {
-    const float* src = part_state(p, unit, i, which) + col;
+    const float* src = where.state(i, which) + col;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -191,7 +261,7 @@ __device__ __forceinline__ void compose_start(void* space, const P& p, int unit,
 #pragma unroll
     for (int u = 0; u < kComposeMaps; ++u) {
       if (first + u < part) {
-        const float* src = part_state(p, unit, first + u, 0) + share;
+        const float* src = where.state(first + u, 0) + share;
 #pragma unroll
         for (int c = 0; c < kShare / 4; ++c) m[u][c] = *reinterpret_cast<const f32x4*>(src + 4 * c);
       }
@@ -313,22 +383,51 @@ inline PartPlan plan_parts(int64_t sequences, int64_t heads, int64_t chunks, int
   return best;
 }
 
-// Bytes of part states of a split call (0 when it does not split).
-inline size_t part_bytes(int64_t units, const PartPlan& plan) {
-  return plan.parts > 1 ? static_cast<size_t>(units) * (plan.parts - 1) * 2 * kStateElems *
-                              sizeof(float)
-                        : 0;
+// Bytes of part states of a split call (0 when it does not split): parts - 1 per
+// unit for equal sequences, caller chunks (planned by their mean) and packed
+// sequences of similar lengths, else as many as the packed tokens can need (see
+// part_slot). Either way it is proportional to the call's tokens, whatever the
+// sequences' lengths. Three sequences of 817 to 1654 tokens take 109.5 us by
+// units and 111.9 by slots (the search for a slot's sequence); 63 single tokens
+// and a prompt of 2048 173.6 by units (most workgroups without a part) and 94.1.
+inline size_t part_bytes(int64_t states) {
+  return static_cast<size_t>(states) * 2 * kStateElems * sizeof(float);
+}
+inline size_t unit_part_bytes(int64_t units, const PartPlan& plan) {
+  return part_bytes(units * (plan.parts - 1));
+}
+// Slots per head of packed sequences, or 0 for states by unit.
+inline int64_t packed_part_slots(int64_t tokens, int64_t sequences, const PartPlan& plan) {
+  const int64_t slots = plan.parts > 1 ? tokens / (kChunk * plan.len) : 0;
+  return sequences * (plan.parts - 1) <= 2 * slots ? 0 : slots;
+}
+inline size_t packed_part_bytes(int64_t tokens, int64_t sequences, int64_t heads,
+                                const PartPlan& plan) {
+  const int64_t slots = packed_part_slots(tokens, sequences, plan);
+  return slots > 0 ? part_bytes(slots * heads) : unit_part_bytes(sequences * heads, plan);
 }
 
-// Splits the call when the caller's scratch holds its part states.
+// Splits the call when the caller's scratch holds its `bytes` of part states.
 template <typename P>
-inline void use_parts(P& p, int64_t units, const PartPlan& plan, void* scratch,
+inline void use_parts(P& p, const PartPlan& plan, size_t bytes, void* scratch,
                       size_t scratch_bytes) {
-  const bool split = plan.parts > 1 && scratch != nullptr &&
-                     scratch_bytes >= part_bytes(units, plan);
+  const bool split = bytes > 0 && scratch != nullptr && scratch_bytes >= bytes;
   p.parts = split ? plan.parts : 1;
   p.part_len = split ? plan.len : 0;
   p.part_states = split ? static_cast<float*>(scratch) : nullptr;
+}
+inline void use_packed_parts(ChunkFwdParams& p, int32_t sequences, const PartPlan& plan,
+                             void* scratch, size_t scratch_bytes) {
+  use_parts(p, plan, packed_part_bytes(p.total_tokens, sequences, p.num_heads, plan), scratch,
+            scratch_bytes);
+  p.packed_sequences = sequences;
+  p.part_slots =
+      p.parts > 1 ? static_cast<int32_t>(packed_part_slots(p.total_tokens, sequences, plan)) : 0;
+}
+template <typename P>
+inline void use_unit_parts(P& p, int64_t units, const PartPlan& plan, void* scratch,
+                           size_t scratch_bytes) {
+  use_parts(p, plan, unit_part_bytes(units, plan), scratch, scratch_bytes);
 }
 
 inline int64_t chunks_of(int64_t tokens) {

@@ -324,11 +324,9 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
   const int cs = wave & 3;        // column slab
   const bool map = wave >= 4;     // M's slab (else N's)
   const int heads = p.num_heads;
-  const int units = static_cast<int>(gridDim.x) / (p.parts - 1);
-  const int part = static_cast<int>(blockIdx.x) / units;
-  const int unit = static_cast<int>(blockIdx.x) % units;
-  const int seq = unit / heads;
-  const int head = unit % heads;
+  const PartPlace place =
+      p.part_slots > 0 ? packed_place<true>(p, lane) : unit_place<true>(p);
+  const int part = place.part, seq = place.seq, head = place.head;
   const int slot = uniform(p.slots != nullptr ? p.slots[seq] : seq);
   if (slot < 0 || slot >= p.state_slots) return;
 
@@ -360,7 +358,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
     c_end = min(begin + r.end * kChunk, end);
     last = r.last;
   }
-  if (last && part > 0) return;  // no part follows
+  if (last) return;  // no part follows
   auto next_segment = [&]() {    // the segment's tokens into [c0, c_end)
     if (p.seg_offsets == nullptr) return;
     c0 = uniform(max(p.seg_starts[seg], 0));
@@ -417,8 +415,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
     rows.v = load(p.v, first, ntok);
   };
 
-  // A part that is its sequence's first and last only keeps the start state.
-  bool more = !(part == 0 && last) && seg < seg_hi;
+  bool more = seg < seg_hi;
   if (more) next_segment();
   while (more && c0 >= c_end) {  // empty segments
     more = ++seg < seg_hi;
@@ -465,7 +462,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
     if (!whole && more) load_rows(rows, c0, min(kChunk, c_end - c0));
   }
 
-  float* dst = part_state(p, unit, part, map ? 0 : 1) + s_off;
+  float* dst = place.state(part, map ? 0 : 1) + s_off;
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -565,11 +562,8 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
   const int cs = wave & 3;
   const bool map = wave >= 4;
   const int heads = p.num_heads;
-  const int units = static_cast<int>(gridDim.x) / (p.parts - 1);
-  const int part = static_cast<int>(blockIdx.x) / units;
-  const int unit = static_cast<int>(blockIdx.x) % units;
-  const int seq = unit / heads;
-  const int head = unit % heads;
+  const PartPlace place = unit_place<true>(p);
+  const int part = place.part, seq = place.seq, head = place.head;
 
   // The part's segments, or its run of chunks of the dense sequence; chunks
   // start at c_begin + 64 j.
@@ -592,7 +586,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
     seg = r.end > r.begin ? 1 : 0;
     last = r.last;
   }
-  if (last && part > 0) return;  // no part follows
+  if (last) return;  // no part follows
 
   f32x4 S[4];
   const uint32_t s_off = static_cast<uint32_t>((4 * g) * kHead + 16 * cs + n);
@@ -653,8 +647,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
     c0 = c_begin + (c_end - c_begin - 1) / kChunk * kChunk;
     return true;
   };
-  // A part that is its sequence's first and last only keeps the end adjoint.
-  bool more = !(part == 0 && last) && seg > seg_lo && previous();
+  bool more = seg > seg_lo && previous();
   TransferRows rows;
   if (more) load_rows(rows, c0, c_end - c0);
   while (more) {
@@ -690,7 +683,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
     if (!whole && more) load_rows(rows, c0, c_end - c0);
   }
 
-  float* dst = part_state(p, unit, part, map ? 0 : 1) + s_off;
+  float* dst = place.state(part, map ? 0 : 1) + s_off;
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
 #pragma unroll
@@ -703,7 +696,8 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
 template <typename T, DecayMode M, typename PoolT, bool kPrecise>
 int launch_chunk_transfer(const ChunkFwdParams& p, int units, hipStream_t stream) {
   hipLaunchKernelGGL((chunk_transfer_kernel<T, M, PoolT, kPrecise>),
-                     dim3(units * (p.parts - 1)), dim3(kTransferThreads), 0, stream, p);
+                     dim3(p.part_slots > 0 ? p.part_slots * p.num_heads : units * (p.parts - 1)),
+                     dim3(kTransferThreads), 0, stream, p);
   return check_launch("chunk_transfer_kernel");
 }
 

@@ -244,3 +244,19 @@ def test_backward_without_interior_or_workspace_is_refused_without_a_gpu():
                                       *tensors[2:], *grads, null, 0, 1.0, None)
     assert rc == 1
     assert b"workspace of 0 bytes given" in lib.frwkv_last_error()
+
+
+# Scratch of a split call follows the tokens, whatever the sequences' lengths: at
+# most 64 KiB per head and 64 tokens (one part per chunk), and a batch of single
+# tokens beside one long prompt needs about what the prompt alone does.
+@pytest.mark.parametrize("kernel", (0, 1), ids=("chunk", "recurrent"))
+@pytest.mark.parametrize("singles", (0, 61, 127, 1000))
+@pytest.mark.parametrize("longest", (512, 8192, 65536))
+def test_split_scratch_follows_the_tokens_without_a_gpu(kernel, singles, longest):
+    from flashrwkv_amd import capi
+
+    heads, bf16 = 40, capi.DTYPE[torch.bfloat16]
+    size = capi.library().frwkv_split_scratch_bytes(kernel, bf16, capi.DECAY_LOGITS, singles + 1,
+                                                    heads, 64, singles + longest, longest)
+    assert size <= (singles + longest) // 64 * heads * 65536
+    assert size <= 2 * 16 * heads * 32768  # at most 16 parts of the prompt

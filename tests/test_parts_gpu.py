@@ -73,6 +73,10 @@ def _case(lengths, dtype, u_low=-5.0, heads=3):
     ((640, 70), torch.bfloat16, torch.float32, 3.0),
     ((640, 70), torch.bfloat16, torch.float32, MIXED),
     ((640, 70), torch.float16, torch.float32, MIXED),
+    # Short sequences before, between and after long ones, more than one round
+    # of the search for a part's sequence.
+    ((1,) * 70 + (700,) + (2,) * 5 + (1400, 63), torch.bfloat16, torch.float32, -5.0),
+    ((1900, 65) + (1,) * 140, torch.bfloat16, torch.bfloat16, -5.0),
 ])
 @pytest.mark.parametrize("kernel", (CHUNK, RECURRENT))
 def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
