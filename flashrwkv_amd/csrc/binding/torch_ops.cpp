@@ -275,14 +275,19 @@ Tensor workspace_like(const Tensor& like, size_t bytes) {
 }
 
 // Scratch of a split call (undefined when the call does not split); total and
-// longest as for frwkv_split_scratch_bytes.
+// longest as for frwkv_split_scratch_bytes. It only makes the call faster, so
+// where the device has no room for it the call runs without.
 Tensor split_scratch(int kernel, int decay_mode, int64_t sequences, int64_t heads,
                      int64_t head_size, int64_t total, int64_t longest, const Tensor& like) {
-  return workspace_like(like, frwkv_split_scratch_bytes(
-                                  kernel, io_code(like.scalar_type()), decay_mode,
-                                  static_cast<int32_t>(sequences),
-                                  static_cast<int32_t>(heads), static_cast<int32_t>(head_size),
-                                  static_cast<int32_t>(total), static_cast<int32_t>(longest)));
+  const size_t bytes = frwkv_split_scratch_bytes(
+      kernel, io_code(like.scalar_type()), decay_mode, static_cast<int32_t>(sequences),
+      static_cast<int32_t>(heads), static_cast<int32_t>(head_size), static_cast<int32_t>(total),
+      static_cast<int32_t>(longest));
+  try {
+    return workspace_like(like, bytes);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
 }
 void* scratch_ptr(const Tensor& scratch) {
   return scratch.defined() ? scratch.data_ptr() : nullptr;

@@ -162,6 +162,40 @@ def test_fp32_matrix_recurrence(dtype, d, lengths):
     parity.check("state", dev["state_pool"], pool_ref, 1e-5)
 
 
+# Without room for the scratch a call runs as one without scratch does.
+def test_no_room_for_scratch():
+    n, heads = 4096, 32
+    case = workloads.make_case(lengths=(n,), heads=heads, head_size=64, dtype=torch.float16,
+                               seed=7, state_std=0.1)
+    dev = {k: v.to(DEV) if isinstance(v, torch.Tensor) else v for k, v in case.items()}
+
+    def run():
+        pool = dev["state_pool"].clone()
+        y = flashrwkv_amd.infer_recurrent_fp32io16_forward_varlen(
+            *(dev[x] for x in NAMES), state_pool=pool, cu_seqlens=dev["cu_seqlens"],
+            state_indices=dev["state_indices"])
+        torch.cuda.synchronize()
+        return y, pool
+
+    before = flashrwkv_amd.tmix.wkv7.set_recurrent_long_route("per_token")
+    try:
+        want = run()
+    finally:
+        flashrwkv_amd.tmix.wkv7.set_recurrent_long_route(before)
+    size = capi.library().frwkv_split_scratch_bytes(RECURRENT, capi.DTYPE[torch.float16],
+                                                    capi.DECAY_LOGITS, 1, heads, 64, n, n)
+    assert size > 128 << 20
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + size // 2) / total)
+    try:
+        got = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+
+
 # Head size 256 training: caller chunks of one piece, of a piece and a token,
 # longer ones and an empty one, and no upstream gradient of y or of the state.
 @pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
