@@ -1137,7 +1137,8 @@ extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_
   using namespace frwkv;
   if (num_sequences <= 0 || num_heads <= 0 || total <= 0) return 0;
   if (kernel == FRWKV_SPLIT_RECURRENT &&
-      piece32_recurrent(io_dtype, decay_mode, head_size, longest)) {
+      piece32_recurrent(io_dtype, decay_mode, head_size, num_sequences, num_heads, total,
+                        longest)) {
     const size_t bytes = piece32_forward_bytes(head_size, num_heads, total, num_sequences);
     return bytes <= kPiece32RecurrentBytes ? bytes : 0;
   }

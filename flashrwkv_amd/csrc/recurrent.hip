@@ -1053,7 +1053,9 @@ extern "C" int frwkv_recurrent_forward_split(
                                            scratch_bytes, stream);
   }
   // Other long 16-bit calls take the fp32 matrix form, given its scratch.
-  if (scratch != nullptr && piece32_recurrent(io_dtype, decay_mode, head_size, max_seqlen) &&
+  if (scratch != nullptr &&
+      piece32_recurrent(io_dtype, decay_mode, head_size, num_sequences, num_heads, total_tokens,
+                        max_seqlen) &&
       scratch_bytes >= piece32_forward_bytes(head_size, num_heads, total_tokens, num_sequences)) {
     Piece32Params q{};
     q.num_heads = num_heads;

@@ -139,8 +139,9 @@ int frwkv_recurrent_forward(int io_dtype, int decay_mode, int32_t num_sequences,
  * same for frwkv_pretrain_backward_split and frwkv_statetune_backward_split.
  * With decay logits, scratch also opens the fp32 matrix form over 16-token
  * pieces where the unsplit call runs the per-token kernel: the recurrent entry
- * with fp16 tokens, or at head sizes 128 and 256, on sequences of at least 32
- * tokens, and training at head size 256. Same fp32 arithmetic, other order of
+ * with fp16 tokens, or at head sizes 128 and 256, where the longest sequence has
+ * at least 32 tokens and the batch is not mostly single tokens, and training at
+ * head size 256. Same fp32 arithmetic, other order of
  * sums. No counterpart in the reference.
  */
 enum {

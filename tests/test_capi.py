@@ -260,3 +260,33 @@ def test_split_scratch_follows_the_tokens_without_a_gpu(kernel, singles, longest
                                                     heads, 64, singles + longest, longest)
     assert size <= (singles + longest) // 64 * heads * 65536
     assert size <= 2 * 16 * heads * 32768  # at most 16 parts of the prompt
+
+
+# The fp32 matrix form's route of the recurrent entry (it has scratch): batches of
+# prompts take it, decoding batches that admit a short prompt keep the per-token
+# kernel. The faster side of every case is measured (piece32.h).
+@pytest.mark.parametrize("head_size,heads,singles,longest,pieces", [
+    (64, 32, 0, 31, False), (64, 32, 0, 32, True), (64, 32, 63, 32, False),
+    (64, 32, 63, 128, True), (64, 32, 255, 32, False), (64, 32, 255, 128, False),
+    (64, 32, 255, 512, True), (128, 16, 63, 32, False), (128, 16, 63, 128, True),
+    (256, 8, 63, 32, False), (256, 8, 63, 512, True),
+])
+def test_fp32_matrix_route_of_mixed_batches_without_a_gpu(head_size, heads, singles, longest,
+                                                          pieces):
+    from flashrwkv_amd import capi
+
+    size = capi.library().frwkv_split_scratch_bytes(
+        1, capi.DTYPE[torch.float16], capi.DECAY_LOGITS, singles + 1, heads, head_size,
+        singles + longest, longest)
+    assert (size > 0) == pieces
+
+
+@pytest.mark.parametrize("head_size,heads", [(64, 32), (128, 16), (256, 8)])
+@pytest.mark.parametrize("sequences", (1, 9, 64))
+@pytest.mark.parametrize("tokens", (32, 64))
+def test_fp32_matrix_route_of_prompts_without_a_gpu(head_size, heads, sequences, tokens):
+    from flashrwkv_amd import capi
+
+    assert capi.library().frwkv_split_scratch_bytes(
+        1, capi.DTYPE[torch.float16], capi.DECAY_LOGITS, sequences, heads, head_size,
+        sequences * tokens, tokens) > 0
