@@ -1068,6 +1068,12 @@ int launch_chunk(const ChunkFwdParams& p, int units, hipStream_t stream) {
                     p.boundary == nullptr && p.state_dot_a == nullptr &&
                     p.interior == nullptr && !p.fill_only && !p.boundary16 &&
                     !p.read_only_state && p.state != nullptr;
+  if constexpr (kPrecise || !__is_same(PoolT, float)) {
+    if (!lean) {
+      return set_error(FRWKV_ERR_UNSUPPORTED,
+                       "split precision and bf16 pools run packed calls with a state only");
+    }
+  }
   if (p.parts > 1) {
     const int rc = launch_chunk_transfer<T, M, PoolT, kPrecise>(p, units, stream);
     if (rc != FRWKV_OK) return rc;
