@@ -1148,6 +1148,7 @@ extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_
     const size_t bytes = piece32_forward_bytes(head_size, num_heads, total, num_sequences);
     return bytes <= kPiece32RecurrentBytes ? bytes : 0;
   }
+  if (kernel == FRWKV_SPLIT_RECURRENT && io_dtype != FRWKV_DTYPE_BF16) return 0;
   if (head_size == 256 && decay_mode == FRWKV_DECAY_LOGITS && kernel == FRWKV_SPLIT_CHUNK) {
     return piece32_forward_bytes(head_size, num_heads, total, num_sequences);
   }

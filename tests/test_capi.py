@@ -281,6 +281,19 @@ def test_fp32_matrix_route_of_mixed_batches_without_a_gpu(head_size, heads, sing
     assert (size > 0) == pieces
 
 
+# Calls that run on the per-token kernel take no scratch: fp32 tokens, raw
+# retentions of fp16 tokens, and fp16 batches too large for the matrix form.
+@pytest.mark.parametrize("dtype,decay,tokens", [
+    (torch.float32, "DECAY_LOGITS", 4096), (torch.float16, "DECAY_RAW_W", 4096),
+    (torch.float16, "DECAY_LOGITS", 100000),
+])
+def test_per_token_calls_have_no_scratch_without_a_gpu(dtype, decay, tokens):
+    from flashrwkv_amd import capi
+
+    assert capi.library().frwkv_split_scratch_bytes(
+        1, capi.DTYPE[dtype], getattr(capi, decay), 1, 32, 64, tokens, tokens) == 0
+
+
 @pytest.mark.parametrize("head_size,heads", [(64, 32), (128, 16), (256, 8)])
 @pytest.mark.parametrize("sequences", (1, 9, 64))
 @pytest.mark.parametrize("tokens", (32, 64))
