@@ -126,18 +126,23 @@ constexpr int kMinParts = 3;
 constexpr int kMaxParts = 16;
 
 constexpr int kStateElems = kHead * kHead;
+// A part's states are [M][N], 64 x 64 each, row-major over keys: M as three bf16
+// planes, M = hi + mid + lo exactly (split3_bf16x2), as compose_start multiplies
+// it (every later part reads it, so it is split once here), N in fp32. Sizes in
+// floats.
+constexpr int kMapElems = 3 * kStateElems / 2;
+constexpr int kPartElems = kMapElems + kStateElems;
 
 // Where a part's workgroup is: its (sequence, head), its part, and the states
-// of the unit's parts. A part's states are [M][N], 64 x 64 fp32 each, row-major
-// over keys. Part 0 keeps the sequence's start state in place of M (the pool is
-// overwritten by the last part while the first one still needs it) and its end
-// state in place of N. The last part has none.
+// of the unit's parts. Part 0 keeps the sequence's start state in place of M
+// (the pool is overwritten by the last part while the first one still needs it)
+// and its end state in place of N, both fp32. The last part has none.
 struct PartPlace {
   int seq, head, part;
   float* states;
   int64_t step;  // from one part's states to the next
   __device__ __forceinline__ float* state(int i, int which) const {
-    return states + i * step + which * kStateElems;
+    return states + i * step + which * kMapElems;
   }
 };
 
@@ -183,8 +188,8 @@ __device__ __forceinline__ PartPlace packed_place(const ChunkFwdParams& p, int l
     at.part = 0;
     first = uniform(part_slot(p, at.seq));
   }
-  at.step = static_cast<int64_t>(p.num_heads) * 2 * kStateElems;
-  at.states = p.part_states + first * at.step + at.head * 2 * kStateElems;
+  at.step = static_cast<int64_t>(p.num_heads) * kPartElems;
+  at.states = p.part_states + first * at.step + at.head * kPartElems;
   return at;
 }
 // Dense sequences and caller chunks: block part * units + unit, so that (for a
@@ -198,7 +203,7 @@ __device__ __forceinline__ PartPlace unit_place(const P& p) {
   at.part = blockIdx.x / units;
   at.seq = unit / p.num_heads;
   at.head = unit % p.num_heads;
-  at.step = 2 * kStateElems;
+  at.step = kPartElems;
   at.states = p.part_states + static_cast<int64_t>(unit) * (p.parts - 1) * at.step;
   return at;
 }
@@ -225,13 +230,13 @@ __device__ __forceinline__ PartRange part_range(const P& p, int count, int part)
 // layout (S[kb][j]: row 16kb + 4g + j, column 16w + n): part 0 takes the kept
 // start state, part j the first part's end state through the maps of parts
 // 1 .. j - 1, S <- M_i S + N_i. All waves need all of each map, so maps go
-// through LDS (tiles: kComposeBytes, not yet in use), four at a time, split
-// into bf16 hi + lo there: M S is the three products hi hi + hi lo + lo hi,
-// about 2^-16 relative error per step, on an fp32 state. The next four maps
-// are loaded while these are applied. (Every wave reading the maps from memory
-// as fp32 MFMA operands took 3.2 us per step; this takes 1.1.)
-constexpr int kComposeMaps = 4;
-constexpr size_t kComposeBytes = kComposeMaps * 2 * kOpTile * sizeof(uint16_t);
+// through LDS (tiles: kComposeBytes, not yet in use), two at a time, and the
+// state is split into three bf16 as they are: M S is the six products of at
+// least 2^-16 times the whole, so the state is carried at fp32's precision, as
+// it is from chunk to chunk. The next two maps are loaded while these are
+// applied.
+constexpr int kComposeMaps = 2;
+constexpr size_t kComposeBytes = kComposeMaps * 3 * kOpTile * sizeof(uint16_t);
 template <int kThreads>
 __device__ __forceinline__ void compose_start(void* space, const PartPlace& where,
                                               f32x4 (&S)[4]) {
@@ -242,7 +247,7 @@ __device__ __forceinline__ void compose_start(void* space, const PartPlace& wher
   const int w = uniform(tid >> 6) & 3;
   const int lane = tid & 63;
   const int g = lane >> 4, n = lane & 15;
-  uint16_t* const tiles = static_cast<uint16_t*>(space);  // [map][hi, lo][row][col]
+  uint16_t* const tiles = static_cast<uint16_t*>(space);  // [map][hi, mid, lo][row][col]
   const int col = (4 * g) * kHead + 16 * w + n;
   auto load_slab = [&](int i, int which, f32x4 (&x)[4]) {
     const float* src = where.state(i, which) + col;
@@ -256,14 +261,21 @@ __device__ __forceinline__ void compose_start(void* space, const PartPlace& wher
   if (part < 2) return;
   const int share = kShare * tid;
   const int place = (tid / kPerRow) * kOpStride + kShare * (tid % kPerRow);
-  f32x4 m[kComposeMaps][kShare / 4], off[kComposeMaps][4];
+  uint4 m[kComposeMaps][3][kShare / 8];
+  f32x4 off[kComposeMaps][4];
   auto load_maps = [&](int first) {
 #pragma unroll
     for (int u = 0; u < kComposeMaps; ++u) {
       if (first + u < part) {
-        const float* src = where.state(first + u, 0) + share;
+        const uint16_t* src =
+            reinterpret_cast<const uint16_t*>(where.state(first + u, 0)) + share;
 #pragma unroll
-        for (int c = 0; c < kShare / 4; ++c) m[u][c] = *reinterpret_cast<const f32x4*>(src + 4 * c);
+        for (int x = 0; x < 3; ++x) {
+#pragma unroll
+          for (int c = 0; c < kShare / 8; ++c) {
+            m[u][x][c] = *reinterpret_cast<const uint4*>(src + x * kStateElems + 8 * c);
+          }
+        }
       }
     }
   };
@@ -277,12 +289,16 @@ __device__ __forceinline__ void compose_start(void* space, const PartPlace& wher
 #pragma unroll
     for (int u = 0; u < kComposeMaps; ++u) {
       if (first + u < part) {
-        uint16_t* hi = tiles + 2 * u * kOpTile + place;
+        uint16_t* dst = tiles + 3 * u * kOpTile + place;
 #pragma unroll
-        for (int c = 0; c < kShare / 4; c += 2) {
-          const float x[8] = {m[u][c][0],     m[u][c][1],     m[u][c][2],     m[u][c][3],
-                              m[u][c + 1][0], m[u][c + 1][1], m[u][c + 1][2], m[u][c + 1][3]};
-          store8_bf16_split(hi + 4 * c, hi + kOpTile + 4 * c, x);
+        for (int x = 0; x < 3; ++x) {
+#pragma unroll
+          for (int c = 0; c < kShare / 8; ++c) {
+            const uint4 q = m[u][x][c];
+            uint2* to = reinterpret_cast<uint2*>(dst + x * kOpTile + 8 * c);
+            to[0] = make_uint2(q.x, q.y);
+            to[1] = make_uint2(q.z, q.w);
+          }
         }
       }
     }
@@ -291,23 +307,29 @@ __device__ __forceinline__ void compose_start(void* space, const PartPlace& wher
 #pragma unroll
     for (int u = 0; u < kComposeMaps; ++u) {
       if (first + u < part) {
-        const uint16_t* hi = tiles + 2 * u * kOpTile;
-        const uint16_t* lo = hi + kOpTile;
-        i16x4 sh[4], sl[4];
+        const uint16_t* map = tiles + 3 * u * kOpTile;
+        i16x4 s[3][4];
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) to_operand_split(S[kb], sh[kb], sl[kb]);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) S[kb] = off[u][kb];
+        for (int kb = 0; kb < 4; ++kb) {
+          to_operand_split3(S[kb], s[0][kb], s[1][kb], s[2][kb]);
+          S[kb] = off[u][kb];
+        }
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-          const i16x8 bh = cat(sh[2 * kk], sh[2 * kk + 1]);
-          const i16x8 bl = cat(sl[2 * kk], sl[2 * kk + 1]);
+          const i16x8 bh = cat(s[0][2 * kk], s[0][2 * kk + 1]);
+          const i16x8 bm = cat(s[1][2 * kk], s[1][2 * kk + 1]);
+          const i16x8 bl = cat(s[2][2 * kk], s[2][2 * kk + 1]);
 #pragma unroll
           for (int rb = 0; rb < 4; ++rb) {
-            const i16x8 ah = lds_operand32<kOpStride>(hi, 16 * rb + n, 32 * kk, g);
-            const i16x8 al = lds_operand32<kOpStride>(lo, 16 * rb + n, 32 * kk, g);
+            const int row = 16 * rb + n;
+            const i16x8 ah = lds_operand32<kOpStride>(map, row, 32 * kk, g);
+            const i16x8 am = lds_operand32<kOpStride>(map + kOpTile, row, 32 * kk, g);
+            const i16x8 al = lds_operand32<kOpStride>(map + 2 * kOpTile, row, 32 * kk, g);
             S[rb] = mfma32(al, bh, S[rb]);
             S[rb] = mfma32(ah, bl, S[rb]);
+            S[rb] = mfma32(am, bm, S[rb]);
+            S[rb] = mfma32(am, bh, S[rb]);
+            S[rb] = mfma32(ah, bm, S[rb]);
             S[rb] = mfma32(ah, bh, S[rb]);
           }
         }
@@ -315,6 +337,36 @@ __device__ __forceinline__ void compose_start(void* space, const PartPlace& wher
     }
   }
   __syncthreads();  // before the chunk tiles are written
+}
+
+// Stores a wave's columns of a map or an offset (C layout, element (4g, column)
+// at `offset` of it): a map of parts 1 .. as planes, all else as fp32.
+__device__ __forceinline__ void store_part_state(const PartPlace& where, int part, bool map,
+                                                 uint32_t offset, const f32x4 (&S)[4]) {
+  float* dst = where.state(part, map ? 0 : 1);
+  if (!map || part == 0) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[offset + (16 * kb + j) * kHead] = S[kb][j];
+    }
+    return;
+  }
+  uint16_t* planes = reinterpret_cast<uint16_t*>(dst) + offset;
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      const uint3 x = split3_bf16x2(S[kb][j], S[kb][j + 1]);
+      uint16_t* row = planes + (16 * kb + j) * kHead;
+      row[0] = static_cast<uint16_t>(x.x);
+      row[kHead] = static_cast<uint16_t>(x.x >> 16);
+      row[kStateElems] = static_cast<uint16_t>(x.y);
+      row[kStateElems + kHead] = static_cast<uint16_t>(x.y >> 16);
+      row[2 * kStateElems] = static_cast<uint16_t>(x.z);
+      row[2 * kStateElems + kHead] = static_cast<uint16_t>(x.z >> 16);
+    }
+  }
 }
 
 // How a call is split: at most `parts` parts of `len` chunks each.
@@ -391,7 +443,7 @@ inline PartPlan plan_parts(int64_t sequences, int64_t heads, int64_t chunks, int
 // units and 111.9 by slots (the search for a slot's sequence); 63 single tokens
 // and a prompt of 2048 173.6 by units (most workgroups without a part) and 94.1.
 inline size_t part_bytes(int64_t states) {
-  return static_cast<size_t>(states) * 2 * kStateElems * sizeof(float);
+  return static_cast<size_t>(states) * kPartElems * sizeof(float);
 }
 inline size_t unit_part_bytes(int64_t units, const PartPlan& plan) {
   return part_bytes(units * (plan.parts - 1));

@@ -462,12 +462,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
     if (!whole && more) load_rows(rows, c0, min(kChunk, c_end - c0));
   }
 
-  float* dst = place.state(part, map ? 0 : 1) + s_off;
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dst[(16 * kb + j) * kHead] = S[kb][j];
-  }
+  store_part_state(place, part, map, s_off, S);
 }
 
 // One chunk's adjoint step of a column slab, dS at the chunk's end to dS at its
@@ -683,12 +678,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_adjoint_kernel(Chun
     if (!whole && more) load_rows(rows, c0, c_end - c0);
   }
 
-  float* dst = place.state(part, map ? 0 : 1) + s_off;
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dst[(16 * kb + j) * kHead] = S[kb][j];
-  }
+  store_part_state(place, part, map, s_off, S);
 }
 
 }  // namespace

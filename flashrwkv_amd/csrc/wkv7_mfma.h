@@ -102,6 +102,15 @@ __device__ __forceinline__ uint2 split_bf16x2(float x0, float x1) {
   return make_uint2(hi, pack_bf16x2(x0 - h0, x1 - h1));
 }
 
+// The same in three parts, x = hi + mid + lo exactly (8 bits of the significand
+// each), for finite x whose low parts are normal numbers.
+__device__ __forceinline__ uint3 split3_bf16x2(float x0, float x1) {
+  const uint32_t hi = pack_bf16x2(x0, x1);
+  const uint2 rest = split_bf16x2(x0 - __uint_as_float(hi << 16),
+                                  x1 - __uint_as_float(hi & 0xffff0000u));
+  return make_uint3(hi, rest.x, rest.y);
+}
+
 // C-layout accumulator -> bf16 operand registers (two packed conversions;
 // a single 4-wide vector conversion is split into per-value conversions plus
 // byte permutes when its result feeds an MFMA operand directly).
@@ -117,6 +126,13 @@ __device__ __forceinline__ void to_operand_split(f32x4 c, i16x4& hi, i16x4& lo) 
   const u32x2 h = {p01.x, p23.x}, l = {p01.y, p23.y};
   hi = __builtin_bit_cast(i16x4, h);
   lo = __builtin_bit_cast(i16x4, l);
+}
+__device__ __forceinline__ void to_operand_split3(f32x4 c, i16x4& hi, i16x4& mid, i16x4& lo) {
+  const uint3 p01 = split3_bf16x2(c[0], c[1]);
+  const uint3 p23 = split3_bf16x2(c[2], c[3]);
+  hi = __builtin_bit_cast(i16x4, u32x2{p01.x, p23.x});
+  mid = __builtin_bit_cast(i16x4, u32x2{p01.y, p23.y});
+  lo = __builtin_bit_cast(i16x4, u32x2{p01.z, p23.z});
 }
 
 // Inverses of I - L for a strictly lower 16 x 16 L, as every chunk form needs

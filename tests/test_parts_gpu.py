@@ -125,6 +125,49 @@ def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
     assert torch.equal(pool[-1], d["state_pool"].to(pool_dtype)[-1])  # the slot of no sequence
 
 
+# Tokens that leave the state alone (a, b, k and v zero, retention 1): every chunk
+# maps S to S, so an fp32 state comes out of the parts bit for bit, as it does of
+# the unsplit kernels, and so does the adjoint at the end in the backward.
+@pytest.mark.parametrize("tokens", (640, 2304))
+@pytest.mark.parametrize("kernel", (CHUNK, RECURRENT, "backward"))
+def test_split_carries_the_state_in_fp32(kernel, tokens):
+    heads, lib, io = 3, capi.library(), capi.DTYPE[torch.bfloat16]
+    zero = torch.zeros((tokens, heads, 64), dtype=torch.bfloat16, device=DEV)
+    one, y = torch.ones_like(zero), torch.empty_like(zero)
+    state = torch.randn((1, heads, 64, 64), generator=torch.Generator().manual_seed(3)).to(DEV)
+    cu, idx = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([0, tokens], [0]))
+    if kernel == "backward":
+        chunks = tokens // 64
+        ends = torch.arange(64, tokens + 1, 64, dtype=torch.int32, device=DEV)
+        lists = torch.tensor([0, chunks], dtype=torch.int32, device=DEV)
+        scratch, size = _scratch(4, io, 1, heads, chunks, tokens)
+        boundary = torch.zeros((chunks, heads, 64, 64), device=DEV)
+        work = capi.workspace(capi.statetune_backward_workspace_bytes(64, heads, tokens, False),
+                              DEV)
+        grads, got = [torch.empty_like(zero) for _ in range(6)], torch.empty_like(state)
+        rc = lib.frwkv_statetune_backward_split(
+            io, 1, 1, heads, 64, tokens, chunks,
+            *(capi._p(x) for x in (lists, ends - 64, ends, boundary, None, zero, one, None, zero,
+                                   zero, zero, zero, None, state, *grads, got, work)),
+            work.numel(), 1.0, None, capi._p(scratch), size, capi._stream())
+    else:
+        status, cu, idx = capi.metadata_validate(cu, idx, tokens, 1)
+        scratch, size = _scratch(kernel, io, 1, heads, tokens, tokens)
+        got = state.clone()
+        ptrs = [capi._p(x) for x in (cu, idx, status, got, zero, one, None, zero, zero, zero, zero,
+                                     y)]
+        area = (capi._p(scratch), size, capi._stream())
+        if kernel == CHUNK:
+            rc = lib.frwkv_chunk_forward_split(io, 1, capi.DTYPE[torch.float32], 1, heads, 64,
+                                               tokens, 1, *ptrs, 1.0, tokens, *area)
+        else:
+            rc = lib.frwkv_recurrent_forward_split(io, 1, 1, heads, 64, tokens, tokens, 1, *ptrs,
+                                                   1.0, *area)
+    capi._check(rc)
+    torch.cuda.synchronize()
+    assert torch.equal(got, state)
+
+
 # Head sizes and lengths around the 16-token pieces of the fp32 matrix form,
 # which the public entries take with fp16 tokens or wide heads (decay logits):
 # one piece and a token, ragged, a sequence in the middle shorter than a piece.
