@@ -65,7 +65,8 @@ PMC_KIB = {  # kernel -> (FETCH_SIZE, WRITE_SIZE)
 # host-only change to chunk_fwd.hip (the interior-state byte count) whose
 # gfx950 assembly was compared equal to the measured one except for the
 # compilation-unit id.
-PMC_SOURCES = ("flashrwkv_amd/csrc/recurrent.hip", "flashrwkv_amd/csrc/chunk_fwd.hip",
+PMC_SOURCES = ("flashrwkv_amd/csrc/recurrent.hip", "flashrwkv_amd/csrc/chunk_fwd_kernel.h",
+               "flashrwkv_amd/csrc/chunk_fwd.hip", "flashrwkv_amd/csrc/chunk_precise.hip",
                "flashrwkv_amd/csrc/chunk_bwd.hip", "flashrwkv_amd/csrc/chunk_common.h",
                "flashrwkv_amd/csrc/wkv7_device.h", "flashrwkv_amd/csrc/wkv7_mfma.h",
                "flashrwkv_amd/_build.py")

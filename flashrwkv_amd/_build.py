@@ -57,7 +57,11 @@ def _run(cmd: list[str]) -> None:
 # per SIMD; LLVM's max-ilp strategy orders their MFMA/LDS chains for
 # instruction-level parallelism instead of register pressure. Same-box A/B,
 # results bitwise identical: backward 1.580 -> 1.556 ms (config 4), dense
-# prefill 0.447 -> 0.440 ms (config 3), varlen unchanged.
+# prefill 0.447 -> 0.440 ms (config 3), varlen unchanged. The split-precision
+# forward (chunk_precise, one wave per SIMD) is faster with the default strategy:
+# 14 sequences of about 290 tokens in 32 heads 80.2 -> 72.7 us, 64 of 512 tokens
+# 467 -> 423; the bf16 forward with it: 8 of 2048 tokens 178 -> 163, 16 of 1024
+# 126 -> 130, full GPUs unchanged.
 FILE_FLAGS = {
     "chunk_fwd": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "chunk_bwd": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],

@@ -67,7 +67,7 @@ int frwkv_train_recurrent_backward(int io_dtype, int decay_mode, int32_t num_seq
 // size (0 when a unit fits one workgroup, i.e. head size 128).
 size_t frwkv_train_slice_bytes(int32_t head_size, int32_t num_heads, int32_t total_tokens);
 
-// The recurrent operator's route for long sequences (chunk_fwd.hip): the
+// The recurrent operator's route for long sequences (chunk_precise.hip): the
 // split-precision chunk kernel on bf16 tokens, head size 64, fp32 pool.
 // Arguments as frwkv_recurrent_forward_split's, already checked by it.
 int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32_t num_heads,

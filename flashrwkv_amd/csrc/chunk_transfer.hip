@@ -2,7 +2,7 @@
 // one (sequence, head), the map M and the offset N with
 // S_end = M S_start + N.
 //
-// Per chunk, with the notation of the forward kernel (chunk_fwd.hip), a state
+// Per chunk, with the notation of the forward kernel (chunk_fwd_kernel.h), a state
 // S (64 keys x any columns) moves by
 //   SA = (I - Lab)^{-1} (At S + Lak V),  S' = diag(2^GC) (S + Bh^T SA + Kh^T V),
 // so N follows it from 0 and M from the identity with V = 0. Neither needs r,
@@ -49,7 +49,7 @@ struct TransferRows {
   uint4 w, a, b, k, v;  // adjoint: r and dy in place of k and v
 };
 
-// Decay-span verdicts of a prepared range (see chunk_fwd.hip), uniform over
+// Decay-span verdicts of a prepared range (see chunk_fwd_kernel.h), uniform over
 // the workgroup.
 struct TransferSpans {
   bool whole;
@@ -164,7 +164,7 @@ __device__ __forceinline__ TransferSpans transfer_prepare(TransferSmem<kPrecise>
 // Lab, Lak ([t][i] blocks) and the diagonal inverses: waves 0-3 the diagonal
 // block of their index and its inverse, waves 4-7 three of the twelve
 // off-diagonal blocks each. Blocks are computed transposed (A operand = Y
-// rows), as in chunk_fwd.hip. The adjoint's second matrix is Arb (Rt Bh^T, with
+// rows), as in chunk_fwd_kernel.h. The adjoint's second matrix is Arb (Rt Bh^T, with
 // its diagonal) in place of Lak. Ends with a barrier.
 template <bool kPrecise, bool kAdjoint = false>
 __device__ __forceinline__ void transfer_intra(TransferSmem<kPrecise>& sm) {
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(kTransferThreads, 4) void chunk_transfer_kernel(Chu
       if (more) next_segment();
     }
     // One pass over the whole chunk, or, where its decay span exceeds the
-    // limit, over 16- or 4-token sub-chunks (as in chunk_fwd.hip).
+    // limit, over 16- or 4-token sub-chunks (as in chunk_fwd_kernel.h).
     TransferSpans spans{};
     bool whole = true, probe = true;
     int lo = 0, hi = ntok;

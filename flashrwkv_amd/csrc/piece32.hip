@@ -3,7 +3,7 @@
 // The per-token kernels (recurrent.hip, train_recurrent.hip) do one dependent
 // step per token: about five VALU instructions per state element and a
 // reduction over the keys on the critical path. This file takes the chunk form
-// of chunk_fwd.hip with 16-token pieces and fp32 operands throughout, on the
+// of chunk_fwd_kernel.h with 16-token pieces and fp32 operands throughout, on the
 // fp32 matrix instruction (v_mfma_f32_16x16x4_f32, twice the rate of unpacked
 // fp32 VALU): per piece, with cumulative decays G (inclusive) and Gp
 // (exclusive), At = a 2^Gp, Rt = r 2^G, Bh = b 2^-G, Kh = k 2^-G,

@@ -11,7 +11,7 @@
 // each sequence's pieces in reverse, carrying the state adjoint dS (dL/dS at
 // the current piece end) in registers.
 //
-// A 16-token piece is one 16 x 16 block of the chunk algebra of chunk_fwd.hip
+// A 16-token piece is one 16 x 16 block of the chunk algebra of chunk_fwd_kernel.h
 // (tokens t, i in 0..15, keys k and values v in 0..127, G the cumulative log2
 // retention from the piece start, Gp = G - log2 w, g = 2^G at the last token):
 //   At = a 2^Gp, Rt = r 2^G, Bh = b 2^-G, Kh = k 2^-G;
