@@ -80,12 +80,12 @@ extern "C" size_t frwkv_split_scratch_bytes(int kernel, int io_dtype, int decay_
   switch (kernel) {
     case FRWKV_SPLIT_CHUNK:  // of equal sequences (pretraining): states by unit
       return packed_part_bytes(total, num_sequences, num_heads,
-                               plan_parts(num_sequences, num_heads, chunks_of(total),
-                                          chunks_of(longest), kForwardTime, kTransferTime));
+                               plan_packed_parts(num_sequences, num_heads, total, longest,
+                                                 kForwardTime, kTransferTime));
     case FRWKV_SPLIT_RECURRENT:
       return packed_part_bytes(total, num_sequences, num_heads,
-                               plan_parts(num_sequences, num_heads, chunks_of(total),
-                                          chunks_of(longest), kPreciseTime, kTransferTime));
+                               plan_packed_parts(num_sequences, num_heads, total, longest,
+                                                 kPreciseTime, kTransferTime));
     case FRWKV_SPLIT_CALLER_CHUNKS:
       return unit_part_bytes(units, plan_caller_chunks(num_sequences, num_heads, total));
     case FRWKV_SPLIT_PRETRAIN_BACKWARD:
@@ -164,8 +164,8 @@ extern "C" int frwkv_chunk_forward_split(
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * head_size;
   const int units = num_sequences * num_heads;
   use_packed_parts(p, num_sequences,
-                   plan_parts(num_sequences, num_heads, chunks_of(total_tokens),
-                              chunks_of(max_seqlen), kForwardTime, kTransferTime),
+                   plan_packed_parts(num_sequences, num_heads, total_tokens, max_seqlen,
+                                     kForwardTime, kTransferTime),
                    scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (pool_dtype == FRWKV_DTYPE_F32) return dispatch_chunk_io<float>(p, io_dtype, decay_mode, units, s);
@@ -420,8 +420,8 @@ extern "C" int frwkv_pretrain_forward_split(
   p.scale = 1.0f;
   p.out_elems = static_cast<int64_t>(batch) * tokens * num_heads * head_size;
   use_unit_parts(p, static_cast<int64_t>(batch) * num_heads,
-                 plan_parts(batch, num_heads, chunks_of(p.total_tokens), chunks_of(tokens),
-                            kForwardTime, kTransferTime),
+                 plan_packed_parts(batch, num_heads, p.total_tokens, tokens, kForwardTime,
+                                   kTransferTime),
                  scratch, scratch_bytes);
   return dispatch_chunk_io<float>(p, io_dtype, decay_mode, batch * num_heads,
                                   static_cast<hipStream_t>(stream));

@@ -38,8 +38,8 @@ int frwkv_recurrent_chunked_forward(int decay_mode, int32_t num_sequences, int32
   p.out_elems = static_cast<int64_t>(total_tokens) * num_heads * kHead;
   const int units = num_sequences * num_heads;
   use_packed_parts(p, num_sequences,
-                   plan_parts(num_sequences, num_heads, chunks_of(total_tokens),
-                              chunks_of(max_seqlen), kPreciseTime, kTransferTime),
+                   plan_packed_parts(num_sequences, num_heads, total_tokens, max_seqlen,
+                                     kPreciseTime, kTransferTime),
                    scratch, scratch_bytes);
   auto s = static_cast<hipStream_t>(stream);
   if (decay_mode == FRWKV_DECAY_LOGITS) {

@@ -262,6 +262,23 @@ def test_split_scratch_follows_the_tokens_without_a_gpu(kernel, singles, longest
     assert size <= 2 * 16 * heads * 32768  # at most 16 parts of the prompt
 
 
+# Batches that a split slows down keep the unsplit kernel (32 heads; the faster
+# side of every case is measured): short sequences that fill the GPU by themselves
+# while the prompt's chain runs.
+@pytest.mark.parametrize("kernel,sequences,tokens,longest,split", [
+    (0, 1, 512, 512, True), (0, 16, 1039, 1024, True), (0, 64, 2111, 2048, True),
+    (0, 256, 767, 512, False), (0, 256, 1279, 1024, False), (0, 64, 32 * 1024, 512, False),
+    (1, 1, 512, 512, True), (1, 16, 1039, 1024, True), (1, 64, 2111, 2048, True),
+    (1, 64, 1087, 1024, False), (1, 16, 1820, 320, False), (1, 256, 1279, 1024, False),
+])
+def test_split_of_mixed_batches_without_a_gpu(kernel, sequences, tokens, longest, split):
+    from flashrwkv_amd import capi
+
+    assert (capi.library().frwkv_split_scratch_bytes(
+        kernel, capi.DTYPE[torch.bfloat16], capi.DECAY_LOGITS, sequences, 32, 64, tokens,
+        longest) > 0) == split
+
+
 # The fp32 matrix form's route of the recurrent entry (it has scratch): batches of
 # prompts take it, decoding batches that admit a short prompt keep the per-token
 # kernel. The faster side of every case is measured (piece32.h).
