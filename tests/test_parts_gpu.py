@@ -4,7 +4,9 @@ cut into parts whose start states are composed from transfer states.
 Split results are compared with the fp64 oracle at the chunk kernel's own
 bounds (normwise 2e-2 for bf16 operands, as in tests/test_chunk_gpu.py) and
 with the same call unsplit (no scratch), from which they differ only by the
-rounding of the states: at most 1e-2 normwise, half the bound both meet.
+rounding of the states: at most 1e-2 normwise, half the bound both meet. The
+split-precision route's state has that route's own bound, 2e-3
+(tests/test_recurrent_gpu.py), and half of it against unsplit.
 """
 
 from __future__ import annotations
@@ -24,6 +26,7 @@ pytestmark = pytest.mark.gpu
 
 DEV = torch.device("cuda")
 TOL, SAME = 2e-2, 1e-2
+TOL_STATE = 2e-3
 NAMES = ("r", "w", "k", "v", "a", "b")
 CHUNK, RECURRENT, CALLER_CHUNKS = 0, 1, 2
 
@@ -119,9 +122,10 @@ def test_split_packed_forward(kernel, lengths, dtype, pool_dtype, u_low):
         case["state_indices"].numpy(), scale=0.75)
     (y, pool), (y1, pool1) = out
     parity.check("y", y, y_ref, TOL)
-    parity.check("state", pool, pool_ref, TOL)
+    parity.check("state", pool, pool_ref, TOL_STATE if kernel == RECURRENT else TOL)
     parity.check("y against unsplit", y, y1.double().cpu(), SAME)
-    parity.check("state against unsplit", pool, pool1.double().cpu(), SAME)
+    parity.check("state against unsplit", pool, pool1.double().cpu(),
+                 TOL_STATE / 2 if kernel == RECURRENT else SAME)
     assert torch.equal(pool[-1], d["state_pool"].to(pool_dtype)[-1])  # the slot of no sequence
 
 
@@ -168,6 +172,47 @@ def test_split_carries_the_state_in_fp32(kernel, tokens):
     assert torch.equal(got, state)
 
 
+# Repeated split calls are equal bit for bit: nothing depends on which workgroup
+# comes first. Through the public entries, forward and backward.
+@pytest.mark.parametrize("entry", ("recurrent", "chunk", "statetune", "pretrain"))
+def test_split_calls_repeat_bitwise(entry):
+    lengths, heads = (900, 610), 2
+    case = workloads.make_case(lengths=lengths, heads=heads, head_size=64, dtype=torch.bfloat16,
+                               seed=23, state_std=0.1)
+    dev = {k: v.to(DEV) if isinstance(v, torch.Tensor) else v for k, v in case.items()}
+    n = sum(lengths)
+
+    def run():
+        if entry in ("recurrent", "chunk"):
+            pool = dev["state_pool"].to(torch.float32 if entry == "recurrent" else torch.bfloat16,
+                                        copy=True)
+            call = (flashrwkv_amd.infer_recurrent_fp32io16_forward_varlen if entry == "recurrent"
+                    else flashrwkv_amd.infer_chunk_bf16_forward_varlen)
+            out = call(*(dev[x] for x in NAMES), state_pool=pool, cu_seqlens=dev["cu_seqlens"],
+                       state_indices=dev["state_indices"], max_seqlen=max(lengths))
+            return [out[0] if isinstance(out, tuple) else out, pool]
+        leaves = [dev[x].clone().requires_grad_() for x in NAMES]
+        if entry == "pretrain":
+            out = [flashrwkv_amd.pretrain_recurrent_bf16(
+                *(x[:1504].reshape(2, 752, heads * 64) for x in leaves))]
+        else:
+            state = dev["state_pool"][:2].clone().requires_grad_()
+            meta = oracle.chunk_metadata(lengths, 64)
+            out = list(flashrwkv_amd.statetune_recurrent_fp32io16(
+                state, *(torch.from_numpy(x).to(DEV) for x in meta[:3]), *leaves)[:2])
+            leaves.append(state)
+        return out + list(torch.autograd.grad([x.float().square().sum() for x in out], leaves))
+
+    kernel = {"recurrent": RECURRENT, "chunk": CHUNK, "statetune": 4, "pretrain": 3}[entry]
+    total, longest = {"statetune": (25, n), "pretrain": (1504, 752)}.get(entry, (n, max(lengths)))
+    assert capi.library().frwkv_split_scratch_bytes(
+        kernel, capi.DTYPE[torch.bfloat16], capi.DECAY_LOGITS, 2, heads, 64, total, longest) > 0
+    first, second = run(), run()
+    torch.cuda.synchronize()
+    for x, y in zip(first, second, strict=True):
+        assert torch.equal(x, y)
+
+
 # Head sizes and lengths around the 16-token pieces of the fp32 matrix form,
 # which the public entries take with fp16 tokens or wide heads (decay logits):
 # one piece and a token, ragged, a sequence in the middle shorter than a piece.
@@ -177,6 +222,7 @@ def test_split_carries_the_state_in_fp32(kernel, tokens):
 @pytest.mark.parametrize("dtype,d,lengths", [
     (torch.float16, 64, (33,)),
     (torch.float16, 64, (1, 48, 7, 65, 16)),
+    (torch.float16, 64, (40,) * 70 + (33, 1, 17)),  # two rounds of the slot search
     (torch.float16, 128, (40, 3)),
     (torch.bfloat16, 128, (32, 95)),
     (torch.float16, 256, (17, 50)),
@@ -184,6 +230,9 @@ def test_split_carries_the_state_in_fp32(kernel, tokens):
 ])
 def test_fp32_matrix_recurrence(dtype, d, lengths):
     heads = 2
+    assert capi.library().frwkv_split_scratch_bytes(
+        RECURRENT, capi.DTYPE[dtype], capi.DECAY_LOGITS, len(lengths), heads, d, sum(lengths),
+        max(lengths)) > 0, "the case is meant to take the matrix form"
     case = workloads.make_case(lengths=lengths, heads=heads, head_size=d, dtype=dtype, seed=5,
                                state_std=0.1, pool_slots=len(lengths) + 1,
                                slots=list(range(len(lengths)))[::-1])

@@ -408,6 +408,38 @@ def test_large_heads_long_sequence(head_size):
     _compare(out, grads, ref_out, ref_grads)
 
 
+def _logits_256(lengths, chunk, heads, seed):
+    """A head-size-256 case with decay logits, the fp32 matrix form's, and its
+    retention (the cases above pass raw retentions, the per-token kernels')."""
+    case = workloads.make_case(lengths=lengths, heads=heads, head_size=256,
+                               dtype=torch.bfloat16, seed=seed, state_std=0.1)
+    gen = torch.Generator().manual_seed(seed)
+    case["w"] = (torch.randn(case["w"].shape, generator=gen) * 2.0).to(torch.bfloat16)
+    return case, oracle.chunk_metadata(lengths, chunk)
+
+
+def test_head256_logits_repeats_bitwise():
+    case, meta = _logits_256((35, 270), 32, 2, 8)
+    o1, g1, _, _ = _run(case, meta, scale=1.0, public=True)
+    o2, g2, _, _ = _run(case, meta, scale=1.0, public=True)
+    for name, a, b in zip(("y", "final state", "boundary", "state_dot_a"), o1, o2):
+        assert torch.equal(a, b), name
+    for nm in (*NAMES, "s0"):
+        assert torch.equal(g1[nm], g2[nm]), nm
+
+
+# A long sequence, and more caller chunks than the piece table numbers at a time
+# (1024).
+@pytest.mark.parametrize("lengths,chunk", [((1000, 37), 64), ((1100,), 1)])
+def test_head256_logits_long_sequence(lengths, chunk):
+    case, meta = _logits_256(lengths, chunk, 1, 124)
+    out, grads, dy, ds = _run(case, meta, scale=1.0, public=True)
+    x = _np(case["w"])
+    w = oracle.retention_from_logits(x)
+    ref_out, ref_grads = _oracle(case, meta, w, scale=1.0, dy=dy, ds=ds, batch=len(lengths))
+    _compare(out, grads, ref_out, ref_grads, dw_factor=w * oracle.retention_log_derivative(x))
+
+
 def test_head128_full_shape_sampled_heads():
     """The head-size-128 leg's shape (B=8, T=4096, H=32, D=128, 64-token caller
     chunks walked as four 16-token pieces, S0 ~ N(0, 0.1)) on the MFMA piece

@@ -8,6 +8,8 @@ import time
 
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from flashrwkv_amd.tmix import wkv7
 from flashrwkv_amd.tmix.wkv7 import pretrain
@@ -152,6 +154,126 @@ def test_whole_call_and_tables_agree(which, monkeypatch):
         assert isinstance(here, list), (form, here)
         for x, y in zip(here, tables, strict=True):
             assert x.dtype == y.dtype and torch.equal(x, y), form
+
+
+class _Seen(TorchDispatchMode):
+    """A dispatch mode that lists the operators it sees."""
+
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+class _SeenFunctions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(getattr(func, "__name__", str(func)))
+        return func(*args, **(kwargs or {}))
+
+
+def _gradients(entry, call, dy=None):
+    out = entry(**call)
+    dy = torch.full_like(out, 0.25) if dy is None else dy
+    return [out.detach(), *torch.autograd.grad(out, [call[n] for n in "rwkvab"], dy)]
+
+
+# Modes see the operators of a call, as through the tables.
+@pytest.mark.parametrize("which", ["fp32", "fp16", "advance", "pretrain"])
+@pytest.mark.parametrize("mode", [_Seen, _SeenFunctions])
+def test_modes_see_the_operators(which, mode, monkeypatch):
+    outcomes, names = [], []
+    for tables in (False, True):
+        entry, call = _call(which)
+        with monkeypatch.context() as patch, mode() as seen:
+            if tables:
+                patch.setattr(wkv7, "_whole_call", lambda name: None)
+                patch.setattr(pretrain.C.native().direct, "clampw_accepts", lambda *x: False)
+            outcomes.append(_outcome(entry, call))
+        names.append(seen.names)
+    torch.cuda.synchronize()
+    assert names[0] == names[1] and (names[0] or which == "advance")
+    for x, y in zip(*outcomes, strict=True):
+        assert torch.equal(x, y)
+
+
+def _under_vmap(entry, call):
+    names = [n for n in "rwkvab" if n in call]
+    fixed = {n: x for n, x in call.items() if n not in names}
+    return torch.vmap(lambda *t: entry(**fixed, **dict(zip(names, t))))(
+        *(torch.stack([call[n], call[n]]) for n in names))
+
+
+def _under_jvp(entry, call):
+    with torch.autograd.forward_ad.dual_level():
+        r = torch.autograd.forward_ad.make_dual(call["r"].detach(), torch.ones_like(call["r"]))
+        return entry(**{**call, "r": r})
+
+
+# Transforms have the same outcome on both, an error here: no derivative or
+# batching rule is passed by.
+@pytest.mark.parametrize("transform", [_under_vmap, _under_jvp])
+def test_transforms_have_the_same_outcome(transform, monkeypatch):
+    outcomes = []
+    for direct in (True, False):
+        entry, call = _call("pretrain")
+        with monkeypatch.context() as patch:
+            if not direct:
+                patch.setattr(torch.compiler, "is_compiling", lambda: True)
+            try:
+                outcomes.append(transform(entry, call))
+            except Exception as error:  # noqa: BLE001 - the outcome itself is compared
+                outcomes.append(type(error))
+        torch.cuda.synchronize()
+    assert outcomes[0] is outcomes[1] and issubclass(outcomes[0], Exception)
+
+
+# Saved tensors go through the hooks of the forward, and a gradient comes in any
+# layout.
+@pytest.mark.parametrize("form", ["hooks", "expanded", "strided", "wrapped"])
+def test_pretraining_backward_takes_every_form(form):
+    entry, call = _call("pretrain")
+    packed, dy = [], torch.full_like(call["r"], 0.25)
+    want = _gradients(entry, call, dy)
+    if form == "hooks":
+        with torch.autograd.graph.saved_tensors_hooks(
+                lambda x: packed.append(x.shape) or x.cpu(), lambda x: x.to(DEV)):
+            got = _gradients(entry, call, dy)
+        assert len(packed) == 8
+    else:
+        given = {"expanded": dy[:, :1, :1].expand(dy.shape), "strided": _strided(dy),
+                 "wrapped": dy.as_subclass(Wrapped)}[form]
+        got = _gradients(entry, call, given)
+    torch.cuda.synchronize()
+    for x, y in zip(got, want, strict=True):
+        assert torch.equal(x, y)
+
+
+# On another stream than the default one the launches are that stream's, and so is
+# the backward's (autograd runs it on the forward's).
+@pytest.mark.parametrize("which", ["fp32", "fp16", "advance", "pretrain"])
+def test_whole_calls_on_another_stream(which):
+    entry, call = _call(which)
+    want = _outcome(entry, call)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        entry, call = _call(which)
+        torch.cuda._sleep(20_000_000)
+        if which != "pretrain":  # the inputs are final only after the wait
+            for x in call.values():
+                if isinstance(x, torch.Tensor) and x.is_floating_point():
+                    x.add_(0)
+        got = _outcome(entry, call)
+        side.synchronize()
+    for x, y in zip(got, want, strict=True):
+        assert torch.equal(x, y)
 
 
 # With a switch interval of minutes a thread that waits for the interpreter runs
