@@ -12,7 +12,7 @@
 //   S' = g (S0 + Bh^T SA + Kh^T V),  g = 2^G(last token).
 // Operands, sums and states are fp32, as in the per-token kernels; results
 // differ by the order of the sums. Decay logits only: their retention is at
-// least exp(-e^{-1/2}), so a piece's decay stays above 2^-14 and one reference
+// least exp(-e^{-1/2}), so a piece's decay stays above 2^-15 and one reference
 // point serves a piece (raw retentions stay on the per-token kernels).
 //
 // The matrix products spread a NaN or an infinity over a whole piece (a masked
@@ -582,8 +582,8 @@ __device__ __forceinline__ void token_form(const Piece32Params& p, const Walk& w
 // 64)), value columns col0 .. +15; S[kb][j] is key 64q + 16kb + 4g + j, column
 // col0 + n. kTrain: boundary, interior and a^T S outputs. Bound by the serial
 // chain of its matrix products (a sequence and head occupy D / 16 waves at
-// D = 64, 4 D / 16 at 256). Measured: 24 pieces in 288 units at D = 64 45 us;
-// 32 pieces in 16 units at D = 256 99 us, where the per-token kernel takes 567.
+// D = 64, 4 D / 16 at 256). Measured: 24 pieces in 288 units at D = 64 46 us;
+// 32 pieces in 16 units at D = 256 98 us, where the per-token kernel takes 567.
 template <typename T, int D, bool kTrain>
 __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p) {
   using L = Tiles<D>;
@@ -830,7 +830,7 @@ __global__ __launch_bounds__(256, 2) void piece32_forward_kernel(Piece32Params p
 // Per piece, with dU = g o dS and dYs = scale dY:
 //   dSA = Bh dU + Arb^T dYs,  dZ = T^T dSA,
 //   dV  = Kh dU + Ark^T dYs + Lak^T dZ,  dS <- dU + Rt^T dYs + At^T dZ.
-// Bound like the forward chain: 32 pieces in 16 units 109 us (the per-token
+// Bound like the forward chain: 32 pieces in 16 units 106 us (the per-token
 // backward, which also forms the gradients, takes 3330).
 template <typename T, int D>
 __global__ __launch_bounds__(256, 1) void piece32_adjoint_kernel(Piece32Params p) {

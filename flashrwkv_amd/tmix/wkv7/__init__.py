@@ -200,11 +200,11 @@ def set_recurrent_long_route(route: str) -> str:
     split-precision chunk kernel: its outputs meet the reference's
     relative-RMSE gate of 0.002, but the pool it leaves differs from the
     per-token fp32 recurrence by about 4e-4 relative RMSE (1e-7 on the
-    per-token kernel). ``"per_token"`` runs every call on the per-token fp32
-    kernel, as the reference computes it, at several times the time for long
-    sequences. Decode, short sequences, fp16 tokens and other head sizes run
-    the per-token kernel either way, and so does any call made under HIP
-    graph capture. The setting is process-wide; returns the previous route.
+    per-token kernel). Prompts of fp16 tokens, or at head sizes 128 and 256,
+    run in fp32 matrix products over 16 tokens at a time. ``"per_token"`` runs
+    every call on the per-token fp32 kernel, as the reference computes it, at
+    several times the time for long sequences. Decode and short sequences run
+    it either way, and so does any call made under HIP graph capture. The setting is process-wide; returns the previous route.
     """
     if route not in _ROUTE_CODES:
         raise ValueError(f"route must be one of {sorted(_ROUTE_CODES)}, got {route!r}")

@@ -128,7 +128,8 @@ int frwkv_recurrent_forward(int io_dtype, int decay_mode, int32_t num_sequences,
  * undefined before and after the call. With no scratch, or less than that, or
  * where that is 0 (enough sequences to fill the GPU, or too short ones), the
  * call runs unsplit, and is then exactly the entry of the same name. Results
- * of the two agree up to the rounding of the state between parts.
+ * of the two agree up to the rounding of the chunks' products; the state goes
+ * from part to part in fp32.
  *
  * frwkv_split_scratch_bytes: total is the call's total tokens (B * T for
  * pretraining) and longest its longest sequence in tokens (max_seqlen, T) for
@@ -297,8 +298,8 @@ int frwkv_statetune_forward(int io_dtype, int decay_mode, int32_t num_sequences,
                             void* output, float* boundary, float* state_dot_a,
                             float* interior, float scale, void* stream);
 
-/* frwkv_statetune_forward with scratch for a split call (see
- * frwkv_split_scratch_bytes; head size 64). */
+/* frwkv_statetune_forward with scratch for a split call at head size 64, or for
+ * the fp32 matrix form at head size 256 (see frwkv_split_scratch_bytes). */
 int frwkv_statetune_forward_split(int io_dtype, int decay_mode, int32_t num_sequences,
                                   int32_t num_heads, int32_t head_size,
                                   int32_t total_tokens, int32_t num_chunks,
@@ -449,8 +450,8 @@ int frwkv_pretrain_forward(int io_dtype, int decay_mode, int32_t batch, int32_t 
                            const void* a, const void* b, void* output, float* boundary,
                            float* state_dot_a, void* stream);
 
-/* frwkv_pretrain_forward with scratch for a split call (see
- * frwkv_split_scratch_bytes; head size 64). */
+/* frwkv_pretrain_forward with scratch for a split call at head size 64, or for
+ * the fp32 matrix form at head size 256 (see frwkv_split_scratch_bytes). */
 int frwkv_pretrain_forward_split(int io_dtype, int decay_mode, int32_t batch, int32_t tokens,
                                  int32_t num_heads, int32_t head_size, const void* r,
                                  const void* decay, const void* k, const void* v,
