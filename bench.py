@@ -50,27 +50,25 @@ _COPY_KIB = 262144.0
 _COPY_FETCH_KIB = 131084.4
 _COPY_WRITE_KIB = 262144.0
 PMC_KIB = {  # kernel -> (FETCH_SIZE, WRITE_SIZE)
-    "recurrent_fp32_kernel<64,64,64,Bf16,kRawW>": (85811.4, 165205.5),
-    "chunk_fwd_kernel<Bf16,kRawW,float>": (790660.5, 270353.9),
-    "chunk_fwd_kernel<Bf16,kRawW,float>/statetune": (790712.8, 1318935.6),
-    "chunk_fwd_kernel<Bf16,kRawW,float>/precise": (395420.7, 135168.0),
-    "chunk_bwd_kernel<Bf16,kRawW>": (1184971.4, 1581074.2),
-    "recurrent_fp16_decode_kernel": (44876.3, 83232.4),
+    "recurrent_fp32_kernel<64,64,64,Bf16,kRawW>": (85811.4, 165202.4),
+    "chunk_fwd_kernel<Bf16,kRawW,float>": (790661.8, 270349.2),
+    "chunk_fwd_kernel<Bf16,kRawW,float>/statetune": (790728.5, 1318981.9),
+    "chunk_fwd_kernel<Bf16,kRawW,float>/precise": (395420.3, 135168.1),
+    "chunk_bwd_kernel<Bf16,kRawW>": (1186079.0, 1581080.5),
+    "recurrent_fp16_decode_kernel": (44876.2, 83229.7),
 }
 
 # The kernel sources PMC_KIB was measured on: sha256 over these files, in
 # order (the build script carries the compile flags). When the tree's sources
 # differ, the constants describe other kernels and pmc_traffic reports None
-# instead of a stale figure. Restamped once without a new measurement: a
-# host-only change to chunk_fwd.hip (the interior-state byte count) whose
-# gfx950 assembly was compared equal to the measured one except for the
-# compilation-unit id.
+# instead of a stale figure.
 PMC_SOURCES = ("flashrwkv_amd/csrc/recurrent.hip", "flashrwkv_amd/csrc/chunk_fwd_kernel.h",
                "flashrwkv_amd/csrc/chunk_fwd.hip", "flashrwkv_amd/csrc/chunk_precise.hip",
                "flashrwkv_amd/csrc/chunk_bwd.hip", "flashrwkv_amd/csrc/chunk_common.h",
+               "flashrwkv_amd/csrc/chunk_parts.h",
                "flashrwkv_amd/csrc/wkv7_device.h", "flashrwkv_amd/csrc/wkv7_mfma.h",
                "flashrwkv_amd/_build.py")
-PMC_SOURCES_SHA = "bba890fa1207aef767566d53c84f672dc60e779206bd164f67bc08a235499919"
+PMC_SOURCES_SHA = "229b38378b07a154271e20e02804e4b5e9600cd49e3f4369c3454129720adcdf"
 
 
 def kernel_sources_sha() -> str:
@@ -96,11 +94,11 @@ def pmc_traffic(kernel: str) -> int | None:
 # (SQ_VALU_MFMA_BUSY_CYCLES / 1024 SIMDs over SQ_BUSY_CU_CYCLES / 256 CUs, in
 # %), from the counter passes of the bench workloads.
 PMC_MFMA_BUSY_PCT = {
-    "chunk_fwd_kernel<Bf16,kRawW,float>": 21.4,
-    "chunk_fwd_kernel<Bf16,kRawW,float>/varlen": 21.0,
-    "chunk_fwd_kernel<Bf16,kRawW,float>/statetune": 15.5,
-    "chunk_fwd_kernel<Bf16,kRawW,float>/precise": 14.8,
-    "chunk_bwd_kernel<Bf16,kRawW>": 13.1,
+    "chunk_fwd_kernel<Bf16,kRawW,float>": 20.4,
+    "chunk_fwd_kernel<Bf16,kRawW,float>/varlen": 20.2,
+    "chunk_fwd_kernel<Bf16,kRawW,float>/statetune": 15.0,
+    "chunk_fwd_kernel<Bf16,kRawW,float>/precise": 15.8,
+    "chunk_bwd_kernel<Bf16,kRawW>": 12.9,
 }
 
 
