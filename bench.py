@@ -68,7 +68,7 @@ PMC_SOURCES = ("flashrwkv_amd/csrc/recurrent.hip", "flashrwkv_amd/csrc/chunk_fwd
                "flashrwkv_amd/csrc/chunk_parts.h",
                "flashrwkv_amd/csrc/wkv7_device.h", "flashrwkv_amd/csrc/wkv7_mfma.h",
                "flashrwkv_amd/_build.py")
-PMC_SOURCES_SHA = "229b38378b07a154271e20e02804e4b5e9600cd49e3f4369c3454129720adcdf"
+PMC_SOURCES_SHA = "d4486c9aa7f36dffaa7c36e5e7b353013b7a141dfc54208170e6815518a01d87"
 
 
 def kernel_sources_sha() -> str:

@@ -445,18 +445,19 @@ inline PartPlan plan_parts(int64_t sequences, int64_t heads, int64_t chunks, int
 // tokens evenly end in half a chunk, and have one chunk at least. A call takes
 // the longer of its longest chain and of all its workgroups' work, and a split
 // adds work: beside short sequences enough to fill the GPU it pays only where
-// the prompt's chain is the longer one by far: the estimate must promise 18%, or
+// the prompt's chain is the longer one by far: the estimate must promise 22%, or
 // 5% where every workgroup has a CU at once.
 //
 // Against every part count, forced, on 142 batches (one to 300 sequences, equal,
 // similar, mixed, and prompts beside short ones or single tokens; 12 to 40
-// heads): 2.0% (bf16) and 2.8% (split-precision) above the fastest in the mean
-// and at most 5% slower than unsplit (one of 70 others by 13%); counting the
-// chunks from the tokens alone, as for caller chunks, 4.2 and 4.4%, and up to
-// 1.26 and 1.44 times unsplit. 32 heads: 15 sequences of 100 tokens and one of
-// 320 in split precision took 1.41 times as long split, 255 single tokens and a
-// prompt of 512 1.20 times and in bf16 1.23 times, and stay whole; 63 single
-// tokens and a prompt of 2048 in bf16 take 171 us unsplit and 86 split.
+// heads): 2.0% (bf16) and 3.0% (split-precision) above the fastest in the mean
+// and at most 5% slower than unsplit (at 18% three of 190 others were 6 to 13%
+// slower); counting the chunks from the tokens alone, as for caller chunks, 4.2
+// and 4.4%, and up to 1.26 and 1.44 times unsplit. 32 heads: 15 sequences of 100
+// tokens and one of 320 in split precision took 1.41 times as long split, 255
+// single tokens and a prompt of 512 1.20 times and in bf16 1.23 times, and stay
+// whole; 63 single tokens and a prompt of 2048 in bf16 take 171 us unsplit and
+// 86 split.
 inline PartPlan plan_packed_parts(int64_t sequences, int64_t heads, int64_t tokens,
                                   int64_t longest_tokens, const ChunkTime& main,
                                   const ChunkTime& transfer) {
@@ -506,12 +507,14 @@ inline PartPlan plan_packed_parts(int64_t sequences, int64_t heads, int64_t toke
       const double work = (chunks * main.shared + maps * main.map) / each + main.part;
       const double all =
           main.rounds ? __builtin_ceil(groups / 256) * work / 2 : groups / 512 * work;
-      const double last = len * main.alone + 0.2 * parts * kForwardTime.alone;
+      // The longest sequence's own parts, at least, run at the same time.
+      const double own = main.rounds ? 256 : __builtin_fmin(heads * (parts - 1.0), 512);
+      const double last = len * main.of(own) + 0.2 * parts * kForwardTime.of(own);
       if (walk < all) walk = all;
       if (walk < last) walk = last;
     }
     const double time = 4.0 + len * transfer.of(groups - units) + walk;
-    if (time < least && time < unsplit * (alone ? 0.95 : 0.82)) {
+    if (time < least && time < unsplit * (alone ? 0.95 : 0.78)) {
       least = time;
       best = PartPlan{parts, static_cast<int32_t>(len)};
     }
